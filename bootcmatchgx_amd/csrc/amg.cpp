@@ -239,6 +239,8 @@ static void build_hierarchy(Context* c, const DCsr& A0, const bcmgx_params& p, H
             abs_row_sum(c, M.n, M.row.get(), M.val.get(), lv.M.get());
             if (l + 1 < H.levels())  // the restriction of the composed prolongator
                 transpose_prolongator(c, M.n, H.L[l + 1]->mat().n, lv.agg.get(), lv.pval.get(), lv.R);
+            else if (coarse_sweeps_fit(M.n, p.relaxnumber_coarse))
+                lv.cix.build(c, M);
             if (level_done) level_done(l);
         };
         if (side) side->run(work);
@@ -445,6 +447,7 @@ void Prec::ensure_work(int k) {
             nl = std::max(nl, hrc(h).levels());
             ncoarse = std::max(ncoarse, hrc(h).L.back()->mat().n);
         }
+        if (coarse_sweeps_fit(ncoarse, p.relaxnumber_coarse)) coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse);
         std::vector<size_t> lsz(nl, 1);
         for (int h = 0; h < n_hrc(); h++)
             for (int l = 0; l < hrc(h).levels(); l++) lsz[l] = std::max(lsz[l], (size_t)hrc(h).L[l]->mat().n);
@@ -564,6 +567,12 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
             // the coarsest-level sweeps run in FP64 on the FP64 operator
             long long nk = (long long)A.n * k;
             double* res;
+            if (k == 1) {  // every sweep in one launch
+                V* y = xzero ? cur : oth;
+                if (coarse_sweeps<V>(c, A, lv.lanesA, lv.M.get(), F, xzero ? nullptr : cur, y, p.relaxnumber_coarse,
+                                     lv.cix, pr->coarse, R.stop))
+                    return y;
+            }
             if (xzero && p.relaxnumber_coarse >= 1) {  // widening and the first sweep from zero in one pass
                 jacobi_from_zero_f32in(c, A.n, k, F, lv.M.get(), pr->cd_F.get(), pr->cd_X.get(), R.stop);
                 res = jacobi_sweeps<double>(c, A, lv.lanesA, lv.M.get(), pr->cd_F.get(), pr->cd_X.get(), pr->cd_X2.get(),
@@ -577,6 +586,12 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
             convert_stop<double, float>(c, res, cur, nk, R.stop);
             return cur;
         } else {
+            if (k == 1) {
+                V* y = xzero ? cur : oth;
+                if (coarse_sweeps<V>(c, A, lv.lanesA, lv.M.get(), F, xzero ? nullptr : cur, y, p.relaxnumber_coarse,
+                                     lv.cix, pr->coarse, R.stop))
+                    return y;
+            }
             return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, p.relaxnumber_coarse, xzero, k, R.stop,
                                     lv.chunkA);
         }

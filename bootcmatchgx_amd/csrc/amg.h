@@ -19,6 +19,7 @@ struct Level {
     DBuf<float> pvalf;
     DCsr R;                 // restrictor P^T (rows sorted by fine index)
     DCsr AP;                // A P, FP32 values only (valf): the first post-smoothing sweep of an FP32 cycle
+    CoarseIndex cix;        // of the coarsest level
     int lanesA = 0, lanesR = 0, lanesAP = 0;
     int chunkA = 0;         // columns per SpMM launch for the current batch width
     const DCsr& mat() const { return Aref ? *Aref : A; }
@@ -60,6 +61,7 @@ struct Prec {
     std::vector<LevelWork<double>> wd;
     std::vector<LevelWork<float>> wf;
     DBuf<double> cd_F, cd_X, cd_X2;  // FP64 coarsest-level buffers of the FP32 cycle
+    CoarseSync coarse;               // what the one-launch coarsest sweeps exchange through
     DBuf<double> tmp;                // AFSAI intermediate / prec_apply staging
     DBuf<double> tmp2, tmp3;         // additive bootstrap composition: the sum and one hierarchy's correction
     double setup_seconds = 0;

@@ -586,6 +586,15 @@ int bcmgx_dump_info(const char* path, const bcmgx_params* p, bcmgx_prec prec, co
     return BCMGX_OK;
 }
 
+// Not part of the public interface (no declaration in bcmgx.h): the clock ticks a wait of the
+// one-launch coarsest sweeps may take on this context before its fallback computes them
+// (negative: no wait, always the fallback).
+int bcmgx_internal_coarse_patience(bcmgx_context ctx, long long ticks) {
+    if (!ctx) return BCMGX_ERR_ARG;
+    ctx->c->coarse_patience = ticks;
+    return BCMGX_OK;
+}
+
 // ------------------------------------------------------ kernel-level API ---
 int bcmgx_spmv(bcmgx_context ctx, bcmgx_matrix A, const double* x, double* y, double alpha, double beta, int op, int lanes, int mem) {
     if (!ctx || !A || !x || !y || op < 0 || op > 2) return BCMGX_ERR_ARG;

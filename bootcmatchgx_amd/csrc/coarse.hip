@@ -1,0 +1,359 @@
+// coarse.hip -- all the l1-Jacobi sweeps of the coarsest level in one launch
+// (relaxCoarsest, GAMG_cycle.cu:186; _jacobi_it_full<0>, l1jacobi.cu:344-379).
+//
+// The coarsest operator has a few thousand rows (max_coarse_size: 40 cbrt(N))
+// and the cycle sweeps it 20 times.  As 20 launches each sweep costs 2.4-4.6 us
+// of dispatch and dependent memory round trips for 0.1-0.5 us of data (about 90 us
+// per cycle at 27-point 128^3, one right-hand side).  Here one launch does them
+// all: every lane keeps its matrix entries in registers, and the iterate moves
+// between the workgroups through memory, or through LDS when one workgroup
+// holds the level.
+//
+// Same bits as the launches it replaces: a row is summed by the same number of
+// lanes with the same stride and the same shuffle tree as k_spmv1, and the
+// update is the same expression.
+#include "kernels.h"
+
+namespace bcmgx {
+
+constexpr int CO_ROWS = 32;          // rows per workgroup of the exchanging kernel
+constexpr int CO_FETCH = 4;          // listed columns a thread of it fetches
+constexpr int CO_SMALL_T = 1024;    // threads of the one-workgroup kernel
+constexpr int CO_SMALL_N = 1024;    // rows it holds in LDS
+constexpr int CO_SMALL_RR = 4;      // rows per lane group there
+constexpr int CO_SMALL_E = 4;       // entries per lane and row there
+
+typedef unsigned long long u64;
+
+// the sum over a row's L lanes, in every lane
+template <int L>
+__device__ __forceinline__ double group_sum(double t) {
+#pragma unroll
+    for (int o = L / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, L);
+    return t;
+}
+
+// a row's entries of this lane: lane, lane + L, ... from the row's start
+template <int L, int E>
+struct RowPart {
+    double a[E];
+    int c[E];  // -1: no entry
+    __device__ __forceinline__ void load(bool on, int r, int lane, const int* __restrict__ row, const int* __restrict__ col,
+                                         const double* __restrict__ val) {
+        int s = 0, e = 0;
+        if (on) {
+            s = row[r];
+            e = row[r + 1];
+        }
+#pragma unroll
+        for (int q = 0; q < E; q++) {
+            int j = s + lane + q * L;
+            c[q] = j < e ? col[j] : -1;
+            a[q] = j < e ? val[j] : 0.0;
+        }
+    }
+    __device__ __forceinline__ double sum(const double* xv) const {
+        double t = 0;
+#pragma unroll
+        for (int q = 0; q < E; q++)
+            if (c[q] >= 0) t += a[q] * xv[q];
+        return group_sum<L>(t);
+    }
+};
+
+// The exchanging kernel: a workgroup owns CO_ROWS rows, L lanes each.  An
+// iterate's element travels as two 64-bit words, each half of the double with a
+// 32-bit tag beside it, written and read with device scope: a reader that finds
+// both tags has the value, so there is no barrier over the grid and no separate
+// flag to wait for.  A workgroup fetches each distinct column of its rows once
+// per sweep (the list made at setup, sorted, so neighbouring threads read
+// neighbouring elements) and its lanes take them from LDS: with every lane
+// fetching its own entries' elements a sweep of the 4096 rows of 27-point 128^3
+// took 4 us, bound by the 100 K scattered requests.  Each sweep has its own
+// slots, so a workgroup that runs ahead overwrites nothing, and tags rise from
+// launch to launch (ctl[0]), so nothing is cleared.  The first sweep from zero,
+// f / D, is formed by every reader itself.
+//
+// The waits need the workgroups to run at the same time.  The launcher keeps the
+// grid to half of what the device holds; whatever else occupies it, each
+// wait is bounded: a workgroup that waits longer than `patience` clock ticks
+// raises ctl[2], all give up, and the workgroup that finishes last computes the
+// sweeps alone.  Workgroups that had their values wrote the same ones.
+template <typename V, int L, int E>
+__global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
+    int n, const int* __restrict__ row, const int* __restrict__ col, const double* __restrict__ val,
+    const double* __restrict__ D, const V* __restrict__ f, const V* __restrict__ x0, V* __restrict__ out, int sweeps,
+    const int* __restrict__ ucnt, const int* __restrict__ ucol, const unsigned short* __restrict__ upos, u64* slots,
+    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience) {
+    constexpr int T = CO_ROWS * L, NU = CO_FETCH;
+    if (stop && *stop) return;
+    __shared__ double xs[2][TILE_MAX_COLS];
+    __shared__ int s_late, s_last;
+    int tid = threadIdx.x, lane = tid % L;
+    int r = blockIdx.x * CO_ROWS + tid / L;
+    bool on = r < n;
+    unsigned base = ctl[0];
+    if (tid == 0) s_late = 0;
+    int rs = on ? row[r] : 0, re = on ? row[r + 1] : 0;
+    // the listed columns this thread fetches (-1: none) and its entries' places among them;
+    // a tile without a list (too many entries or columns) has every lane fetch its own
+    // entries' elements, one after another
+    int U = ucnt[blockIdx.x];
+    bool listed = U > 0 && U <= NU * T;
+    int uc[NU], at[E];
+    double a[E];
+#pragma unroll
+    for (int w = 0; w < NU; w++)
+        uc[w] = listed && tid + w * T < U ? ucol[(size_t)blockIdx.x * TILE_MAX_COLS + tid + w * T] : -1;
+#pragma unroll
+    for (int q = 0; q < E; q++) {
+        int j = rs + lane + q * L;
+        at[q] = listed && j < re ? upos[j] : -1;
+        a[q] = listed && j < re ? val[j] : 0.0;
+    }
+    double fr = on ? (double)f[r] : 0.0, Dr = on ? D[r] : 1.0;
+    double xr;
+    int done = x0 ? 0 : 1;
+    // the iterate that costs no exchange: the guess, or the sweep from zero ((-0 + f) / D) + 0
+    auto first = [&](int c) { return x0 ? (double)x0[c] : (double)f[c] / D[c]; };
+    xr = x0 ? (on ? (double)x0[r] : 0.0) : fr / Dr;
+    bool given_up = false;  // uniform over the workgroup
+    for (int s = done; s < sweeps; s++) {
+        double* xc = xs[s & 1];
+        double t = 0;
+        if (s == done) {
+            if (listed) {
+#pragma unroll
+                for (int w = 0; w < NU; w++)
+                    if (uc[w] >= 0) xc[tid + w * T] = first(uc[w]);
+            } else {
+                for (int j = rs + lane; j < re; j += L) t += val[j] * first(col[j]);
+            }
+        } else {  // the elements that sweep s - 1 published
+            const u64* p = slots + (size_t)(s - 1) * n * 2;
+            unsigned tag = base + (unsigned)s;
+            auto fetch = [&](int c, double& v) {
+                u64 lo = __hip_atomic_load(p + (size_t)c * 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                u64 hi = __hip_atomic_load(p + (size_t)c * 2 + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                v = __hiloint2double((int)(unsigned)hi, (int)(unsigned)lo);
+                return (unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag;
+            };
+            long long t0 = 0;
+            bool late = patience < 0;  // negative: no waiting at all
+            int j = rs + lane;         // without a list: the entry waited for
+            for (int poll = 0; !late; poll++) {
+                bool ready = true;
+                if (listed) {
+                    double v[NU];
+                    bool ok[NU];
+#pragma unroll
+                    for (int w = 0; w < NU; w++) ok[w] = uc[w] < 0 || fetch(uc[w], v[w]);
+#pragma unroll
+                    for (int w = 0; w < NU; w++) {
+                        if (uc[w] >= 0 && ok[w]) xc[tid + w * T] = v[w];
+                        ready = ready && ok[w];
+                    }
+                } else {
+                    double v;
+                    while (j < re && fetch(col[j], v)) {
+                        t += val[j] * v;
+                        j += L;
+                    }
+                    ready = j >= re;
+                }
+                if (ready) break;
+                if ((poll & 15) == 15) {
+                    if (poll == 15) t0 = wall_clock64();
+                    else if (wall_clock64() - t0 > patience) late = true;
+                    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) late = true;
+                }
+            }
+            if (late) {
+                s_late = s + 1;
+                __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __syncthreads();  // the other half of xs is written before the next one
+        if (s_late == s + 1) {  // not a faster wave's of the next sweep
+            given_up = true;
+            break;
+        }
+        if (listed) {
+#pragma unroll
+            for (int q = 0; q < E; q++)
+                if (at[q] >= 0) t += a[q] * xc[at[q]];
+        }
+        t = group_sum<L>(t);
+        xr = ((-t + fr) / Dr) + xr;
+        if (s + 1 < sweeps && on && lane == 0) {
+            u64* p = slots + ((size_t)s * n + r) * 2;
+            u64 tag = (u64)(base + (unsigned)s + 1u) << 32;
+            __hip_atomic_store(p, tag | (unsigned)__double2loint(xr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(p + 1, tag | (unsigned)__double2hiint(xr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    if (!given_up && on && lane == 0) out[r] = (V)xr;
+    __syncthreads();
+    if (tid == 0) {
+        __threadfence();
+        s_last = atomicAdd(ctl + 1, 1u) == gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the last workgroup: every other one has passed its waits for good
+    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        double* cur = scratch;
+        double* nxt = scratch + n;
+        for (int i = tid; i < n; i += T) cur[i] = first(i);
+        __threadfence();
+        __syncthreads();
+        for (int s = done; s < sweeps; s++) {
+            for (int i0 = 0; i0 < n; i0 += CO_ROWS) {
+                int i = i0 + tid / L;
+                double t = 0;
+                if (i < n)
+                    for (int j = row[i] + lane; j < row[i + 1]; j += L) t += val[j] * cur[col[j]];
+                t = group_sum<L>(t);
+                if (i < n && lane == 0) nxt[i] = ((-t + (double)f[i]) / D[i]) + cur[i];
+            }
+            __threadfence();
+            __syncthreads();
+            double* w = cur;
+            cur = nxt;
+            nxt = w;
+        }
+        for (int i = tid; i < n; i += T) out[i] = (V)cur[i];
+        __syncthreads();
+    }
+    if (tid == 0) {
+        ctl[0] = base + (unsigned)sweeps + 1u;
+        ctl[1] = 0;
+        ctl[2] = 0;
+    }
+}
+
+// The one-workgroup kernel: the iterate in LDS, one barrier per sweep.
+template <typename V, int L>
+__global__ __launch_bounds__(CO_SMALL_T) void k_coarse_small(int n, const int* __restrict__ row, const int* __restrict__ col,
+                                                             const double* __restrict__ val, const double* __restrict__ D,
+                                                             const V* __restrict__ f, const V* __restrict__ x0,
+                                                             V* __restrict__ out, int sweeps, const int* __restrict__ stop) {
+    if (stop && *stop) return;
+    constexpr int RR = CO_SMALL_RR, E = CO_SMALL_E, G = CO_SMALL_T / L;
+    __shared__ double xs[2][CO_SMALL_N];
+    int lane = threadIdx.x % L, g = threadIdx.x / L;
+    RowPart<L, E> part[RR];
+    double fr[RR], Dr[RR], xr[RR];
+#pragma unroll
+    for (int w = 0; w < RR; w++) {
+        int r = w * G + g;
+        bool on = r < n;
+        part[w].load(on, r, lane, row, col, val);
+        fr[w] = on ? (double)f[r] : 0.0;
+        Dr[w] = on ? D[r] : 1.0;
+        xr[w] = x0 ? (on ? (double)x0[r] : 0.0) : fr[w] / Dr[w];
+        if (on && lane == 0) xs[0][r] = xr[w];
+    }
+    __syncthreads();
+    int cur = 0;
+    for (int s = x0 ? 0 : 1; s < sweeps; s++) {
+#pragma unroll
+        for (int w = 0; w < RR; w++) {
+            if (w * G >= n) break;  // uniform
+            double xv[E];
+#pragma unroll
+            for (int q = 0; q < E; q++) xv[q] = part[w].c[q] >= 0 ? xs[cur][part[w].c[q]] : 0.0;
+            double t = part[w].sum(xv);
+            xr[w] = ((-t + fr[w]) / Dr[w]) + xr[w];
+            int r = w * G + g;
+            if (r < n && lane == 0) xs[cur ^ 1][r] = xr[w];
+        }
+        cur ^= 1;
+        __syncthreads();
+    }
+#pragma unroll
+    for (int w = 0; w < RR; w++) {
+        int r = w * G + g;
+        if (r < n && lane == 0) out[r] = (V)xr[w];
+    }
+}
+
+template <typename V, int L, int E>
+static bool launch_exchange(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int sweeps,
+                            const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+    auto kern = k_coarse_exchange<V, L, E>;
+    static int resident = 0;  // workgroups the device holds, per instantiation; identical devices assumed within a process
+    if (!resident) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, CO_ROWS * L, 0) != hipSuccess) per_cu = 0;
+        resident = c->num_cus * per_cu + 1;
+    }
+    unsigned grid = grid_for(A.n, CO_ROWS);
+    if ((long long)grid * 2 > resident) return false;
+    kern<<<grid, CO_ROWS * L, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, sweeps,
+                                              ix.ucnt.get(), ix.ucol.get(), ix.upos.get(), cs.slots.get(),
+                                              cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience);
+    BCMGX_LAUNCHED();
+    return true;
+}
+
+void CoarseIndex::build(Context* c, const DCsr& A) {
+    if (A.n <= 0 || A.n > CO_MAX_N) return;
+    unsigned nt = grid_for(A.n, CO_ROWS);
+    ucnt.reset(c, nt);
+    ucol.reset(c, (size_t)nt * TILE_MAX_COLS);
+    upos.reset(c, (size_t)std::max(A.nnz, 2));
+    tile_columns_strided(c, A, CO_ROWS, ucnt.get(), ucol.get(), upos.get());
+}
+
+void CoarseSync::reserve(Context* c, int n, int sweeps) {
+    size_t need = (size_t)n * (size_t)std::max(sweeps, 1) * 2;
+    if (slots.size() >= need && scratch.size() >= (size_t)n * 2) return;
+    slots.reset(c, need);
+    scratch.reset(c, (size_t)n * 2);
+    ctl.reset(c, 4);
+    fill<long long>(c, (long long*)slots.get(), (long long)need, 0);
+    fill<int>(c, (int*)ctl.get(), 4, 0);
+}
+
+static bool coarse_one_workgroup(const DCsr& A, int L) {
+    return A.n <= CO_SMALL_N && (long long)A.n * L <= (long long)CO_SMALL_RR * CO_SMALL_T && A.maxrow <= CO_SMALL_E * L;
+}
+
+bool coarse_sweeps_fit(int n, int sweeps) { return n > 0 && n <= CO_MAX_N && sweeps >= 2 && sweeps <= CO_MAX_SWEEPS; }
+
+template <typename V>
+bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const V* f, const V* x0, V* out, int sweeps,
+                   const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+    int L = lanes != 0 ? lanes : default_lanes(A.nnz, A.n);
+    if (!coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || L < 2 || L > 32 || (const void*)out == (const void*)x0) return false;
+    // One workgroup while it holds the level's entries in registers (n <= 4096 / L): a
+    // sweep is then a barrier and LDS reads, 0.5 us against 1.2 us for the exchange.
+    if (coarse_one_workgroup(A, L)) {
+#define BCMGX_CS(LL)                                                                                                     \
+    case LL:                                                                                                             \
+        k_coarse_small<V, LL><<<1, CO_SMALL_T, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, \
+                                                               sweeps, stop);                                            \
+        break;
+        switch (L) { BCMGX_CS(2) BCMGX_CS(4) BCMGX_CS(8) BCMGX_CS(16) BCMGX_CS(32) }
+#undef BCMGX_CS
+        BCMGX_LAUNCHED();
+        return true;
+    }
+    if (!ix.ucnt || cs.slots.size() < (size_t)A.n * sweeps * 2 || cs.scratch.size() < (size_t)A.n * 2) return false;
+#define BCMGX_CX(LL)                                                                                         \
+    case LL:                                                                                                 \
+        if (A.maxrow <= 2 * LL) return launch_exchange<V, LL, 2>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
+        if (A.maxrow <= 4 * LL) return launch_exchange<V, LL, 4>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
+        if (A.maxrow <= 8 * LL) return launch_exchange<V, LL, 8>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
+        return false;
+    switch (L) { BCMGX_CX(2) BCMGX_CX(4) BCMGX_CX(8) BCMGX_CX(16) BCMGX_CX(32) }
+#undef BCMGX_CX
+    return false;
+}
+template bool coarse_sweeps<double>(Context*, const DCsr&, int, const double*, const double*, const double*, double*, int,
+                                    const CoarseIndex&, CoarseSync&, const int*);
+template bool coarse_sweeps<float>(Context*, const DCsr&, int, const double*, const float*, const float*, float*, int,
+                                   const CoarseIndex&, CoarseSync&, const int*);
+
+}  // namespace bcmgx

@@ -120,6 +120,8 @@ struct Context {
     size_t pinned_bytes = 0;
     // autotune cache: matrix signature -> lanes per row
     std::map<std::string, int> tuned_lanes;
+    // clock ticks (100 MHz) a wait of the one-launch coarsest sweeps may take before its fallback
+    long long coarse_patience = 500000;
     // this device's copy of the fixed scratch array of the allocation-free entry point
     void* scratch = nullptr;
 

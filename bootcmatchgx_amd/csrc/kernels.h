@@ -262,6 +262,36 @@ void prolongator_csr(Context* c, int n, int nc, const int* agg, const double* pv
 // g[k] = -sum_c lambda[row(k), c] x[col(k), c]
 void sparse_outer_grad(Context* c, const DCsr& A, const double* lambda, const double* x, int k, double* g);
 
+// per tile of `rows` rows: the distinct columns sorted at ucol[t * TILE_MAX_COLS], their number (0: over
+// the tile limits) and each entry's position in the list; nothing is read back
+void tile_columns_strided(Context* c, const DCsr& A, int rows, int* ucnt, int* ucol, unsigned short* upos);
+
+// ---- coarsest-level sweeps (coarse.hip) ---------------------------------------------
+constexpr int CO_MAX_N = 32768;      // rows and sweeps the one-launch form takes (its slots: 16 bytes per row and sweep)
+constexpr int CO_MAX_SWEEPS = 64;
+bool coarse_sweeps_fit(int n, int sweeps);
+// What the one-launch sweeps exchange through, kept with a preconditioner (one stream):
+// ctl = {tag base, finished workgroups, a wait gave up}, zero between launches but the base
+struct CoarseSync {
+    DBuf<unsigned long long> slots;  // [sweep][row][2]
+    DBuf<double> scratch;            // 2 n, for the workgroup that finishes after waits gave up
+    DBuf<unsigned> ctl;
+    void reserve(Context* c, int n, int sweeps);
+};
+// the distinct columns of each 32-row tile of a coarsest operator, listed at setup (setup.hip's
+// tile columns at a fixed stride)
+struct CoarseIndex {
+    DBuf<int> ucnt, ucol;
+    DBuf<unsigned short> upos;
+    void build(Context* c, const DCsr& A);
+};
+// `sweeps` l1-Jacobi sweeps of A (FP64) on one right-hand side in one launch: out from the guess
+// x0 (null: zero; never out itself), f and x0 widened from V, the result rounded to V; the bits of
+// sweep after sweep through k_spmv1 with `lanes`.  False (nothing launched) where it does not apply.
+template <typename V>
+bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const V* f, const V* x0, V* out, int sweeps,
+                   const CoarseIndex& ix, CoarseSync& cs, const int* stop);
+
 // ---- AFSAI (afsai.hip) ------------------------------------------------------------
 void afsai_build(Context* c, const DCsr& A, DCsr& G, DCsr& GT);
 

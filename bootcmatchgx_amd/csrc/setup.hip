@@ -1499,26 +1499,27 @@ bool galerkin(Context* c, const DCsr& A, int nc, const int* agg, const double* p
 }
 
 // ------------------------------------------------------- row-tile index ---
-// One workgroup per tile of TILE_ROWS rows: its columns sorted in LDS (bitonic,
+// One workgroup per tile of `rows` rows: its columns sorted in LDS (bitonic,
 // padded to a power of two), the distinct ones counted (phase 0) or listed and
-// every entry given its position in the list (phase 1).  A tile is indexed when
+// every entry given its position in the list (phase 1), or all of that at once
+// with the lists TILE_MAX_COLS apart (phase 2).  A tile is indexed when
 // it has entries, its paired loads from an even start fit one pass
 // (cnt + (base & 1) <= TILE_MAX_ENTRIES) and it has at most TILE_MAX_COLS
 // distinct columns; others count 0.
-__global__ __launch_bounds__(WG) void k_tile_cols(int n, const int* __restrict__ row, const int* __restrict__ col,
-                                                  int* __restrict__ ucnt, const int* __restrict__ tu,
+__global__ __launch_bounds__(WG) void k_tile_cols(int n, int rows, const int* __restrict__ row,
+                                                  const int* __restrict__ col, int* __restrict__ ucnt, const int* __restrict__ tu,
                                                   int* __restrict__ tucol, unsigned short* __restrict__ tlidx, int phase) {
     __shared__ int keys[TILE_MAX_ENTRIES];
     __shared__ int uniq[TILE_MAX_COLS];
     __shared__ int wsum[WG / 64];
     int t = blockIdx.x, tid = threadIdx.x;
-    int r0 = t * TILE_ROWS;
-    int rend = r0 + TILE_ROWS < n ? r0 + TILE_ROWS : n;
+    int r0 = t * rows;
+    int rend = r0 + rows < n ? r0 + rows : n;
     int base = row[r0], cnt = row[rend] - base;
     bool fits = cnt > 0 && cnt + (base & 1) <= TILE_MAX_ENTRIES;
     if (phase == 1 && tu[t + 1] == tu[t]) return;  // not indexed
     if (!fits) {
-        if (phase == 0 && tid == 0) ucnt[t] = 0;
+        if (phase != 1 && tid == 0) ucnt[t] = 0;
         return;
     }
     int P = 1;
@@ -1553,18 +1554,18 @@ __global__ __launch_bounds__(WG) void k_tile_cols(int n, const int* __restrict__
         __syncthreads();
         int off = carry;
         for (int q = 0; q < w; q++) off += wsum[q];
-        if (phase == 1 && head && off + below < TILE_MAX_COLS) uniq[off + below] = keys[p];
+        if (phase != 0 && head && off + below < TILE_MAX_COLS) uniq[off + below] = keys[p];
         int tot = 0;
         for (int q = 0; q < WG / 64; q++) tot += wsum[q];
         carry += tot;
         __syncthreads();
     }
     int U = carry <= TILE_MAX_COLS ? carry : 0;
-    if (phase == 0) {
+    if (phase != 1) {
         if (tid == 0) ucnt[t] = U;
-        return;
+        if (phase == 0 || U == 0) return;
     }
-    int u0 = tu[t];
+    int u0 = phase == 1 ? tu[t] : t * TILE_MAX_COLS;
     for (int u = tid; u < U; u += WG) tucol[u0 + u] = uniq[u];
     for (int j = tid; j < cnt; j += WG) {
         int c = col[base + j];
@@ -1578,16 +1579,21 @@ __global__ __launch_bounds__(WG) void k_tile_cols(int n, const int* __restrict__
     }
 }
 
+void tile_columns_strided(Context* c, const DCsr& A, int rows, int* ucnt, int* ucol, unsigned short* upos) {
+    k_tile_cols<<<grid_for(A.n, rows), WG, 0, c->stream>>>(A.n, rows, A.row.get(), A.col.get(), ucnt, nullptr, ucol, upos, 2);
+    BCMGX_LAUNCHED();
+}
+
 void build_tile_index(Context* c, DCsr& A) {
     if (A.tiled() || A.n <= 0) return;
     int nt = (A.n + TILE_ROWS - 1) / TILE_ROWS;
     DBuf<int> cnt(c, nt), tu(c, (size_t)nt + 1);
-    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), cnt.get(), nullptr, nullptr, nullptr, 0);
+    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, TILE_ROWS, A.row.get(), A.col.get(), cnt.get(), nullptr, nullptr, nullptr, 0);
     BCMGX_LAUNCHED();
     long long tot = scan_exclusive(c, cnt.get(), tu.get(), nt);
     DBuf<int> tucol(c, (size_t)std::max<long long>(tot, 1));
     DBuf<unsigned short> tlidx(c, (size_t)std::max(A.nnz, 2));
-    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), cnt.get(), tu.get(), tucol.get(), tlidx.get(), 1);
+    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, TILE_ROWS, A.row.get(), A.col.get(), cnt.get(), tu.get(), tucol.get(), tlidx.get(), 1);
     BCMGX_LAUNCHED();
     A.tu = std::move(tu);
     A.tucol = std::move(tucol);
