@@ -7,7 +7,11 @@
 // per cycle at 27-point 128^3, one right-hand side).  Here one launch does them
 // all: every lane keeps its matrix entries in registers, and the iterate moves
 // between the workgroups through memory, or through LDS when one workgroup
-// holds the level.
+// holds the level.  Measured for 20 sweeps, the launches it replaces -> here:
+// 4096 rows (27-point 128^3) 92 -> 42 us, 1954 rows (7-point 50^3) 55 -> 28 us,
+// 250 rows (7-point 10^3) 50 -> 12 us, 11270 rows (7-point diffusion 160^3)
+// 102 -> 77 us.  What is left is the latency of a store and of the loads that
+// find it, 2 us a sweep across the XCDs' L2s.
 //
 // Same bits as the launches it replaces: a row is summed by the same number of
 // lanes with the same stride and the same shuffle tree as k_spmv1, and the
@@ -69,7 +73,7 @@ struct RowPart {
 // per sweep (the list made at setup, sorted, so neighbouring threads read
 // neighbouring elements) and its lanes take them from LDS: with every lane
 // fetching its own entries' elements a sweep of the 4096 rows of 27-point 128^3
-// took 4 us, bound by the 100 K scattered requests.  Each sweep has its own
+// took 4 us, bound by the 100 K scattered requests (2.1 us with the list).  Each sweep has its own
 // slots, so a workgroup that runs ahead overwrites nothing, and tags rise from
 // launch to launch (ctl[0]), so nothing is cleared.  The first sweep from zero,
 // f / D, is formed by every reader itself.
@@ -328,7 +332,7 @@ bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const 
     int L = lanes != 0 ? lanes : default_lanes(A.nnz, A.n);
     if (!coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || L < 2 || L > 32 || (const void*)out == (const void*)x0) return false;
     // One workgroup while it holds the level's entries in registers (n <= 4096 / L): a
-    // sweep is then a barrier and LDS reads, 0.5 us against 1.2 us for the exchange.
+    // sweep is then a barrier and LDS reads, 0.5 us against 1.4-2 us for the exchange.
     if (coarse_one_workgroup(A, L)) {
 #define BCMGX_CS(LL)                                                                                                     \
     case LL:                                                                                                             \
