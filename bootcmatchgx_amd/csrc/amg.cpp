@@ -150,6 +150,16 @@ int tune_chunk(Context* c, const DCsr& A, bool fp32, int k) {
     return best;
 }
 
+// One-column products with an AFSAI factor: the CSR-stream kernel with 8 lanes a row.  The
+// factors hold up to 31 entries a row left of the diagonal over scattered columns, so 16 or 32
+// lanes a row leave most of a wave's loads uncoalesced: at 27-point 128^3 G / G^T take 289 / 308 us
+// with 32 lanes a row and 157 / 163 us streamed (40^3: 10.3 / 11.9 and 6.5 / 7.2 us), 4 lanes 159 /
+// 177 us (G^T's longer blocks leave the LDS tile).  Short rows and small factors, where a launch is
+// latency, keep the lanes of their row length.
+static int factor_lanes(const DCsr& G) {
+    return G.n >= 16384 && (long long)G.nnz >= 8ll * G.n ? -8 : default_lanes(G.nnz, G.n);
+}
+
 // ----------------------------------------------------------- hierarchy ----
 // setMaxCoarseSize (AMG.cu:238-241), truncation included
 static int reference_max_coarse_size(long long n) { return (int)(40 * std::pow((double)n, (double)1. / 3.)); }
@@ -883,8 +893,8 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
         break;
     case BCMGX_PREC_AFSAI:
         afsai_build(c, A, pr->G, pr->GT);
-        pr->lanesG = default_lanes(pr->G.nnz, pr->G.n);
-        pr->lanesGT = default_lanes(pr->GT.nnz, pr->GT.n);
+        pr->lanesG = factor_lanes(pr->G);
+        pr->lanesGT = factor_lanes(pr->GT);
         break;
     case BCMGX_PREC_BCMG: {
         BCMGX_CHECK(p.aggr_type == 0, BCMGX_ERR_UNSUPPORTED, "aggr_type != 0 is not supported");
