@@ -97,7 +97,7 @@ static float time_spmm(Context* c, const DCsr& A, const void* val, int k, int ch
     fill<V>(c, x.get(), (long long)A.m * k, (V)1);
     SpmvArgs a;
     a.n = A.n; a.row = A.row.get(); a.col = A.col.get(); a.val = val; a.nnz = A.nnz;
-    a.x = x.get(); a.y = y.get(); a.k = k; a.kchunk = chunk;
+    a.x = x.get(); a.y = y.get(); a.k = k; a.kchunk = chunk; a.blk = &A.blk;
     spmv<V, V>(c, SpOp::AX, a);
     BCMGX_HIP(hipEventRecord(e0, c->stream));
     for (int r = 0; r < 3; r++) spmv<V, V>(c, SpOp::AX, a);
@@ -111,7 +111,9 @@ static float time_spmm(Context* c, const DCsr& A, const void* val, int k, int ch
 int tune_chunk(Context* c, const DCsr& A, bool fp32, int k) {
     if (k <= 4 || A.n < 65536) return k;
     if (fp32 && !A.valf) throw Error(BCMGX_ERR_STATE, "tune_chunk: FP32 values not built");
-    std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + (fp32 ? "f" : "d") + ":k" + std::to_string(k);
+    bool blocks = fp32 && A.blk.built() && A.blk.val32 && blk_width(k);
+    std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + (fp32 ? "f" : "d") + ":k" + std::to_string(k) +
+                      (blocks ? "b" : "");
     auto it = c->tuned_lanes.find(sig);
     if (it != c->tuned_lanes.end()) return it->second;
     hipEvent_t e0, e1;
@@ -135,6 +137,7 @@ int tune_chunk(Context* c, const DCsr& A, bool fp32, int k) {
             cands.push_back(-16 - lg);
         }
     }
+    if (blocks) cands.push_back(BLK_CODE);  // the block form on the matrix cores
     for (int ch = (k + 1) / 2; ch >= 4; ch = (ch + 1) / 2) {
         cands.push_back(ch);
         if (ch == 4) break;
@@ -406,6 +409,8 @@ struct SolveWork {
     bool z32 = false;
     DBuf<float> zf;
     int z32_blocks = 0;
+    int z32_blk = 0;    // the fused product from the block form: its kchunk code (0: k_spmmp) and grid
+    int z32_blk_grid = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     hipGraph_t cg_graph = nullptr;  // one CG iteration
@@ -440,6 +445,14 @@ void Prec::ensure_work(int k) {
     if (ptype == BCMGX_PREC_BCMG && k > 1 && k != tuned_k) {
         // SpMM column chunk for this batch width (tuned outside any graph capture)
         bool f32 = p.precision == BCMGX_PRECISION_FP32;
+        // the caller's matrix in block form (its pattern once, kept with the matrix) for the FP32
+        // cycle's products with it: rows of 6 entries and more, which can share columns
+        if (f32 && p.autotune && blk_width(k) && A->n >= 65536 && (long long)A->nnz >= 6ll * A->n) {
+            DCsr& M = const_cast<DCsr&>(*A);
+            const Level& l0 = *H.L[0];
+            // tiles of rows that aggregate together share the most columns
+            if (H.levels() > 1 && l0.R.nnz == A->n && build_blocks(ctx, M, l0.R.col.get())) block_values32(ctx, M);
+        }
         for (int h = 0; h < n_hrc(); h++)
             for (auto& lp : hrc(h).L) lp->chunkA = p.autotune ? tune_chunk(ctx, lp->mat(), f32, k) : k;
         tuned_k = k;
@@ -958,16 +971,27 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
 // The same iteration with z in FP32: the direction d and its image q are updated
 // in place (no ping-pong), w holds A z.  The same operations in the same order as
 // the widened-FP64 iteration; only the dot products group their sums differently.
-static void fcg_iteration_z32(Context* c, const DCsr& A, Prec* prec, SolveWork& s, int idx) {
-    const int* stop = s.flags.get();
-    prec->apply_entry_f32(s.r.get(), s.zf.get(), s.k, stop);
+// w = A z and the dot products' partials; returns their number
+static int fused_z32(Context* c, const DCsr& A, SolveWork& s, const double* wold, const int* stop, const int* all_done) {
     SpmvArgs a;
     a.n = A.n; a.row = A.row.get(); a.col = A.col.get(); a.val = A.val.get(); a.nnz = A.nnz;
     set_tiles(a, A);
-    a.x = s.zf.get(); a.y = s.w.get(); a.k = s.k; a.lanes = s.lanesA; a.stop = stop; a.kchunk = s.chunkA;
-    BCMGX_CHECK(spmm_dots_z32(c, a, s.r.get(), s.q.get(), s.fb.partials, s.z32_blocks, s.fb.all_done), BCMGX_ERR_STATE,
+    a.x = s.zf.get(); a.y = s.w.get(); a.k = s.k; a.lanes = s.lanesA; a.stop = stop;
+    if (s.z32_blk) {
+        a.kchunk = s.z32_blk;
+        if (spmm_blocked_dots(c, a, s.r.get(), wold, s.fb.partials, s.z32_blk_grid, all_done)) return s.z32_blk_grid;
+    }
+    a.kchunk = s.chunkA;
+    BCMGX_CHECK(spmm_dots_z32(c, a, s.r.get(), wold, s.fb.partials, s.z32_blocks, all_done), BCMGX_ERR_STATE,
                 "fused FP32-z product not applicable");
-    fcg_scalars3(c, s.fb, s.z32_blocks, idx);
+    return s.z32_blocks;
+}
+
+static void fcg_iteration_z32(Context* c, const DCsr& A, Prec* prec, SolveWork& s, int idx) {
+    const int* stop = s.flags.get();
+    prec->apply_entry_f32(s.r.get(), s.zf.get(), s.k, stop);
+    int nblk = fused_z32(c, A, s, s.q.get(), stop, s.fb.all_done);
+    fcg_scalars3(c, s.fb, nblk, idx);
     fcg_update_z32(c, s.fb, s.zf.get(), s.d.get(), s.w.get(), s.q.get(), s.X.get(), s.r.get(), idx, s.entry);
     fcg_finish_iteration(c, s.fb, idx);
 }
@@ -1017,7 +1041,8 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
         s.fb.nblk = fcg_partial_blocks(n);
         s.mv_blocks = spmm_dots_blocks(c, n, k);
         s.z32_blocks = spmm_dots_z32_blocks(c, n, k);
-        s.partials.reset(c, (size_t)std::max({s.fb.nblk, s.mv_blocks, s.z32_blocks}) * k * 3);
+        s.z32_blk_grid = spmm_blocked_dots_blocks(c, k);
+        s.partials.reset(c, (size_t)std::max({s.fb.nblk, s.mv_blocks, s.z32_blocks, s.z32_blk_grid}) * k * 3);
         s.st.reset(c, k);
         s.flags.reset(c, 3);
         s.fb.partials = s.partials.get();
@@ -1044,6 +1069,13 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     s.fused = prec->fused_entry(k, &s.entry);
     // z in FP32 when the FP32 cycle is entered from the update and the fused FP32-z product applies
     bool z32 = s.fused && p.fcg_z32 && s.z32_blocks > 0 && s.z32_blocks % 8 == 0 && (s.chunkA <= 0 || s.chunkA >= k);
+    // where the cycle's products with A run from the block form, so does the fused product
+    int blk = z32 && s.z32_blk_grid > 0 && prec->H.L[0]->chunkA == BLK_CODE &&
+                      block_values64(c, const_cast<DCsr&>(A))
+                  ? BLK_CODE
+                  : 0;
+    if (blk != s.z32_blk) s.drop_graph();
+    s.z32_blk = blk;
     if (z32 != s.z32) s.drop_graph();  // the captured iterations differ
     s.z32 = z32;
     if (s.z32 && !s.zf) s.zf.reset(c, (size_t)std::max(n, 1) * k);
@@ -1075,13 +1107,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
         // v = B r kept in FP32; w = A v with (r.v, w.v) in the fused product (its third
         // dot, against r here, is not used)
         prec->apply_entry_f32(s.r.get(), s.zf.get(), k, nullptr);
-        SpmvArgs a;
-        a.n = n; a.row = A.row.get(); a.col = A.col.get(); a.val = A.val.get(); a.nnz = A.nnz;
-        set_tiles(a, A);
-        a.x = s.zf.get(); a.y = s.w.get(); a.k = k; a.lanes = s.lanesA; a.kchunk = s.chunkA;
-        BCMGX_CHECK(spmm_dots_z32(c, a, s.r.get(), s.r.get(), s.fb.partials, s.z32_blocks, nullptr), BCMGX_ERR_STATE,
-                    "fused FP32-z product not applicable");
-        fcg_init_scalars(c, s.fb, s.z32_blocks);
+        fcg_init_scalars(c, s.fb, fused_z32(c, A, s, s.r.get(), nullptr, nullptr));
         fcg_init_update_z32(c, s.fb, s.X.get(), s.r.get(), s.zf.get(), s.w.get(), s.d.get(), s.q.get(), s.entry);
     } else {
         prec->apply(s.r.get(), s.v.get(), k, true, nullptr, s.fused);

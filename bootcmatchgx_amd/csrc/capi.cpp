@@ -292,6 +292,7 @@ int bcmgx_csr_update_values(bcmgx_matrix A, const double* val, int mem) {
         BCMGX_HIP(hipMemcpyAsync(M.val.get(), val, sizeof(double) * (size_t)M.nnz, k, c->stream));
         // an FP32 copy (built by an FP32 hierarchy on this matrix) follows the new values
         if (M.valf) convert<double, float>(c, M.val.get(), M.valf.get(), M.nnz);
+        refresh_blocks(c, M);
         // so do the level-0 divisors of the preconditioners set up on it
         for (auto* p : A->ctx->precs)
             if (p->A == A && p->P) p->P->refresh_level0();
@@ -593,6 +594,56 @@ int bcmgx_internal_coarse_patience(bcmgx_context ctx, long long ticks) {
     if (!ctx) return BCMGX_ERR_ARG;
     ctx->c->coarse_patience = ticks;
     return BCMGX_OK;
+}
+
+// Not part of the public interface: one product of the block form (blocked.hip) over tiles of
+// 16 rows in `order`, on host arrays of k interleaved columns.  op 1: y = A x, 2: y = b - A x (b
+// FP32), 3: the Jacobi sweep with D, 4: b in FP64 and y = b - A x, all FP32; 5: y = A x in FP64 with
+// the column sums of (r x, y x, wold x) in dots, r and wold the two halves of b.
+int bcmgx_internal_block_product(bcmgx_context ctx, bcmgx_matrix A, const int* order, int k, int op, const float* x,
+                                 const void* b, const float* D, void* y, double* dots) {
+    if (!ctx || !A || !order || !x || !y || !blk_width(k) || op < 1 || op > 5) return BCMGX_ERR_ARG;
+    API_BEGIN
+    Context* c = ctx->c;
+    BCMGX_HIP(hipSetDevice(c->device));
+    DCsr& M = A->A;
+    size_t nx = (size_t)M.m * k, ny = (size_t)M.n * k;
+    DBuf<int> ord(c, M.n);
+    c->h2d(ord.get(), order, M.n);
+    BCMGX_CHECK(build_blocks(c, M, ord.get(), 0.0), BCMGX_ERR_UNSUPPORTED, "no block form of this matrix");
+    DBuf<float> X(c, nx), Y(c, ny), Bf(c, ny), Df(c, M.n);
+    DBuf<double> Y64(c, ny), B64(c, 2 * ny);
+    c->h2d(X.get(), x, nx);
+    SpmvArgs a;
+    a.n = M.n; a.row = M.row.get(); a.nnz = M.nnz; a.k = k; a.kchunk = BLK_CODE; a.blk = &M.blk;
+    a.x = X.get(); a.y = Y.get();
+    bool ran;
+    if (op == 5) {
+        block_values64(c, M);
+        c->h2d(B64.get(), (const double*)b, 2 * ny);
+        int nblk = spmm_blocked_dots_blocks(c, k);
+        DBuf<double> part(c, (size_t)nblk * k * 3);
+        a.y = Y64.get();
+        ran = spmm_blocked_dots(c, a, B64.get(), B64.get() + ny, part.get(), nblk, nullptr);
+        std::vector<double> h((size_t)nblk * k * 3);
+        c->d2h(h.data(), part.get(), h.size());
+        for (int j = 0; j < 3 * k; j++) dots[j] = 0;
+        for (int i = 0; i < nblk; i++)
+            for (int j = 0; j < 3 * k; j++) dots[j] += h[(size_t)i * 3 * k + j];
+        c->d2h((double*)y, Y64.get(), ny);
+    } else {
+        block_values32(c, M);
+        if (op == 2 || op == 3) c->h2d(Bf.get(), (const float*)b, ny);
+        if (op == 3) c->h2d(Df.get(), D, M.n);
+        if (op == 4) c->h2d(B64.get(), (const double*)b, ny);
+        a.b = op == 4 ? nullptr : Bf.get();
+        a.b64 = op == 4 ? B64.get() : nullptr;
+        a.D = Df.get();
+        ran = spmm_blocked_f32(c, op == 1 ? SpOp::AX : op == 3 ? SpOp::JACOBI : SpOp::RES, a);
+        c->d2h((float*)y, Y.get(), ny);
+    }
+    return ran ? BCMGX_OK : BCMGX_ERR_UNSUPPORTED;
+    API_END(ctx)
 }
 
 // ------------------------------------------------------ kernel-level API ---

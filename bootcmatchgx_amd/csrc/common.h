@@ -196,6 +196,24 @@ constexpr int TILE_ROWS = 64;
 constexpr int TILE_MAX_ENTRIES = 2048;
 constexpr int TILE_MAX_COLS = 1024;
 
+// The 16-row block form of a matrix for k-column products on the matrix cores
+// (blocked.hip), built on demand and kept with the matrix.
+constexpr int BLK_ROWS = 16;
+struct BlockForm {
+    DBuf<int> rows;                 // the tiles' rows, BLK_ROWS each
+    DBuf<int> vptr;                 // tile -> its first value
+    DBuf<int> gptr, bptr;           // tile -> first group of four columns; first block of 16 groups' columns
+    DBuf<int> col;                  // 64 per block
+    DBuf<unsigned long long> mask;  // per group
+    DBuf<unsigned short> upos;      // per CSR entry: its column's place in the tile's list
+    DBuf<float> val32;              // values in block order (either may be absent)
+    DBuf<double> val64;
+    int m = 0;                      // columns of the matrix
+    long long groups = 0;
+    bool refused = false;           // the pattern shares too few columns
+    bool built() const { return (bool)mask; }
+};
+
 struct DCsr {
     int n = 0, m = 0, nnz = 0;
     DBuf<int> row, col;
@@ -203,6 +221,7 @@ struct DCsr {
     DBuf<float> valf;  // FP32 copy for the mixed-precision cycle (may be empty)
     DBuf<int> tu, tucol;            // row-tile index (empty until built)
     DBuf<unsigned short> tlidx;
+    BlockForm blk;                  // block form (empty until built)
     bool unit_rows = false;         // row i holds exactly entry i (row pointers 0, 1, .., n): a prolongator
     int maxrow = -1;                // entries in the longest row (-1: not known)
     bool tiled() const { return (bool)tu; }

@@ -72,12 +72,14 @@ struct SpmvArgs {
     const int* tu = nullptr;    // the matrix's row-tile index (DCsr::tu, tucol, tlidx), or null
     const int* tucol = nullptr;
     const unsigned short* tlidx = nullptr;
+    const BlockForm* blk = nullptr; // the matrix's block form, used when kchunk asks for it (BLK_CODE)
 };
 // the row-tile index of A into a (k = 1 launches whose lanes code asks for the tiled kernel use it)
 inline void set_tiles(SpmvArgs& a, const DCsr& A) {
     a.tu = A.tu.get();
     a.tucol = A.tucol.get();
     a.tlidx = A.tlidx.get();
+    a.blk = &A.blk;
 }
 // build A's row-tile index (once: a built index is kept)
 void build_tile_index(Context* c, DCsr& A);
@@ -265,6 +267,25 @@ void sparse_outer_grad(Context* c, const DCsr& A, const double* lambda, const do
 // per tile of `rows` rows: the distinct columns sorted at ucol[t * TILE_MAX_COLS], their number (0: over
 // the tile limits) and each entry's position in the list; nothing is read back
 void tile_columns_strided(Context* c, const DCsr& A, int rows, int* ucnt, int* ucol, unsigned short* upos);
+
+// ---- k-column products from the block form (blocked.hip) ----------------------------
+// kchunk code of the block form; k = 8, 16, 32 or 64
+constexpr int BLK_CODE = -64;
+inline bool blk_width(int k) { return k == 8 || k == 16 || k == 32 || k == 64; }
+constexpr double BLK_MIN_REUSE = 1.5;  // entries per x row loaded below which the form is not used
+// A's block form over tiles of 16 rows taken from order (a permutation of the rows, on the device);
+// false (nothing kept) where rows are too long or share too few columns
+bool build_blocks(Context* c, DCsr& A, const int* order, double min_reuse = BLK_MIN_REUSE);
+// the values in block order, on first need; false: no memory for them
+bool block_values32(Context* c, DCsr& A);
+bool block_values64(Context* c, DCsr& A);
+void refresh_blocks(Context* c, DCsr& A);  // after A's values changed
+// AX, RES or JACOBI on FP32 columns; false where the form or the code does not apply
+bool spmm_blocked_f32(Context* c, SpOp op, const SpmvArgs& a);
+// the fused product of spmm_dots_z32 (fcg.hip's partials, over this grid)
+int spmm_blocked_dots_blocks(Context* c, int k);
+bool spmm_blocked_dots(Context* c, const SpmvArgs& a, const double* r, const double* wold, double* partials, int nblk,
+                       const int* all_done);
 
 // ---- coarsest-level sweeps (coarse.hip) ---------------------------------------------
 constexpr int CO_MAX_N = 32768;      // rows and sweeps the one-launch form takes (its slots: 16 bytes per row and sweep)

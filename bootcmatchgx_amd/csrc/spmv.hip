@@ -1034,6 +1034,14 @@ void spmv(Context* c, SpOp op, const SpmvArgs& a) {
         case SpOp::JACOBI: launch1<T, V, SpOp::JACOBI>(c, a, L); break;
         }
     } else {
+        if (a.kchunk == BLK_CODE) {  // the block form's code: only where it was built for this matrix and width
+            if constexpr (std::is_same<V, float>::value)
+                if (spmm_blocked_f32(c, op, a)) return;
+            SpmvArgs b = a;  // an operation it does not have: the pipelined kernel
+            b.kchunk = 0;
+            spmv<T, V>(c, op, b);
+            return;
+        }
         switch (op) {
         case SpOp::AX: launchk<T, V, SpOp::AX>(c, a); break;
         case SpOp::RES: launchk<T, V, SpOp::RES>(c, a); break;
