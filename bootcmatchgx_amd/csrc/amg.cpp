@@ -859,7 +859,7 @@ static void bootstrap(Context* c, const DCsr& A, Prec* pr, Build build_next) {
     while (pr->n_hrc() < p.max_hrc) {
         pr->ensure_work(1);
         DBuf<double> x(c, std::max(n, 1)), ax(c, std::max(n, 1)), zero(c, std::max(n, 1)), dots(c, solver_it + 1);
-        int nblk = fcg_partial_blocks(n);
+        int nblk = fcg_partial_blocks(n, 1);
         DBuf<double> part(c, std::max(nblk, 1));
         fill<double>(c, zero.get(), n, 0.0);
         boot_random(c, x.get(), n, (unsigned long long)pr->n_hrc());
@@ -1038,7 +1038,7 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
         s.w.reset(c, nk); s.d.reset(c, nk); s.q.reset(c, nk);
         s.fb.n = n;
         s.fb.k = k;
-        s.fb.nblk = fcg_partial_blocks(n);
+        s.fb.nblk = fcg_partial_blocks(n, k);
         s.mv_blocks = spmm_dots_blocks(c, n, k);
         s.z32_blocks = spmm_dots_z32_blocks(c, n, k);
         s.z32_blk_grid = spmm_blocked_dots_blocks(c, k);

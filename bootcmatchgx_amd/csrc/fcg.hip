@@ -7,7 +7,7 @@
 // replayed from a hipGraph and the host only polls a flag.
 //
 // Reductions are deterministic: a fixed number of partial blocks (a function
-// of n only), a fixed in-block tree, then one block per column summing the
+// of n and k only), a fixed in-block tree, then one block per column summing the
 // partials in a fixed tree.  k vectors are interleaved (x[i*k + c]); every
 // column has its own scalars and stop flag.
 #include "kernels.h"
@@ -16,37 +16,66 @@
 
 namespace bcmgx {
 
-// partial-sum blocks of the streaming FCG kernels: a function of n only, so
-// the reduction order never changes
-int fcg_partial_blocks(int n) {
-    long long b = ((long long)n + 2047) / 2048;
+// Partial-sum blocks of the streaming FCG and CG kernels: a function of n and k
+// only, so the reduction order never changes.  These kernels are bound by
+// memory, so what counts is bytes in flight: a block per 512 elements (two a
+// thread) until the 256 CUs hold four blocks each.  Counting rows alone (one
+// block per 2048 rows) left the chip idle on several columns: the update of
+// 65600 x 64 took 463 us in 33 blocks and takes 49 in 1024, 720000 x 16
+// 225 -> 132 us, 131150 x 5 (CG) 31 -> 7.5 us, 125000 x 1 6.2 -> 4.4 us.  Blocks
+// of 256 or 1024 elements are within noise of these; 2048 blocks gain 5 % at
+// 720000 x 16 and lose 8 % at 2097152 x 32 and 1-2 us in each of the two
+// kernels that sum the partials.
+int fcg_partial_blocks(int n, int k) {
+    long long b = ((long long)n * k + 511) / 512;
     if (b < 1) b = 1;
     if (b > 1024) b = 1024;
     return (int)b;
 }
 
-static inline int kpad(int k) {
-    int p = 1;
-    while (p < k) p <<= 1;
-    return p;
-}
+// the streaming kernels' split of a block: its first R * k threads (R = WG / k)
+// take R rows of k columns each, one element a thread, so a block reads
+// consecutive elements and keeps its lanes busy for any k (255 of 256 at k = 5,
+// 231 at k = 33), and s[][] holds the rows' sums in the same order as a split by
+// a power of two when k is one
+struct RowSplit {
+    int R, rl, c;
+    __device__ explicit RowSplit(int k) {
+        R = WG / k;
+        rl = threadIdx.x / k;
+        c = threadIdx.x - rl * k;
+    }
+    __device__ bool active() const { return rl < R; }
+    // s[c] <- the sum of column c over the block's R rows, in a fixed tree
+    template <int NV>
+    __device__ void sum(double (*s)[WG], int k) const {
+        int h = 1;
+        while (2 * h < R) h <<= 1;
+        for (; h > 0; h >>= 1) {
+            if (rl < h && rl + h < R)
+#pragma unroll
+                for (int m = 0; m < NV; m++) s[m][threadIdx.x] += s[m][threadIdx.x + h * k];
+            __syncthreads();
+        }
+    }
+};
 
 // NV dot products per column over a row range; partials[(blk*k + c)*3 + m]
 template <int NV>
-__global__ __launch_bounds__(WG) void k_dots(int n, int k, int KP, const double* __restrict__ a0, const double* __restrict__ b0,
+__global__ __launch_bounds__(WG) void k_dots(int n, int k, const double* __restrict__ a0, const double* __restrict__ b0,
                                              const double* __restrict__ a1, const double* __restrict__ b1,
                                              const double* __restrict__ a2, const double* __restrict__ b2,
                                              double* __restrict__ partials, const int* __restrict__ all_done) {
     if (all_done && *all_done) return;
     __shared__ double s[NV][WG];
     int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
+    const RowSplit sp(k);
+    int c = sp.c;
     double acc[NV];
 #pragma unroll
     for (int m = 0; m < NV; m++) acc[m] = 0.0;
-    if (c < k) {
-        for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+    if (sp.active()) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
             long long o = i * k + c;
             acc[0] += a0[o] * b0[o];
             if (NV > 1) acc[1] += a1[o] * b1[o];
@@ -56,13 +85,7 @@ __global__ __launch_bounds__(WG) void k_dots(int n, int k, int KP, const double*
 #pragma unroll
     for (int m = 0; m < NV; m++) s[m][tid] = acc[m];
     __syncthreads();
-    for (int st = WG / 2; st >= KP; st >>= 1) {
-        if (tid < st) {
-#pragma unroll
-            for (int m = 0; m < NV; m++) s[m][tid] += s[m][tid + st];
-        }
-        __syncthreads();
-    }
+    sp.sum<NV>(s, k);
     if (tid < k) {
 #pragma unroll
         for (int m = 0; m < NV; m++) partials[((long long)blockIdx.x * k + tid) * 3 + m] = s[m][tid];
@@ -119,15 +142,15 @@ __global__ __launch_bounds__(WG) void k_norm_final(const double* __restrict__ pa
 
 // ||r||^2 partials in k_dots<1>'s blocks and order, with the FP32 cycle's
 // level-0 entry (F = (float) r, X = F/M) written on the way, as k_update does
-__global__ __launch_bounds__(WG) void k_norm_entry(int n, int k, int KP, const double* __restrict__ r,
+__global__ __launch_bounds__(WG) void k_norm_entry(int n, int k, const double* __restrict__ r,
                                                    double* __restrict__ partials, FcgEntry e) {
-    __shared__ double s[WG];
+    __shared__ double s[1][WG];
     int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
+    const RowSplit sp(k);
+    int c = sp.c;
     double acc = 0.0;
-    if (c < k) {
-        for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+    if (sp.active()) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
             long long o = i * k + c;
             double rr = r[o];
             acc += rr * rr;
@@ -136,26 +159,21 @@ __global__ __launch_bounds__(WG) void k_norm_entry(int n, int k, int KP, const d
             e.X[o] = fv / e.M[i];
         }
     }
-    s[tid] = acc;
+    s[0][tid] = acc;
     __syncthreads();
-    for (int st = WG / 2; st >= KP; st >>= 1) {
-        if (tid < st) s[tid] += s[tid + st];
-        __syncthreads();
-    }
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[tid];
+    sp.sum<1>(s, k);
+    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
 }
 
 void fcg_norm_entry(Context* c, const FcgBufs& f, const double* r, int mode, const FcgEntry& e) {
-    int KP = kpad(f.k);
-    k_norm_entry<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, r, f.partials, e);
+    k_norm_entry<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, f.partials, e);
     BCMGX_LAUNCHED();
     k_norm_final<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, mode, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();
 }
 
 void fcg_norm(Context* c, const FcgBufs& f, const double* v, int mode) {
-    int KP = kpad(f.k);
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, v, v, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
+    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, v, v, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
     BCMGX_LAUNCHED();
     k_norm_final<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, mode, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();
@@ -177,8 +195,7 @@ __global__ __launch_bounds__(WG) void k_init_scalars(const double* __restrict__ 
 }
 
 void fcg_init_dots(Context* c, const FcgBufs& f, const double* r, const double* v, const double* w) {
-    int KP = kpad(f.k);
-    k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, r, v, w, v, nullptr, nullptr, f.partials, nullptr);
+    k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, v, w, v, nullptr, nullptr, f.partials, nullptr);
     BCMGX_LAUNCHED();
     fcg_init_scalars(c, f, f.nblk);
 }
@@ -260,8 +277,7 @@ void fcg_scalars3(Context* c, const FcgBufs& f, int nblk, int phase) {
 }
 
 void fcg_dots3(Context* c, const FcgBufs& f, const double* r, const double* p0, const double* w0, const double* w1, int phase) {
-    int KP = kpad(f.k);
-    k_dots<3><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, r, p0, w0, p0, w1, p0, f.partials, f.all_done);
+    k_dots<3><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, p0, w0, p0, w1, p0, f.partials, f.all_done);
     BCMGX_LAUNCHED();
     k_scalars3<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done, phase);
     BCMGX_LAUNCHED();
@@ -274,24 +290,24 @@ void fcg_dots3(Context* c, const FcgBufs& f, const double* r, const double* p0, 
 // phase 1 forms x = theta2' t' + (pend p1 + x) -- the two steps in the
 // reference's order, so x has the same bits -- and saves one x read and write.
 template <int PHASE>
-__global__ __launch_bounds__(WG) void k_update(int n, int k, int KP, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_update(int n, int k, const FcgState* __restrict__ st,
                                                double* __restrict__ p0, const double* __restrict__ p1,
                                                double* __restrict__ w0, const double* __restrict__ w1,
                                                double* __restrict__ x, double* __restrict__ r,
                                                double* __restrict__ partials, const int* __restrict__ all_done,
                                                FcgEntry e) {
     if (*all_done) return;
-    __shared__ double s[WG];
+    __shared__ double s[1][WG];
     int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
+    const RowSplit sp(k);
+    int c = sp.c;
     double acc = 0.0;
-    if (c < k) {
+    if (sp.active()) {
         const FcgState S = st[c];
         double mth = -S.theta, th2 = S.theta2, mth2 = -S.theta2;
         bool waiting = PHASE == 1 && S.pad1;  // the pair's first step, still to be added
         double pend = S.pend;
-        for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
             long long o = i * k + c;
             double rr;
             if (!S.done) {
@@ -319,43 +335,39 @@ __global__ __launch_bounds__(WG) void k_update(int n, int k, int KP, const FcgSt
             }
         }
     }
-    s[tid] = acc;
+    s[0][tid] = acc;
     __syncthreads();
-    for (int stp = WG / 2; stp >= KP; stp >>= 1) {
-        if (tid < stp) s[tid] += s[tid + stp];
-        __syncthreads();
-    }
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[tid];
+    sp.sum<1>(s, k);
+    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
 }
 
 void fcg_update(Context* c, const FcgBufs& f, double* p0, const double* p1, double* w0, const double* w1, double* x, double* r,
                 int phase, const FcgEntry& e) {
-    int KP = kpad(f.k);
-    if (phase == 0) k_update<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
-    else k_update<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
+    if (phase == 0) k_update<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
+    else k_update<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
     BCMGX_LAUNCHED();
 }
 
 // k_update with z in FP32 (widened exactly) and p, w updated in place
 template <int PHASE>
-__global__ __launch_bounds__(WG) void k_update_z32(int n, int k, int KP, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_update_z32(int n, int k, const FcgState* __restrict__ st,
                                                    const float* __restrict__ z, double* __restrict__ p,
                                                    const double* __restrict__ w0, double* __restrict__ w,
                                                    double* __restrict__ x, double* __restrict__ r,
                                                    double* __restrict__ partials, const int* __restrict__ all_done,
                                                    FcgEntry e) {
     if (*all_done) return;
-    __shared__ double s[WG];
+    __shared__ double s[1][WG];
     int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
+    const RowSplit sp(k);
+    int c = sp.c;
     double acc = 0.0;
-    if (c < k) {
+    if (sp.active()) {
         const FcgState S = st[c];
         double mth = -S.theta, th2 = S.theta2, mth2 = -S.theta2;
         bool waiting = PHASE == 1 && S.pad1;
         double pend = S.pend;
-        for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
             long long o = i * k + c;
             double rr;
             if (!S.done) {
@@ -383,20 +395,16 @@ __global__ __launch_bounds__(WG) void k_update_z32(int n, int k, int KP, const F
             }
         }
     }
-    s[tid] = acc;
+    s[0][tid] = acc;
     __syncthreads();
-    for (int stp = WG / 2; stp >= KP; stp >>= 1) {
-        if (tid < stp) s[tid] += s[tid + stp];
-        __syncthreads();
-    }
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[tid];
+    sp.sum<1>(s, k);
+    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
 }
 
 void fcg_update_z32(Context* c, const FcgBufs& f, const float* z, double* p, const double* w0, double* w, double* x, double* r,
                     int phase, const FcgEntry& e) {
-    int KP = kpad(f.k);
-    if (phase == 0) k_update_z32<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
-    else k_update_z32<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
+    if (phase == 0) k_update_z32<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
+    else k_update_z32<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
     BCMGX_LAUNCHED();
 }
 
@@ -426,14 +434,13 @@ void fcg_finish_iteration(Context* c, const FcgBufs& f, int phase) {
     BCMGX_LAUNCHED();
 }
 
-__global__ __launch_bounds__(WG) void k_flush_pending(int n, int k, int KP, FcgState* st, const double* __restrict__ t,
+__global__ __launch_bounds__(WG) void k_flush_pending(int n, int k, FcgState* st, const double* __restrict__ t,
                                                       double* __restrict__ x) {
-    int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
-    if (c >= k || !st[c].pad1) return;
+    const RowSplit sp(k);
+    int c = sp.c;
+    if (!sp.active() || !st[c].pad1) return;
     double pend = st[c].pend;
-    for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+    for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
         long long o = i * k + c;
         x[o] = pend * t[o] + x[o];
     }
@@ -450,8 +457,7 @@ void fcg_clear_pending(Context* c, const FcgBufs& f) {
 }
 
 void fcg_flush_pending(Context* c, const FcgBufs& f, const double* t, double* x) {
-    int KP = kpad(f.k);
-    k_flush_pending<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, t, x);
+    k_flush_pending<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, t, x);
     BCMGX_LAUNCHED();
     k_clear_pending<<<1, 64, 0, c->stream>>>(f.k, f.st);
     BCMGX_LAUNCHED();
@@ -488,8 +494,7 @@ __global__ __launch_bounds__(WG) void k_cg_init(const double* __restrict__ parti
 }
 
 void cg_init(Context* c, const FcgBufs& f, const double* r, int stopcrit) {
-    int KP = kpad(f.k);
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, r, r, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
+    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, r, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
     BCMGX_LAUNCHED();
     k_cg_init<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, stopcrit, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();
@@ -512,28 +517,26 @@ __global__ __launch_bounds__(WG) void k_cg_beta(const double* __restrict__ parti
 }
 
 // p = 1 u + beta p  (my_axpby, basic.cu:114-130; CG_HS.cu:103-107)
-__global__ __launch_bounds__(WG) void k_cg_direction(int n, int k, int KP, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_cg_direction(int n, int k, const FcgState* __restrict__ st,
                                                      const double* __restrict__ u, double* __restrict__ p,
                                                      const int* __restrict__ all_done) {
     if (*all_done) return;
-    int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
-    if (c >= k || st[c].done) return;
+    const RowSplit sp(k);
+    int c = sp.c;
+    if (!sp.active() || st[c].done) return;
     double be = st[c].theta;
-    for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+    for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
         long long o = i * k + c;
         p[o] = 1.0 * u[o] + be * p[o];
     }
 }
 
 void cg_beta_direction(Context* c, const FcgBufs& f, const double* r, const double* u, double* p) {
-    int KP = kpad(f.k);
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, r, u, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
+    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, u, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
     BCMGX_LAUNCHED();
     k_cg_beta<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
     BCMGX_LAUNCHED();
-    k_cg_direction<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, u, p, f.all_done);
+    k_cg_direction<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, u, p, f.all_done);
     BCMGX_LAUNCHED();
 }
 
@@ -557,13 +560,12 @@ __global__ __launch_bounds__(WG) void k_cg_alpha(const double* __restrict__ part
 }
 
 void cg_alpha(Context* c, const FcgBufs& f, const double* p, const double* s, const double* u, const double* r, bool first) {
-    int KP = kpad(f.k);
     if (first) {
-        k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, p, s, u, r, nullptr, nullptr, f.partials, f.all_done);
+        k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, u, r, nullptr, nullptr, f.partials, f.all_done);
         BCMGX_LAUNCHED();
         k_cg_alpha<2><<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
     } else {
-        k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, p, s, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
+        k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
         BCMGX_LAUNCHED();
         k_cg_alpha<1><<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
     }
@@ -571,20 +573,20 @@ void cg_alpha(Context* c, const FcgBufs& f, const double* p, const double* s, co
 }
 
 // x = alpha p + 1 x; r = -alpha s + 1 r (CG_HS.cu:131-132), with the ||r||^2 partials
-__global__ __launch_bounds__(WG) void k_cg_update(int n, int k, int KP, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_cg_update(int n, int k, const FcgState* __restrict__ st,
                                                   const double* __restrict__ p, const double* __restrict__ sv,
                                                   double* __restrict__ x, double* __restrict__ r,
                                                   double* __restrict__ partials, const int* __restrict__ all_done) {
     if (*all_done) return;
-    __shared__ double s[WG];
+    __shared__ double s[1][WG];
     int tid = threadIdx.x;
-    int R = WG / KP;
-    int rl = tid / KP, c = tid % KP;
+    const RowSplit sp(k);
+    int c = sp.c;
     double acc = 0.0;
-    if (c < k) {
+    if (sp.active()) {
         const FcgState S = st[c];
         double al = S.theta2;
-        for (long long i = (long long)blockIdx.x * R + rl; i < n; i += (long long)gridDim.x * R) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
             long long o = i * k + c;
             double rr;
             if (!S.done) {
@@ -597,13 +599,10 @@ __global__ __launch_bounds__(WG) void k_cg_update(int n, int k, int KP, const Fc
             acc += rr * rr;
         }
     }
-    s[tid] = acc;
+    s[0][tid] = acc;
     __syncthreads();
-    for (int stp = WG / 2; stp >= KP; stp >>= 1) {
-        if (tid < stp) s[tid] += s[tid + stp];
-        __syncthreads();
-    }
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[tid];
+    sp.sum<1>(s, k);
+    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
 }
 
 // l2 = ||r||; converged when l2 < rtol delta0, else the iteration count
@@ -634,8 +633,7 @@ __global__ __launch_bounds__(WG) void k_cg_finish(const double* __restrict__ par
 }
 
 void cg_update_finish(Context* c, const FcgBufs& f, const double* p, const double* s, double* x, double* r) {
-    int KP = kpad(f.k);
-    k_cg_update<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, KP, f.st, p, s, x, r, f.partials, f.all_done);
+    k_cg_update<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p, s, x, r, f.partials, f.all_done);
     BCMGX_LAUNCHED();
     k_cg_finish<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.rtol, f.itnlim, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();

@@ -141,14 +141,14 @@ void interleaved_to_colmajor(Context* c, const double* s, double* d, int ld, int
                              const double* p = nullptr);
 struct FcgBufs {
     int n = 0, k = 1;
-    int nblk = 0;              // partial-sum blocks (fixed for a given n)
+    int nblk = 0;              // partial-sum blocks (fixed for a given n and k)
     double* partials = nullptr;  // nblk * k * 3
     FcgState* st = nullptr;      // k states
     int* all_done = nullptr;     // 1 when every column stopped
     double rtol = 1e-6;
     int itnlim = 2000;
 };
-int fcg_partial_blocks(int n);
+int fcg_partial_blocks(int n, int k);
 // ||v||^2 partials of each column -> st[c].l2 = sqrt(sum); mode 0: delta0 = l2 (initial)
 void fcg_norm(Context* c, const FcgBufs& f, const double* v, int mode);
 // Optional level-0 entry of an FP32 V-cycle written by the FCG updates: with

@@ -97,7 +97,7 @@ struct SstepRun {
     DBuf<double> partials, dvm, dab;  // moments; alpha (s) then beta (s x s)
     SstepRun(Context* c_, const DCsr& A_, Prec* p_, int s_, int lanes_)
         : c(c_), A(A_), prec(p_), precon(p_->ptype != BCMGX_PREC_NONE), n(A_.n), s(s_), lanes(lanes_) {
-        nblk = fcg_partial_blocks(n);
+        nblk = fcg_partial_blocks(n, 1);
         partials.reset(c, (size_t)nblk * 2 * s + 1);
         dvm.reset(c, 2 * s + 1);
         dab.reset(c, s + s * s);
