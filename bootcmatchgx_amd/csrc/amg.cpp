@@ -987,6 +987,48 @@ static int fused_z32(Context* c, const DCsr& A, SolveWork& s, const double* wold
     return s.z32_blocks;
 }
 
+// The block form's code where the fused product is faster from it than from
+// k_spmmp, else 0: timed once for each (n, nnz, k) on the workspace's own
+// vectors.  It is asked only where the cycle's FP32 products run from the block
+// form, and is a choice of its own: the block form saves half of the reads of x,
+// but here it gathers w's and r's rows as well, in the tiles' order.  27-point
+// 128^3, 32 columns: 517 us from the block form, 672 from k_spmmp; 7-point 465
+// against 433; 27-point 41x40x40, 64 columns: 43 against 36; 7-point 100x90x80, 16
+// columns: 110 against 84.
+static int tune_fused_z32(Context* c, DCsr& A, SolveWork& s) {
+    std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + "z:k" + std::to_string(s.k);
+    auto it = c->tuned_lanes.find(sig);
+    if (it != c->tuned_lanes.end()) return it->second == BLK_CODE && block_values64(c, A) ? BLK_CODE : 0;
+    bool had = (bool)A.blk.val64;  // another width's captured iterations may hold them
+    if (!block_values64(c, A)) return 0;  // no room for the values: asked again by the next solve
+    long long nk = (long long)A.n * s.k;
+    fill<float>(c, s.zf.get(), nk, 1.0f);
+    fill<double>(c, s.r.get(), nk, 1.0);
+    fill<double>(c, s.q.get(), nk, 1.0);
+    hipEvent_t e0, e1;
+    BCMGX_HIP(hipEventCreate(&e0));
+    BCMGX_HIP(hipEventCreate(&e1));
+    int best = 0;
+    float bestms = 1e30f;
+    for (int code : {0, BLK_CODE}) {
+        s.z32_blk = code;
+        fused_z32(c, A, s, s.q.get(), nullptr, nullptr);
+        BCMGX_HIP(hipEventRecord(e0, c->stream));
+        for (int r = 0; r < 3; r++) fused_z32(c, A, s, s.q.get(), nullptr, nullptr);
+        BCMGX_HIP(hipEventRecord(e1, c->stream));
+        BCMGX_HIP(hipEventSynchronize(e1));
+        float ms;
+        BCMGX_HIP(hipEventElapsedTime(&ms, e0, e1));
+        if (ms < bestms) { bestms = ms; best = code; }
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    s.drop_graph();
+    c->tuned_lanes[sig] = best;
+    if (best != BLK_CODE && !had) A.blk.val64.release();
+    return best;
+}
+
 static void fcg_iteration_z32(Context* c, const DCsr& A, Prec* prec, SolveWork& s, int idx) {
     const int* stop = s.flags.get();
     prec->apply_entry_f32(s.r.get(), s.zf.get(), s.k, stop);
@@ -1069,16 +1111,13 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     s.fused = prec->fused_entry(k, &s.entry);
     // z in FP32 when the FP32 cycle is entered from the update and the fused FP32-z product applies
     bool z32 = s.fused && p.fcg_z32 && s.z32_blocks > 0 && s.z32_blocks % 8 == 0 && (s.chunkA <= 0 || s.chunkA >= k);
-    // where the cycle's products with A run from the block form, so does the fused product
-    int blk = z32 && s.z32_blk_grid > 0 && prec->H.L[0]->chunkA == BLK_CODE &&
-                      block_values64(c, const_cast<DCsr&>(A))
-                  ? BLK_CODE
-                  : 0;
+    if (z32 && !s.zf) s.zf.reset(c, (size_t)std::max(n, 1) * k);
+    int blk = 0;
+    if (z32 && s.z32_blk_grid > 0 && prec->H.L[0]->chunkA == BLK_CODE) blk = tune_fused_z32(c, const_cast<DCsr&>(A), s);
     if (blk != s.z32_blk) s.drop_graph();
     s.z32_blk = blk;
     if (z32 != s.z32) s.drop_graph();  // the captured iterations differ
     s.z32 = z32;
-    if (s.z32 && !s.zf) s.zf.reset(c, (size_t)std::max(n, 1) * k);
     long long nk = (long long)n * k;
     int* xzero = s.flags.get() + 2;  // the initial guess holds only zeros (set while staging it)
     if (io) {
