@@ -91,6 +91,20 @@ int cached_lanes(Context* c, const DCsr& A, bool fp32) {
     return default_lanes(A.nnz, A.n);
 }
 
+// Lanes per row of R and of A P (one column): their rows are short (1 entry a fine
+// row and 3 to 9), so a wave of the vector kernel has few entries in flight and the
+// CSR-stream kernel with as few lanes as fill the chip wins.  One lane (256 rows a
+// workgroup) from 262144 rows, 1024 workgroups: A P of 7-point 160^3 98 us from the
+// vector kernel, 66 with two lanes, 51 with one; of 27-point 128^3 123, 53, 49; R
+// of 512000 rows 23, 14.5, 15, of 262144 in FP64 15.4, 13.7, 12.1.  Two lanes from
+// 65536 rows: 227072 rows of A P 13.6, 7.0, 8.8.  Below that all take what a launch
+// costs (64000 rows: 4.5, 4.6, 4.6).  Rows of over 12 entries on average keep the
+// vector kernel: 256 of them overrun the stream kernel's 4096 staged products.
+static int transfer_lanes(const DCsr& M) {
+    if (M.n >= 65536 && (long long)M.nnz <= 12ll * M.n) return M.n >= 262144 ? -1 : -2;
+    return default_lanes(M.nnz, M.n);
+}
+
 template <typename V>
 static float time_spmm(Context* c, const DCsr& A, const void* val, int k, int chunk, hipEvent_t e0, hipEvent_t e1) {
     DBuf<V> x(c, (size_t)A.m * k), y(c, (size_t)A.n * k);
@@ -356,7 +370,7 @@ static void make_level_product(Context* c, Hierarchy& H, int l) {
     lv.AP.valf.reset(c, std::max(lv.AP.nnz, 1));
     convert<double, float>(c, lv.AP.val.get(), lv.AP.valf.get(), lv.AP.nnz);
     lv.AP.val.release();
-    lv.lanesAP = default_lanes(lv.AP.nnz, lv.AP.n);
+    lv.lanesAP = transfer_lanes(lv.AP);
 }
 // The same product queued with no host synchronisation (false when A_l's rows
 // are too long for it); level_product_lengths reads the lengths afterwards
@@ -373,7 +387,7 @@ static void level_product_lengths(Context* c, const std::vector<Level*>& lvs) {
     for (size_t t = 0; t < lvs.size(); t++) {
         Level& lv = *lvs[t];
         lv.AP.nnz = h[t];
-        lv.lanesAP = default_lanes(lv.AP.nnz, lv.AP.n);
+        lv.lanesAP = transfer_lanes(lv.AP);
     }
 }
 
@@ -506,14 +520,23 @@ static const V* mat_val(const DCsr& A) {
     else return A.val.get();
 }
 
+// a level's result asked for as its correction of the finer level instead: to.out = P x + to.in
+template <typename V>
+struct Correction {
+    RowProlong<V> to;
+    bool done = false;  // set by the kernel that forms the result, where it can
+};
+
 // k sweeps of l1-Jacobi; (cur, oth) is the ping-pong pair, cur holds the
 // guess (ignored when xzero).  Returns the buffer holding the result.  With
 // `out64` (FP32 sweeps only) the last sweep (one from a nonzero guess) writes
 // its result widened to FP64 there instead, and nullptr is returned; with
-// `outv` it writes it there (same type) and returns outv.
+// `outv` it writes it there (same type) and returns outv; with `up` (one
+// column) it hands it to the finer level and the returned buffer is not written.
 template <typename V>
 static V* jacobi_sweeps(Context* c, const DCsr& A, int lanes, const V* M, const V* F, V* cur, V* oth, int s, bool xzero,
-                        int k, const int* stop, int chunk = 0, double* out64 = nullptr, V* outv = nullptr) {
+                        int k, const int* stop, int chunk = 0, double* out64 = nullptr, V* outv = nullptr,
+                        Correction<V>* up = nullptr) {
     int done = 0;
     if (s <= 0) {
         if (xzero) fill<V>(c, cur, (long long)A.n * k, (V)0);
@@ -533,6 +556,13 @@ static V* jacobi_sweeps(Context* c, const DCsr& A, int lanes, const V* M, const 
             a.y64 = out64;
             spmv<V, V>(c, SpOp::JACOBI, a);
             return nullptr;
+        }
+        if (last && up) {
+            a.up_row = up->to.row; a.up_col = up->to.col; a.up_val = up->to.val;
+            a.up_in = up->to.in; a.up_out = up->to.out;
+            spmv<V, V>(c, SpOp::JACOBI, a);
+            up->done = true;
+            return oth;
         }
         if (last && outv) {
             a.y = outv;
@@ -572,7 +602,7 @@ static const V* lvl_pval(const Level& l) {
 // holding the level's result.
 template <typename V>
 static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep_done = false, double* out64 = nullptr,
-                     V* outv = nullptr) {
+                     V* outv = nullptr, Correction<V>* up = nullptr) {
     Context* c = R.c;
     Prec* pr = R.pr;
     const bcmgx_params& p = pr->p;
@@ -612,11 +642,13 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
             if (k == 1) {
                 V* y = xzero ? cur : oth;
                 if (coarse_sweeps<V>(c, A, lv.lanesA, lv.M.get(), F, xzero ? nullptr : cur, y, p.relaxnumber_coarse,
-                                     lv.cix, pr->coarse, R.stop))
+                                     lv.cix, pr->coarse, R.stop, up ? up->to : RowProlong<V>())) {
+                    if (up) up->done = true;
                     return y;
+                }
             }
             return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, p.relaxnumber_coarse, xzero, k, R.stop,
-                                    lv.chunkA);
+                                    lv.chunkA, nullptr, nullptr, up);
         }
     }
     int coeff = p.cycle_type == BCMGX_CYCLE_VARIABLE_V ? (1 << l) : 1;
@@ -658,27 +690,38 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
         spmv<V, V>(c, SpOp::AX, a);
     }
     V* xc = nullptr;
+    int post = p.postrelax_sweeps * coeff;
+    // from A P in FP32: the prolongation and the first post-smoothing sweep in one pass,
+    // f - A (x + P e) = (f - A x) - (A P) e, the first term still in w.Res
+    bool from_ap = std::is_same<V, float>::value && post >= 1 && lv.AP.valf;
+    // else, for one column, the coarser level's last sweep prolongs its result by the
+    // rows of R (every fine row is in one of them) and x is corrected without a pass of
+    // its own; into the other buffer, since the coarsest level's kernel may do it twice
+    Correction<V> corr;
+    if (k == 1 && !from_ap && lv.R.nnz == A.n && lv.R.m == A.n)
+        corr.to = {lv.R.row.get(), lv.R.col.get(), mat_val<V>(lv.R), cur, oth};
     if (nl > 2 || p.relaxnumber_coarse > 0) {
         int gs = 1;  // setGridSweeps (AMG.cu:306-331)
         if (p.cycle_type == BCMGX_CYCLE_W && l < nl - 2) gs = 2;
         if (p.cycle_type == BCMGX_CYCLE_H && (l % 2) == 0) gs = 2;
         for (int i = 1; i <= gs; i++) {
-            xc = gamg_cycle<V>(R, l + 1, wc.F.get(), xc, i == 1 && sweep0);
-            if (l + 1 == nl - 1) break;
+            bool last = i == gs || l + 1 == nl - 1;
+            xc = gamg_cycle<V>(R, l + 1, wc.F.get(), xc, i == 1 && sweep0, nullptr, nullptr,
+                               last && corr.to.out ? &corr : nullptr);
+            if (last) break;
         }
     }
-    oth = (cur == w.X.get()) ? w.X2.get() : w.X.get();
-    int post = p.postrelax_sweeps * coeff;
     if constexpr (std::is_same<V, float>::value) {
-        // the prolongation and the first post-smoothing sweep from A P in one pass:
-        // f - A (x + P e) = (f - A x) - (A P) e, the first term still in w.Res
-        if (xc && post >= 1 && lv.AP.valf) {
+        if (xc && from_ap) {
             V* y = post == 1 && outv ? outv : oth;
             SpmvArgs a;
             a.n = lv.AP.n; a.row = lv.AP.row.get(); a.col = lv.AP.col.get(); a.val = lv.AP.valf.get();
             a.nnz = lv.AP.nnz; a.x = xc; a.y = y; a.b = w.Res.get(); a.D = lvl_M<V>(lv); a.k = k;
             a.lanes = lv.lanesAP; a.stop = R.stop;
+            bool wide = k == 1 && post == 1 && out64;  // one column: widened in the same pass
+            if (wide) a.y64 = out64;
             galerkin_post_sweep<V>(c, a, lv.agg.get(), lvl_pval<V>(lv), cur);
+            if (wide) return nullptr;
             if (post == 1) {
                 if (!out64) return y;
                 convert_stop<V, double>(c, y, out64, (long long)A.n * k, R.stop);  // the result widened
@@ -687,11 +730,12 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
             cur = y;
             oth = (cur == w.X.get()) ? w.X2.get() : w.X.get();
             return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, post - 1, false, k, R.stop, lv.chunkA,
-                                    out64, outv);
+                                    out64, outv, up);
         }
     }
-    if (xc) prolong_add<V>(c, A.n, k, lv.agg.get(), lvl_pval<V>(lv), xc, cur, R.stop);
-    cur = jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, post, false, k, R.stop, lv.chunkA, out64, outv);
+    if (corr.done) std::swap(cur, oth);
+    else if (xc) prolong_add<V>(c, A.n, k, lv.agg.get(), lvl_pval<V>(lv), xc, cur, R.stop);
+    cur = jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, post, false, k, R.stop, lv.chunkA, out64, outv, up);
     return cur;
 }
 
@@ -710,10 +754,13 @@ void Prec::refresh_level0() {
 
 bool Prec::fused_entry(int k, FcgEntry* e) {
     f0_from_r = false;
-    if (ptype != BCMGX_PREC_BCMG || p.precision != BCMGX_PRECISION_FP32 || H.levels() < 2 || p.prerelax_sweeps < 1 ||
-        n_hrc() > 1)
-        return false;
+    if (ptype != BCMGX_PREC_BCMG || H.levels() < 2 || p.prerelax_sweeps < 1 || n_hrc() > 1) return false;
     ensure_work(k);
+    if (p.precision != BCMGX_PRECISION_FP32) {
+        e->X64 = wd[0].X.get();
+        e->M64 = H.L[0]->M.get();
+        return true;
+    }
     // level 0's F is read only by the residual after the first sweep when that sweep
     // is the only pre-smoothing, the first post-smoothing sweep comes from A P and is
     // the only one, and a coarse correction exists; the residual then takes r (FP64)
@@ -764,7 +811,8 @@ void Prec::apply_hrc(int h, const double* r, double* u, int k, bool x_zero, cons
         }
         if (res) convert_stop<float, double>(c, res, u, nk, stop);
     } else {
-        BCMGX_CHECK(!entry_ready, BCMGX_ERR_STATE, "level-0 entry not applicable");
+        BCMGX_CHECK(!entry_ready || (x_zero && h == 0 && Hh.levels() >= 2 && p.prerelax_sweeps >= 1), BCMGX_ERR_STATE,
+                    "level-0 entry not applicable");
         CycleRun<double> R{c, this, &Hh, &wd, k, stop};
         double* xin = nullptr;
         if (!x_zero) {
@@ -772,7 +820,7 @@ void Prec::apply_hrc(int h, const double* r, double* u, int k, bool x_zero, cons
             xin = wd[0].X.get();
         }
         // the last level-0 sweep writes u directly when the cycle ends in one
-        double* res = gamg_cycle<double>(R, 0, r, xin, false, nullptr, u);
+        double* res = gamg_cycle<double>(R, 0, r, xin, entry_ready, nullptr, u);
         if (res != u) convert_stop<double, double>(c, res, u, nk, stop);
     }
 }
@@ -944,7 +992,7 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
                 Level& l = *lp;
                 const DCsr& M = l.mat();
                 l.lanesA = p.autotune ? tune_lanes(c, M, f32) : default_lanes(M.nnz, M.n);
-                l.lanesR = l.R.n > 0 ? default_lanes(l.R.nnz, l.R.n) : 1;
+                l.lanesR = l.R.n > 0 ? transfer_lanes(l.R) : 1;
             }
         };
         build_hierarchy(c, A, p, pr->H, nullptr, &side, level_done(pr->H));
@@ -1110,7 +1158,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     s.entry = FcgEntry();
     s.fused = prec->fused_entry(k, &s.entry);
     // z in FP32 when the FP32 cycle is entered from the update and the fused FP32-z product applies
-    bool z32 = s.fused && p.fcg_z32 && s.z32_blocks > 0 && s.z32_blocks % 8 == 0 && (s.chunkA <= 0 || s.chunkA >= k);
+    bool z32 = s.entry.X && p.fcg_z32 && s.z32_blocks > 0 && s.z32_blocks % 8 == 0 && (s.chunkA <= 0 || s.chunkA >= k);
     if (z32 && !s.zf) s.zf.reset(c, (size_t)std::max(n, 1) * k);
     int blk = 0;
     if (z32 && s.z32_blk_grid > 0 && prec->H.L[0]->chunkA == BLK_CODE) blk = tune_fused_z32(c, const_cast<DCsr&>(A), s);

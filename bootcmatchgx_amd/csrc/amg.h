@@ -75,14 +75,14 @@ struct Prec {
     void ensure_work(int k);
     void drop_graphs();
     // u <- B r for k interleaved columns; `x_zero`: u holds zeros on entry (the FCG case).
-    // `entry_ready`: the level-0 entry of the FP32 cycle (see fused_entry) already
-    // holds F = (float) r (unless the cycle reads r itself) and the first sweep X = F / M.
+    // `entry_ready`: the level-0 entry of the cycle (see fused_entry) already holds the
+    // first sweep X = F / M and, in FP32, F = (float) r (unless the cycle reads r itself).
     void apply(const double* r, double* u, int k, bool x_zero, const int* stop, bool entry_ready = false);
     // one cycle of bootstrap hierarchy h alone: u <- cycle_h(r) from the guess u
     void apply_hrc(int h, const double* r, double* u, int k, bool x_zero, const int* stop, bool entry_ready = false);
-    // the level-0 buffers an FCG update can fill for the next apply (FP32 BCMG
-    // with at least two levels and a pre-smoothing sweep); false otherwise.  When
-    // the level's right-hand side is read only by the residual after the first
+    // the level-0 buffers an FCG update can fill for the next apply (BCMG with at
+    // least two levels and a pre-smoothing sweep); false otherwise.  FP64: X64 alone.
+    // FP32: when the level's right-hand side is read only by the residual after the first
     // sweep and that runs on the pipelined SpMM, F is left out (e->F = null) and
     // the cycle rounds r there itself (f0_from_r)
     bool fused_entry(int k, FcgEntry* e);

@@ -88,7 +88,7 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
     int n, const int* __restrict__ row, const int* __restrict__ col, const double* __restrict__ val,
     const double* __restrict__ D, const V* __restrict__ f, const V* __restrict__ x0, V* __restrict__ out, int sweeps,
     const int* __restrict__ ucnt, const int* __restrict__ ucol, const unsigned short* __restrict__ upos, u64* slots,
-    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience) {
+    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience, RowProlong<V> up) {
     constexpr int T = CO_ROWS * L, NU = CO_FETCH;
     if (stop && *stop) return;
     __shared__ double xs[2][TILE_MAX_COLS];
@@ -196,7 +196,10 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
             __hip_atomic_store(p + 1, tag | (unsigned)__double2hiint(xr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
-    if (!given_up && on && lane == 0) out[r] = (V)xr;
+    if (!given_up && on) {
+        if (up.out) up.template put<L>(r, lane, (V)xr);
+        else if (lane == 0) out[r] = (V)xr;
+    }
     __syncthreads();
     if (tid == 0) {
         __threadfence();
@@ -226,7 +229,10 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
             cur = nxt;
             nxt = w;
         }
-        for (int i = tid; i < n; i += T) out[i] = (V)cur[i];
+        for (int i = tid; i < n; i += T) {
+            if (up.out) up.template put<1>(i, 0, (V)cur[i]);
+            else out[i] = (V)cur[i];
+        }
         __syncthreads();
     }
     if (tid == 0) {
@@ -241,7 +247,8 @@ template <typename V, int L>
 __global__ __launch_bounds__(CO_SMALL_T) void k_coarse_small(int n, const int* __restrict__ row, const int* __restrict__ col,
                                                              const double* __restrict__ val, const double* __restrict__ D,
                                                              const V* __restrict__ f, const V* __restrict__ x0,
-                                                             V* __restrict__ out, int sweeps, const int* __restrict__ stop) {
+                                                             V* __restrict__ out, int sweeps, const int* __restrict__ stop,
+                                                             RowProlong<V> up) {
     if (stop && *stop) return;
     constexpr int RR = CO_SMALL_RR, E = CO_SMALL_E, G = CO_SMALL_T / L;
     __shared__ double xs[2][CO_SMALL_N];
@@ -278,13 +285,15 @@ __global__ __launch_bounds__(CO_SMALL_T) void k_coarse_small(int n, const int* _
 #pragma unroll
     for (int w = 0; w < RR; w++) {
         int r = w * G + g;
-        if (r < n && lane == 0) out[r] = (V)xr[w];
+        if (r >= n) continue;
+        if (up.out) up.template put<L>(r, lane, (V)xr[w]);
+        else if (lane == 0) out[r] = (V)xr[w];
     }
 }
 
 template <typename V, int L, int E>
 static bool launch_exchange(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int sweeps,
-                            const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+                            const CoarseIndex& ix, CoarseSync& cs, const int* stop, const RowProlong<V>& up) {
     auto kern = k_coarse_exchange<V, L, E>;
     static int resident = 0;  // workgroups the device holds, per instantiation; identical devices assumed within a process
     if (!resident) {
@@ -296,7 +305,7 @@ static bool launch_exchange(Context* c, const DCsr& A, const double* D, const V*
     if ((long long)grid * 2 > resident) return false;
     kern<<<grid, CO_ROWS * L, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, sweeps,
                                               ix.ucnt.get(), ix.ucol.get(), ix.upos.get(), cs.slots.get(),
-                                              cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience);
+                                              cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience, up);
     BCMGX_LAUNCHED();
     return true;
 }
@@ -328,7 +337,7 @@ bool coarse_sweeps_fit(int n, int sweeps) { return n > 0 && n <= CO_MAX_N && swe
 
 template <typename V>
 bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const V* f, const V* x0, V* out, int sweeps,
-                   const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+                   const CoarseIndex& ix, CoarseSync& cs, const int* stop, const RowProlong<V>& up) {
     int L = lanes != 0 ? lanes : default_lanes(A.nnz, A.n);
     if (!coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || L < 2 || L > 32 || (const void*)out == (const void*)x0) return false;
     // One workgroup while it holds the level's entries in registers (n <= 4096 / L): a
@@ -337,7 +346,7 @@ bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const 
 #define BCMGX_CS(LL)                                                                                                     \
     case LL:                                                                                                             \
         k_coarse_small<V, LL><<<1, CO_SMALL_T, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, \
-                                                               sweeps, stop);                                            \
+                                                               sweeps, stop, up);                                          \
         break;
         switch (L) { BCMGX_CS(2) BCMGX_CS(4) BCMGX_CS(8) BCMGX_CS(16) BCMGX_CS(32) }
 #undef BCMGX_CS
@@ -347,17 +356,17 @@ bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const 
     if (!ix.ucnt || cs.slots.size() < (size_t)A.n * sweeps * 2 || cs.scratch.size() < (size_t)A.n * 2) return false;
 #define BCMGX_CX(LL)                                                                                         \
     case LL:                                                                                                 \
-        if (A.maxrow <= 2 * LL) return launch_exchange<V, LL, 2>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
-        if (A.maxrow <= 4 * LL) return launch_exchange<V, LL, 4>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
-        if (A.maxrow <= 8 * LL) return launch_exchange<V, LL, 8>(c, A, D, f, x0, out, sweeps, ix, cs, stop);     \
+        if (A.maxrow <= 2 * LL) return launch_exchange<V, LL, 2>(c, A, D, f, x0, out, sweeps, ix, cs, stop, up);     \
+        if (A.maxrow <= 4 * LL) return launch_exchange<V, LL, 4>(c, A, D, f, x0, out, sweeps, ix, cs, stop, up);     \
+        if (A.maxrow <= 8 * LL) return launch_exchange<V, LL, 8>(c, A, D, f, x0, out, sweeps, ix, cs, stop, up);     \
         return false;
     switch (L) { BCMGX_CX(2) BCMGX_CX(4) BCMGX_CX(8) BCMGX_CX(16) BCMGX_CX(32) }
 #undef BCMGX_CX
     return false;
 }
 template bool coarse_sweeps<double>(Context*, const DCsr&, int, const double*, const double*, const double*, double*, int,
-                                    const CoarseIndex&, CoarseSync&, const int*);
+                                    const CoarseIndex&, CoarseSync&, const int*, const RowProlong<double>&);
 template bool coarse_sweeps<float>(Context*, const DCsr&, int, const double*, const float*, const float*, float*, int,
-                                   const CoarseIndex&, CoarseSync&, const int*);
+                                   const CoarseIndex&, CoarseSync&, const int*, const RowProlong<float>&);
 
 }  // namespace bcmgx

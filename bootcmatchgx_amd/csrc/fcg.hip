@@ -140,8 +140,8 @@ __global__ __launch_bounds__(WG) void k_norm_final(const double* __restrict__ pa
     }
 }
 
-// ||r||^2 partials in k_dots<1>'s blocks and order, with the FP32 cycle's
-// level-0 entry (F = (float) r, X = F/M) written on the way, as k_update does
+// ||r||^2 partials in k_dots<1>'s blocks and order, with the cycle's
+// level-0 entry (FP32: F = (float) r, X = F/M) written on the way, as k_update does
 __global__ __launch_bounds__(WG) void k_norm_entry(int n, int k, const double* __restrict__ r,
                                                    double* __restrict__ partials, FcgEntry e) {
     __shared__ double s[1][WG];
@@ -154,9 +154,7 @@ __global__ __launch_bounds__(WG) void k_norm_entry(int n, int k, const double* _
             long long o = i * k + c;
             double rr = r[o];
             acc += rr * rr;
-            float fv = (float)rr;
-            if (e.F) e.F[o] = fv;
-            e.X[o] = fv / e.M[i];
+            e.put(o, i, rr);
         }
     }
     s[0][tid] = acc;
@@ -225,11 +223,7 @@ __global__ __launch_bounds__(WG) void k_init_update(int n, int k, const FcgState
     }
     d[t] = vv;                // d = clone(v), q = clone(w)  (FCG.cu:98-99)
     q[t] = ww;
-    if (e.X) {
-        float f = (float)rr;
-        if (e.F) e.F[t] = f;
-        e.X[t] = f / e.M[i];
-    }
+    e.put(t, i, rr);
 }
 
 void fcg_init_update(Context* c, const FcgBufs& f, double* x, double* r, const double* v, const double* w, double* d, double* q,
@@ -328,11 +322,7 @@ __global__ __launch_bounds__(WG) void k_update(int n, int k, const FcgState* __r
                 if (waiting) x[o] = pend * p1[o] + x[o];
             }
             acc += rr * rr;
-            if (e.X) {
-                float f = (float)rr;
-                if (e.F) e.F[o] = f;
-                e.X[o] = f / e.M[i];
-            }
+            e.put(o, i, rr);
         }
     }
     s[0][tid] = acc;
@@ -388,11 +378,7 @@ __global__ __launch_bounds__(WG) void k_update_z32(int n, int k, const FcgState*
                 if (waiting) x[o] = pend * p[o] + x[o];
             }
             acc += rr * rr;
-            if (e.X) {
-                float f = (float)rr;
-                if (e.F) e.F[o] = f;
-                e.X[o] = f / e.M[i];
-            }
+            e.put(o, i, rr);
         }
     }
     s[0][tid] = acc;

@@ -47,6 +47,26 @@ enum class SpOp {
     JACOBI   // y = ((-(A x) + b) / D) + x                (_jacobi_it_full<0>, l1jacobi.cu:344-379)
 };
 
+// x_out = P e + x_in row by row of R = P^T, for a kernel that has just formed e_r
+template <typename V>
+struct RowProlong {
+    const int* row = nullptr;
+    const int* col = nullptr;
+    const V* val = nullptr;
+    const V* in = nullptr;
+    V* out = nullptr;
+    // by the TPR lanes of row r's group, each with the same v = e_r
+    template <int TPR>
+    __device__ __forceinline__ void put(int r, int sub, V v) const {
+        int e = row[r + 1];
+        for (int q = row[r] + sub; q < e; q += TPR) {
+            int i = col[q];
+            V t = val[q] * v;
+            out[i] = t + in[i];
+        }
+    }
+};
+
 struct SpmvArgs {
     int n = 0;
     const int* row = nullptr;
@@ -72,6 +92,17 @@ struct SpmvArgs {
     const int* tu = nullptr;    // the matrix's row-tile index (DCsr::tu, tucol, tlidx), or null
     const int* tucol = nullptr;
     const unsigned short* tlidx = nullptr;
+    // one vector, JACOBI: instead of storing y, prolong it: up_out = P y + up_in over the
+    // rows of R = P^T (up_row, up_col, up_val; each row of up_out in one row of R)
+    const int* up_row = nullptr;
+    const int* up_col = nullptr;
+    const void* up_val = nullptr;  // V*
+    const void* up_in = nullptr;   // V*
+    void* up_out = nullptr;        // V*
+    // set by galerkin_post_sweep
+    const int* agg = nullptr;
+    const void* pv = nullptr;
+    const void* xpre = nullptr;
     const BlockForm* blk = nullptr; // the matrix's block form, used when kchunk asks for it (BLK_CODE)
 };
 // the row-tile index of A into a (k = 1 launches whose lanes code asks for the tiled kernel use it)
@@ -151,15 +182,28 @@ struct FcgBufs {
 int fcg_partial_blocks(int n, int k);
 // ||v||^2 partials of each column -> st[c].l2 = sqrt(sum); mode 0: delta0 = l2 (initial)
 void fcg_norm(Context* c, const FcgBufs& f, const double* v, int mode);
-// Optional level-0 entry of an FP32 V-cycle written by the FCG updates: with
+// Optional level-0 entry of a V-cycle (FP32) written by the FCG updates: with
 // the new residual r, F = (float) r and X = F / M (the first l1-Jacobi sweep
 // from a zero guess), so the next preconditioner application starts there.
 // F may be null: then only X is written and the cycle rounds r itself where it
 // needs the level's right-hand side.
+// An FP64 cycle's entry is X64 = r / M64 alone.
 struct FcgEntry {
     float* F = nullptr;
     float* X = nullptr;
     const float* M = nullptr;
+    double* X64 = nullptr;
+    const double* M64 = nullptr;
+    // element o of row i from its residual
+    __device__ __forceinline__ void put(long long o, long long i, double r) const {
+        if (X) {
+            float f = (float)r;
+            if (F) F[o] = f;
+            X[o] = f / M[i];
+        } else if (X64) {
+            X64[o] = r / M64[i];
+        }
+    }
 };
 // fcg_norm of r that also writes the FP32 cycle's level-0 entry from r
 void fcg_norm_entry(Context* c, const FcgBufs& f, const double* r, int mode, const FcgEntry& e);
@@ -308,10 +352,11 @@ struct CoarseIndex {
 };
 // `sweeps` l1-Jacobi sweeps of A (FP64) on one right-hand side in one launch: out from the guess
 // x0 (null: zero; never out itself), f and x0 widened from V, the result rounded to V; the bits of
-// sweep after sweep through k_spmv1 with `lanes`.  False (nothing launched) where it does not apply.
+// sweep after sweep through k_spmv1 with `lanes`.  With up.out the result is prolonged there instead
+// (it may be prolonged twice, so up.in is another buffer).  False (nothing launched) where it does not apply.
 template <typename V>
 bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const V* f, const V* x0, V* out, int sweeps,
-                   const CoarseIndex& ix, CoarseSync& cs, const int* stop);
+                   const CoarseIndex& ix, CoarseSync& cs, const int* stop, const RowProlong<V>& up = RowProlong<V>());
 
 // ---- AFSAI (afsai.hip) ------------------------------------------------------------
 void afsai_build(Context* c, const DCsr& A, DCsr& G, DCsr& GT);

@@ -15,11 +15,52 @@
 
 namespace bcmgx {
 
-template <typename T, typename V, int L, SpOp OP>
+// What a one-vector kernel does with a row's sum t (OP, then EPI):
+// EPI_X0 (AX): also x0 = t / D, the first l1-Jacobi sweep from zero on the
+// restricted residual; EPI_POST (AX with A P): the post-smoothing sweep
+// ((-t + b) / D) + (p_i e[agg_i] + xpre), widened into y64 when given; EPI_UP
+// (JACOBI): the new x_r is not stored but prolonged to its aggregate's rows,
+// up_out_i = p_i x_r + up_in_i over row r of R = P^T.  Each is a pass of its own
+// otherwise, with the same operations on the same values, and on levels of up to
+// some 100000 rows a pass costs what its launch does (4.7 us in a replayed
+// graph, whatever it computes).
+enum { EPI_NONE, EPI_X0, EPI_POST, EPI_UP };
+template <typename V>
+struct RowEpilogue {
+    V* x0;
+    const int* agg;
+    const V* pv;
+    const V* xpre;
+    double* y64;
+    RowProlong<V> up;
+};
+// by every lane of the row's group of TPR; sub: the lane
+template <int TPR, SpOp OP, int EPI, typename V>
+__device__ __forceinline__ void finish_row(int r, int sub, V t, const V* x, V* y, const V* b, const V* D, V beta,
+                                           const RowEpilogue<V>& ep) {
+    if constexpr (EPI == EPI_UP) {
+        V v = ((-t + b[r]) / D[r]) + x[r];
+        ep.up.template put<TPR>(r, sub, v);
+    } else if (sub == 0) {
+        if constexpr (EPI == EPI_POST) {
+            V z = ((-t + b[r]) / D[r]) + (ep.pv[r] * x[ep.agg[r]] + ep.xpre[r]);
+            if (ep.y64) ep.y64[r] = (double)z;
+            else y[r] = z;
+            return;
+        }
+        if (OP == SpOp::AX) y[r] = t;
+        else if (OP == SpOp::RES) y[r] = b[r] - t;
+        else if (OP == SpOp::AXPBY) y[r] = t + beta * y[r];
+        else y[r] = ((-t + b[r]) / D[r]) + x[r];
+        if constexpr (EPI == EPI_X0) ep.x0[r] = t / D[r];
+    }
+}
+
+template <typename T, typename V, int L, SpOp OP, int EPI>
 __global__ __launch_bounds__(WG) void k_spmv1(int n, const int* __restrict__ row, const int* __restrict__ col,
                                               const T* __restrict__ val, const V* __restrict__ x, V* __restrict__ y,
                                               const V* __restrict__ b, const V* __restrict__ D, V alpha, V beta,
-                                              const int* __restrict__ stop) {
+                                              const int* __restrict__ stop, RowEpilogue<V> ep) {
     if (stop && *stop) return;
     constexpr int RPB = WG / L;
     int blk = xcd_remap(blockIdx.x, gridDim.x);
@@ -36,12 +77,7 @@ __global__ __launch_bounds__(WG) void k_spmv1(int n, const int* __restrict__ row
     }
 #pragma unroll
     for (int o = L / 2; o > 0; o >>= 1) t += __shfl_xor(t, o, L);
-    if (lane == 0) {
-        if (OP == SpOp::AX) y[r] = t;
-        else if (OP == SpOp::RES) y[r] = b[r] - t;
-        else if (OP == SpOp::AXPBY) y[r] = t + beta * y[r];
-        else y[r] = ((-t + b[r]) / D[r]) + x[r];
-    }
+    finish_row<L, OP, EPI>(r, lane, t, x, y, b, D, beta, ep);
 }
 
 // order LDS accesses of the lanes of one wave (compiler fence; no hardware barrier)
@@ -532,11 +568,11 @@ bool spmm_dots_z32(Context* c, const SpmvArgs& a, const double* r, const double*
 // thread in flight), then TPR lanes reduce each row from LDS.  The LDS tile
 // holds 32 nonzeros per row on average (so a block stays small enough for
 // full occupancy); blocks with more reduce straight from global memory.
-template <typename T, typename V, int TPR, SpOp OP>
+template <typename T, typename V, int TPR, SpOp OP, int EPI>
 __global__ __launch_bounds__(WG) void k_spmv_stream(int n, const int* __restrict__ row, const int* __restrict__ col,
                                                     const T* __restrict__ val, const V* __restrict__ x, V* __restrict__ y,
                                                     const V* __restrict__ b, const V* __restrict__ D, V alpha, V beta,
-                                                    const int* __restrict__ stop, int sb) {
+                                                    const int* __restrict__ stop, int sb, RowEpilogue<V> ep) {
     if (stop && *stop) return;
     constexpr int RB = WG / TPR;
     constexpr int CAP = RB * 32 < 4096 ? RB * 32 : 4096;
@@ -595,12 +631,7 @@ __global__ __launch_bounds__(WG) void k_spmv_stream(int n, const int* __restrict
     }
 #pragma unroll
     for (int o = TPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, TPR);
-    if (sub == 0) {
-        if (OP == SpOp::AX) y[r] = acc;
-        else if (OP == SpOp::RES) y[r] = b[r] - acc;
-        else if (OP == SpOp::AXPBY) y[r] = acc + beta * y[r];
-        else y[r] = ((-acc + b[r]) / D[r]) + x[r];
-    }
+    finish_row<TPR, OP, EPI>(r, sub, acc, x, y, b, D, beta, ep);
 }
 
 // The CSR-stream SpMV with the matrix streamed in pairs: every thread loads
@@ -609,12 +640,12 @@ __global__ __launch_bounds__(WG) void k_spmv_stream(int n, const int* __restrict
 // memory instructions.  Same chunks, staging and per-row reduction as
 // k_spmv_stream, hence the same bits.  The final pair of the matrix is read
 // element by element when nnz is odd (no read past the arrays).
-template <typename T, typename V, int TPR, SpOp OP>
+template <typename T, typename V, int TPR, SpOp OP, int EPI>
 __global__ __launch_bounds__(WG) void k_spmv_stream2(int n, long long nnz, const int* __restrict__ row,
                                                      const int* __restrict__ col, const T* __restrict__ val,
                                                      const V* __restrict__ x, V* __restrict__ y, const V* __restrict__ b,
                                                      const V* __restrict__ D, V alpha, V beta,
-                                                     const int* __restrict__ stop, int sb) {
+                                                     const int* __restrict__ stop, int sb, RowEpilogue<V> ep) {
     typedef T T2 __attribute__((ext_vector_type(2)));
     typedef int I2 __attribute__((ext_vector_type(2)));
     if (stop && *stop) return;
@@ -694,12 +725,7 @@ __global__ __launch_bounds__(WG) void k_spmv_stream2(int n, long long nnz, const
     }
 #pragma unroll
     for (int o = TPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, TPR);
-    if (sub == 0) {
-        if (OP == SpOp::AX) y[r] = acc;
-        else if (OP == SpOp::RES) y[r] = b[r] - acc;
-        else if (OP == SpOp::AXPBY) y[r] = acc + beta * y[r];
-        else y[r] = ((-acc + b[r]) / D[r]) + x[r];
-    }
+    finish_row<TPR, OP, EPI>(r, sub, acc, x, y, b, D, beta, ep);
 }
 
 // CSR-stream SpMV over the matrix's row-tile index: a workgroup owns one tile of
@@ -712,13 +738,13 @@ __global__ __launch_bounds__(WG) void k_spmv_stream2(int n, long long nnz, const
 // per row on the 27-point grid) and a handful of coalesced x loads per tile
 // instead of one gather per entry.  A tile the index leaves out is read by
 // column index from global memory.
-template <typename T, typename V, SpOp OP>
+template <typename T, typename V, SpOp OP, int EPI>
 __global__ __launch_bounds__(WG) void k_spmv_tiled(int n, long long nnz, const int* __restrict__ row,
                                                    const int* __restrict__ col, const T* __restrict__ val,
                                                    const int* __restrict__ tu, const int* __restrict__ tucol,
                                                    const unsigned short* __restrict__ tlidx, const V* __restrict__ x,
                                                    V* __restrict__ y, const V* __restrict__ b, const V* __restrict__ D,
-                                                   V alpha, V beta, const int* __restrict__ stop, int sb) {
+                                                   V alpha, V beta, const int* __restrict__ stop, int sb, RowEpilogue<V> ep) {
     constexpr int TPR = WG / TILE_ROWS, RB = TILE_ROWS, UP = 4, XP = TILE_MAX_COLS / WG;
     static_assert(2 * UP * WG == TILE_MAX_ENTRIES, "one pass of paired loads covers an indexed tile");
     typedef T T2 __attribute__((ext_vector_type(2)));
@@ -815,12 +841,7 @@ __global__ __launch_bounds__(WG) void k_spmv_tiled(int n, long long nnz, const i
     }
 #pragma unroll
     for (int o = TPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, TPR);
-    if (sub == 0) {
-        if (OP == SpOp::AX) y[r] = acc;
-        else if (OP == SpOp::RES) y[r] = b[r] - acc;
-        else if (OP == SpOp::AXPBY) y[r] = acc + beta * y[r];
-        else y[r] = ((-acc + b[r]) / D[r]) + x[r];
-    }
+    finish_row<TPR, OP, EPI>(r, sub, acc, x, y, b, D, beta, ep);
 }
 
 int default_lanes(long long nnz, int n) {
@@ -835,7 +856,7 @@ int default_lanes(long long nnz, int n) {
     return 64;
 }
 
-template <typename T, typename V, SpOp OP>
+template <typename T, typename V, SpOp OP, int EPI = EPI_NONE>
 static void launch1(Context* c, const SpmvArgs& a, int L) {
     const T* val = (const T*)a.val;
     const V* x = (const V*)a.x;
@@ -843,6 +864,8 @@ static void launch1(Context* c, const SpmvArgs& a, int L) {
     const V* b = (const V*)a.b;
     const V* D = (const V*)a.D;
     V al = (V)a.alpha, be = (V)a.beta;
+    RowEpilogue<V> ep{(V*)a.x0, a.agg, (const V*)a.pv, (const V*)a.xpre, a.y64,
+                      {a.up_row, a.up_col, (const V*)a.up_val, (const V*)a.up_in, (V*)a.up_out}};
     // L < 0: CSR-stream kernels, L = -(1000 s + P + T): T lanes per row
     // reduction, P = 200 for the (val, col) pair stream, P = 400 for the
     // row-tile kernel (T = 4, A's tile index in a), s = 0 for per-XCD
@@ -858,8 +881,8 @@ static void launch1(Context* c, const SpmvArgs& a, int L) {
         bool ok = a.tu && a.tucol && a.tlidx && (((uintptr_t)a.val) & (2 * sizeof(T) - 1)) == 0 &&
                   (((uintptr_t)a.tlidx) & 3) == 0;
         if (ok) {
-            k_spmv_tiled<T, V, OP><<<grid_for(a.n, TILE_ROWS), WG, 0, c->stream>>>(
-                a.n, a.nnz, a.row, a.col, val, a.tu, a.tucol, a.tlidx, x, y, b, D, al, be, a.stop, sb);
+            k_spmv_tiled<T, V, OP, EPI><<<grid_for(a.n, TILE_ROWS), WG, 0, c->stream>>>(
+                a.n, a.nnz, a.row, a.col, val, a.tu, a.tucol, a.tlidx, x, y, b, D, al, be, a.stop, sb, ep);
             BCMGX_LAUNCHED();
             return;
         }
@@ -872,8 +895,8 @@ static void launch1(Context* c, const SpmvArgs& a, int L) {
     if (L <= -200) {
 #define BCMGX_S2(TT)                                                                                           \
     case TT:                                                                                                   \
-        k_spmv_stream2<T, V, TT, OP><<<grid_for(a.n, WG / TT), WG, 0, c->stream>>>(a.n, a.nnz, a.row, a.col, val, x, \
-                                                                                  y, b, D, al, be, a.stop, sb); \
+        k_spmv_stream2<T, V, TT, OP, EPI><<<grid_for(a.n, WG / TT), WG, 0, c->stream>>>(a.n, a.nnz, a.row, a.col, val, x, \
+                                                                                  y, b, D, al, be, a.stop, sb, ep); \
         break;
         switch (-L - 200) {
             BCMGX_S2(1) BCMGX_S2(2) BCMGX_S2(4) BCMGX_S2(8) BCMGX_S2(16)
@@ -886,8 +909,8 @@ static void launch1(Context* c, const SpmvArgs& a, int L) {
     if (L < 0) {  // CSR-stream variant, TPR = -L lanes per row
 #define BCMGX_S(TT)                                                                                                 \
     case TT:                                                                                                        \
-        k_spmv_stream<T, V, TT, OP><<<grid_for(a.n, WG / TT), WG, 0, c->stream>>>(a.n, a.row, a.col, val, x, y, b, D, \
-                                                                                 al, be, a.stop, sb);               \
+        k_spmv_stream<T, V, TT, OP, EPI><<<grid_for(a.n, WG / TT), WG, 0, c->stream>>>(a.n, a.row, a.col, val, x, y, b, D, \
+                                                                                 al, be, a.stop, sb, ep);               \
         break;
         switch (-L) {
             BCMGX_S(1) BCMGX_S(2) BCMGX_S(4) BCMGX_S(8) BCMGX_S(16)
@@ -899,8 +922,8 @@ static void launch1(Context* c, const SpmvArgs& a, int L) {
     }
 #define BCMGX_L(LL)                                                                                            \
     case LL:                                                                                                   \
-        k_spmv1<T, V, LL, OP><<<grid_for(a.n, WG / LL), WG, 0, c->stream>>>(a.n, a.row, a.col, val, x, y, b, D, \
-                                                                          al, be, a.stop);                   \
+        k_spmv1<T, V, LL, OP, EPI><<<grid_for(a.n, WG / LL), WG, 0, c->stream>>>(a.n, a.row, a.col, val, x, y, b, D, \
+                                                                          al, be, a.stop, ep);                   \
         break;
     switch (L) {
         BCMGX_L(1) BCMGX_L(2) BCMGX_L(4) BCMGX_L(8) BCMGX_L(16) BCMGX_L(32) BCMGX_L(64)
@@ -1011,6 +1034,8 @@ void spmv(Context* c, SpOp op, const SpmvArgs& a) {
             SpmvArgs b = a;
             b.kchunk = 0;
             dispatch_spmmp<T, V, SpOp::AX, 3>(c, b, ex, 0);
+        } else if (a.k == 1 && a.n > 0 && a.row && (a.nnz == 0 || (a.col && a.val && a.x))) {
+            launch1<T, V, SpOp::AX, EPI_X0>(c, a, a.lanes != 0 ? a.lanes : default_lanes(a.nnz, a.n));
         } else {
             SpmvArgs b = a;
             b.x0 = nullptr;
@@ -1025,8 +1050,14 @@ void spmv(Context* c, SpOp op, const SpmvArgs& a) {
         throw Error(BCMGX_ERR_STATE, "spmv: null operand");
     if (a.b64 && (a.k == 1 || op != SpOp::RES || !std::is_same<V, float>::value))
         throw Error(BCMGX_ERR_STATE, "spmv: an FP64 right-hand side only on the pipelined k-column residual");
+    if (a.up_out && (a.k != 1 || op != SpOp::JACOBI || !a.up_row || !a.up_col || !a.up_val || !a.up_in || a.up_out == a.up_in))
+        throw Error(BCMGX_ERR_STATE, "spmv: bad prolongation operand");
     if (a.k == 1) {
         int L = a.lanes != 0 ? a.lanes : default_lanes(a.nnz, a.n);  // < 0: CSR-stream kernel
+        if (a.up_out) {
+            launch1<T, V, SpOp::JACOBI, EPI_UP>(c, a, L);
+            return;
+        }
         switch (op) {
         case SpOp::AX: launch1<T, V, SpOp::AX>(c, a, L); break;
         case SpOp::RES: launch1<T, V, SpOp::RES>(c, a, L); break;
@@ -1199,6 +1230,13 @@ void galerkin_post_sweep(Context* c, const SpmvArgs& a, const int* agg, const V*
         return;
     }
     SpmvArgs b = a;
+    if (a.k == 1) {
+        b.agg = agg;
+        b.pv = pval;
+        b.xpre = xpre;
+        launch1<V, V, SpOp::AX, EPI_POST>(c, b, a.lanes != 0 ? a.lanes : default_lanes(a.nnz, a.n));
+        return;
+    }
     b.b = nullptr;
     b.D = nullptr;
     spmv<V, V>(c, SpOp::AX, b);  // t = (A P) e into y
