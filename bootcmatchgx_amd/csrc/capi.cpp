@@ -92,6 +92,18 @@ static void stage_out(Context* c, const double* src_interleaved, double* dst, in
     }
 }
 
+// n 8-byte aligned doubles at p that kernels of this context's device can use in place
+static bool on_device(Context* c, const double* p) {
+    hipPointerAttribute_t at;
+    if (((uintptr_t)p & 7) != 0) return false;
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();  // memory that HIP does not know
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == c->device;
+}
+static bool apart(const double* x, size_t nx, const double* y, size_t ny) { return x + nx <= y || y + ny <= x; }
+
 extern "C" {
 
 const char* bcmgx_error_string(int s) {
@@ -750,6 +762,26 @@ int bcmgx_spmm(bcmgx_context ctx, bcmgx_matrix A, const double* x, double* y, in
     BCMGX_HIP(hipSetDevice(c->device));
     const DCsr& M = A->A;
     if (ld < std::max(M.n, M.m)) throw Error(BCMGX_ERR_ARG, "leading dimension smaller than the matrix");
+    SpOp o = op == 1 ? SpOp::AX : (op == 2 ? SpOp::RES : SpOp::AXPBY);
+    // device columns that do not overlap: multiplied where they are
+    size_t span = (size_t)ld * (k - 1);
+    if (mem != BCMGX_MEM_HOST && M.n > 0 && kchunk == 0 && on_device(c, x) && on_device(c, y) &&
+        apart(x, span + M.m, y, span + M.n)) {
+        if (k == 1) {
+            SpmvArgs a;
+            a.n = M.n; a.row = M.row.get(); a.col = M.col.get(); a.val = M.val.get(); a.nnz = M.nnz;
+            set_tiles(a, M);
+            a.x = x; a.y = y; a.b = y; a.alpha = alpha; a.beta = beta;
+            a.lanes = tune_lanes(c, M, false);
+            spmv<double, double>(c, o, a);
+            c->sync();
+            return BCMGX_OK;
+        }
+        if (spmm_colmajor(c, o, M, x, y, k, ld, alpha, beta)) {
+            c->sync();
+            return BCMGX_OK;
+        }
+    }
     DBuf<double> X(c, (size_t)std::max(M.m, 1) * k), Y(c, (size_t)std::max(M.n, 1) * k), tmp;
     stage_in(c, x, ld, mem, M.m, k, X.get(), tmp);
     if (op != 1) stage_in(c, y, ld, mem, M.n, k, Y.get(), tmp);
@@ -758,7 +790,6 @@ int bcmgx_spmm(bcmgx_context ctx, bcmgx_matrix A, const double* x, double* y, in
     set_tiles(a, M);
     a.x = X.get(); a.y = Y.get(); a.b = Y.get(); a.alpha = alpha; a.beta = beta; a.k = k; a.kchunk = kchunk;
     a.lanes = k == 1 ? tune_lanes(c, M, false) : 0;
-    SpOp o = op == 1 ? SpOp::AX : (op == 2 ? SpOp::RES : SpOp::AXPBY);
     spmv<double, double>(c, o, a);
     stage_out(c, Y.get(), y, ld, mem, M.n, k, tmp);
     c->sync();

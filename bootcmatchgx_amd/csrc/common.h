@@ -221,6 +221,9 @@ struct DCsr {
     DBuf<float> valf;  // FP32 copy for the mixed-precision cycle (may be empty)
     DBuf<int> tu, tucol;            // row-tile index (empty until built)
     DBuf<unsigned short> tlidx;
+    long long tile_cols = 0, tile_runs = 0;  // its listed columns, and the runs of consecutive ones
+    int tile_widest = 0;            // the most columns of a tile
+    int tiles_left_out = 0;         // tiles with entries that it does not index
     BlockForm blk;                  // block form (empty until built)
     bool unit_rows = false;         // row i holds exactly entry i (row pointers 0, 1, .., n): a prolongator
     int maxrow = -1;                // entries in the longest row (-1: not known)

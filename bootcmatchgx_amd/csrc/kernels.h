@@ -331,6 +331,12 @@ int spmm_blocked_dots_blocks(Context* c, int k);
 bool spmm_blocked_dots(Context* c, const SpmvArgs& a, const double* r, const double* wold, double* partials, int nblk,
                        const int* all_done);
 
+// ---- k-column products over the row-tile index (tiled.hip) --------------------------
+// AX, RES (y - A x) or AXPBY on k column-major columns (leading dimension ld, x and y apart, both on the
+// context's device), the bits of the interleaved kernels; false (nothing launched) where the index is not
+// there, leaves tiles out, or lists columns in short runs
+bool spmm_colmajor(Context* c, SpOp op, const DCsr& A, const double* x, double* y, int k, int ld, double alpha, double beta);
+
 // ---- coarsest-level sweeps (coarse.hip) ---------------------------------------------
 constexpr int CO_MAX_N = 32768;      // rows and sweeps the one-launch form takes (its slots: 16 bytes per row and sweep)
 constexpr int CO_MAX_SWEEPS = 64;

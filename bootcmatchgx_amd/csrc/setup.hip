@@ -1508,7 +1508,8 @@ bool galerkin(Context* c, const DCsr& A, int nc, const int* agg, const double* p
 // distinct columns; others count 0.
 __global__ __launch_bounds__(WG) void k_tile_cols(int n, int rows, const int* __restrict__ row,
                                                   const int* __restrict__ col, int* __restrict__ ucnt, const int* __restrict__ tu,
-                                                  int* __restrict__ tucol, unsigned short* __restrict__ tlidx, int phase) {
+                                                  int* __restrict__ tucol, unsigned short* __restrict__ tlidx, int phase,
+                                                  int* __restrict__ runs = nullptr) {
     __shared__ int keys[TILE_MAX_ENTRIES];
     __shared__ int uniq[TILE_MAX_COLS];
     __shared__ int wsum[WG / 64];
@@ -1519,7 +1520,10 @@ __global__ __launch_bounds__(WG) void k_tile_cols(int n, int rows, const int* __
     bool fits = cnt > 0 && cnt + (base & 1) <= TILE_MAX_ENTRIES;
     if (phase == 1 && tu[t + 1] == tu[t]) return;  // not indexed
     if (!fits) {
-        if (phase != 1 && tid == 0) ucnt[t] = 0;
+        if (phase != 1 && tid == 0) {
+            ucnt[t] = 0;
+            if (runs) runs[t] = cnt > 0 ? -1 : 0;
+        }
         return;
     }
     int P = 1;
@@ -1544,10 +1548,11 @@ __global__ __launch_bounds__(WG) void k_tile_cols(int n, int rows, const int* __
     }
     // distinct columns in order: heads of runs, ranked by a block scan per chunk of WG
     int lane = tid & 63, w = tid >> 6;
-    int carry = 0;
+    int carry = 0, nrun = 0;
     for (int c0 = 0; c0 < cnt; c0 += WG) {
         int p = c0 + tid;
         bool head = p < cnt && (p == 0 || keys[p] != keys[p - 1]);
+        if (runs) nrun += __syncthreads_count(head && (p == 0 || keys[p] != keys[p - 1] + 1));
         unsigned long long m = __ballot(head);
         int below = __popcll(m & ((1ull << lane) - 1ull));
         if (lane == 0) wsum[w] = __popcll(m);
@@ -1562,7 +1567,10 @@ __global__ __launch_bounds__(WG) void k_tile_cols(int n, int rows, const int* __
     }
     int U = carry <= TILE_MAX_COLS ? carry : 0;
     if (phase != 1) {
-        if (tid == 0) ucnt[t] = U;
+        if (tid == 0) {
+            ucnt[t] = U;
+            if (runs) runs[t] = U > 0 ? nrun : -1;
+        }
         if (phase == 0 || U == 0) return;
     }
     int u0 = phase == 1 ? tu[t] : t * TILE_MAX_COLS;
@@ -1584,13 +1592,51 @@ void tile_columns_strided(Context* c, const DCsr& A, int rows, int* ucnt, int* u
     BCMGX_LAUNCHED();
 }
 
+// out = {runs of all tiles, tiles left out, columns of the widest} (one workgroup: some 1e5 tiles at most)
+__global__ __launch_bounds__(1024) void k_tile_runs(int nt, const int* __restrict__ runs, const int* __restrict__ ucnt,
+                                                    long long* __restrict__ out) {
+    __shared__ long long s[3][1024];
+    long long a = 0;
+    int b = 0, m = 0;
+    for (int t = threadIdx.x; t < nt; t += 1024) {
+        int v = runs[t], u = ucnt[t];
+        if (v < 0) b++;
+        else a += v;
+        if (u > m) m = u;
+    }
+    s[0][threadIdx.x] = a;
+    s[1][threadIdx.x] = b;
+    s[2][threadIdx.x] = m;
+    __syncthreads();
+    for (int o = 512; o > 0; o >>= 1) {
+        if (threadIdx.x < o) {
+            s[0][threadIdx.x] += s[0][threadIdx.x + o];
+            s[1][threadIdx.x] += s[1][threadIdx.x + o];
+            s[2][threadIdx.x] = std::max(s[2][threadIdx.x], s[2][threadIdx.x + o]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 3) out[threadIdx.x] = s[threadIdx.x][0];
+}
+
 void build_tile_index(Context* c, DCsr& A) {
     if (A.tiled() || A.n <= 0) return;
     int nt = (A.n + TILE_ROWS - 1) / TILE_ROWS;
-    DBuf<int> cnt(c, nt), tu(c, (size_t)nt + 1);
-    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, TILE_ROWS, A.row.get(), A.col.get(), cnt.get(), nullptr, nullptr, nullptr, 0);
+    DBuf<int> cnt(c, nt), runs(c, nt), tu(c, (size_t)nt + 1);
+    DBuf<long long> sums(c, 3);
+    k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, TILE_ROWS, A.row.get(), A.col.get(), cnt.get(), nullptr, nullptr, nullptr, 0,
+                                          runs.get());
     BCMGX_LAUNCHED();
-    long long tot = scan_exclusive(c, cnt.get(), tu.get(), nt);
+    k_tile_runs<<<1, 1024, 0, c->stream>>>(nt, runs.get(), cnt.get(), sums.get());
+    BCMGX_LAUNCHED();
+    scan_exclusive_async(c, cnt.get(), tu.get(), nt);
+    int tot = 0;
+    long long rs[3];
+    c->d2h2(&tot, tu.get() + nt, 1, rs, sums.get(), 3);
+    A.tile_cols = tot;
+    A.tile_runs = rs[0];
+    A.tiles_left_out = (int)rs[1];
+    A.tile_widest = (int)rs[2];
     DBuf<int> tucol(c, (size_t)std::max<long long>(tot, 1));
     DBuf<unsigned short> tlidx(c, (size_t)std::max(A.nnz, 2));
     k_tile_cols<<<nt, WG, 0, c->stream>>>(A.n, TILE_ROWS, A.row.get(), A.col.get(), cnt.get(), tu.get(), tucol.get(), tlidx.get(), 1);
