@@ -484,7 +484,7 @@ void Prec::ensure_work(int k) {
             nl = std::max(nl, hrc(h).levels());
             ncoarse = std::max(ncoarse, hrc(h).L.back()->mat().n);
         }
-        if (coarse_sweeps_fit(ncoarse, p.relaxnumber_coarse)) coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse);
+        if (coarse_sweeps_fit(ncoarse, p.relaxnumber_coarse)) coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse, k);
         std::vector<size_t> lsz(nl, 1);
         for (int h = 0; h < n_hrc(); h++)
             for (int l = 0; l < hrc(h).levels(); l++) lsz[l] = std::max(lsz[l], (size_t)hrc(h).L[l]->mat().n);
@@ -625,6 +625,11 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
                 if (coarse_sweeps<V>(c, A, lv.lanesA, lv.M.get(), F, xzero ? nullptr : cur, y, p.relaxnumber_coarse,
                                      lv.cix, pr->coarse, R.stop))
                     return y;
+            } else {
+                V* y = xzero ? cur : oth;
+                if (coarse_sweeps_columns<V>(c, A, lv.M.get(), F, xzero ? nullptr : cur, y, k, p.relaxnumber_coarse, lv.cix,
+                                             pr->coarse, R.stop))
+                    return y;
             }
             if (xzero && p.relaxnumber_coarse >= 1) {  // widening and the first sweep from zero in one pass
                 jacobi_from_zero_f32in(c, A.n, k, F, lv.M.get(), pr->cd_F.get(), pr->cd_X.get(), R.stop);
@@ -646,6 +651,11 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
                     if (up) up->done = true;
                     return y;
                 }
+            } else {
+                V* y = xzero ? cur : oth;
+                if (coarse_sweeps_columns<V>(c, A, lv.M.get(), F, xzero ? nullptr : cur, y, k, p.relaxnumber_coarse, lv.cix,
+                                             pr->coarse, R.stop))
+                    return y;
             }
             return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, p.relaxnumber_coarse, xzero, k, R.stop,
                                     lv.chunkA, nullptr, nullptr, up);

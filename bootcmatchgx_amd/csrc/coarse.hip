@@ -22,6 +22,10 @@ namespace bcmgx {
 
 constexpr int CO_ROWS = 32;          // rows per workgroup of the exchanging kernel
 constexpr int CO_FETCH = 4;          // listed columns a thread of it fetches
+constexpr int CO_COLS = 8;           // columns per workgroup of the k-column kernel
+constexpr int CO_COL_PLACES = 512;   // its LDS places: distinct columns of a tile, and a zero
+constexpr int CO_COL_FETCH = 8;      // elements a thread of it has in flight
+constexpr size_t CO_SLOT_WORDS = size_t(8) << 20;  // 64 MB
 constexpr int CO_SMALL_T = 1024;    // threads of the one-workgroup kernel
 constexpr int CO_SMALL_N = 1024;    // rows it holds in LDS
 constexpr int CO_SMALL_RR = 4;      // rows per lane group there
@@ -319,8 +323,12 @@ void CoarseIndex::build(Context* c, const DCsr& A) {
     tile_columns_strided(c, A, CO_ROWS, ucnt.get(), ucol.get(), upos.get());
 }
 
-void CoarseSync::reserve(Context* c, int n, int sweeps) {
+void CoarseSync::reserve(Context* c, int n, int sweeps, int k) {
     size_t need = (size_t)n * (size_t)std::max(sweeps, 1) * 2;
+    if (k > 1) {  // whole groups of columns
+        size_t all = need * CO_COLS * ((k + CO_COLS - 1) / CO_COLS);
+        if (all <= CO_SLOT_WORDS) need = all;
+    }
     if (slots.size() >= need && scratch.size() >= (size_t)n * 2) return;
     slots.reset(c, need);
     scratch.reset(c, (size_t)n * 2);
@@ -368,5 +376,209 @@ template bool coarse_sweeps<double>(Context*, const DCsr&, int, const double*, c
                                     const CoarseIndex&, CoarseSync&, const int*, const RowProlong<double>&);
 template bool coarse_sweeps<float>(Context*, const DCsr&, int, const double*, const float*, const float*, float*, int,
                                    const CoarseIndex&, CoarseSync&, const int*, const RowProlong<float>&);
+
+// The exchanging kernel for k columns: CC of them per workgroup, a thread per row and column, the row
+// summed in order as the k-column kernels do (the same bits).  Slots: [group of CC columns][sweep][row][CC][2],
+// so the columns of an element are fetched together; a group past k carries zeros.  The entries' values
+// and places are in registers, one LDS buffer holds the tile's distinct elements (place U: zero).
+// 8 columns of 4096 rows (27-point 128^3), 20 sweeps: 186 us as launches (130 in a replayed graph), 60 here;
+// 3 us a sweep, two rounds of loads through the memory side and the row sums from LDS.
+template <typename V, int E>
+__global__ __launch_bounds__(CO_ROWS * CO_COLS, E > 32 ? 2 : E > 16 ? 3 : 4) void k_coarse_columns(
+    int n, int k, const int* __restrict__ row, const int* __restrict__ col, const double* __restrict__ val,
+    const double* __restrict__ D, const V* __restrict__ f, const V* __restrict__ x0, V* __restrict__ out, int sweeps,
+    const int* __restrict__ ucnt, const int* __restrict__ ucol, const unsigned short* __restrict__ upos, u64* slots,
+    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience) {
+    constexpr int CC = CO_COLS, T = CO_ROWS * CC, NU = CO_COL_FETCH;
+    if (stop && *stop) return;
+    __shared__ double xs[CO_COL_PLACES * CC];
+    __shared__ int s_late, s_last;
+    int tid = threadIdx.x, cl = tid % CC;
+    int r = blockIdx.x * CO_ROWS + tid / CC;
+    int c = (int)blockIdx.y * CC + cl;
+    bool on = r < n, act = c < k;
+    unsigned base = ctl[0];
+    u64* mine = slots + (size_t)blockIdx.y * sweeps * n * CC * 2;
+    int U = ucnt[blockIdx.x];
+    bool listed = U > 0 && U < CO_COL_PLACES;
+    const int* list = ucol + (size_t)blockIdx.x * TILE_MAX_COLS;
+    if (tid == 0) s_late = 0;
+    if (listed && tid < CC) xs[U * CC + tid] = 0.0;
+    int rs = on ? row[r] : 0, re = on ? row[r + 1] : 0;
+    double a[E];
+    unsigned at[E / 2];
+#pragma unroll
+    for (int q = 0; q < E; q += 2) {
+        bool i0 = listed && rs + q < re, i1 = listed && rs + q + 1 < re;
+        a[q] = i0 ? val[rs + q] : 0.0;
+        a[q + 1] = i1 ? val[rs + q + 1] : 0.0;
+        at[q / 2] = (i0 ? upos[rs + q] : (listed ? U : 0)) | (unsigned)(i1 ? upos[rs + q + 1] : (listed ? U : 0)) << 16;
+    }
+    double fr = on && act ? (double)f[(size_t)r * k + c] : 0.0, Dr = on ? D[r] : 1.0;
+    auto first = [&](int i) {
+        return !act ? 0.0 : x0 ? (double)x0[(size_t)i * k + c] : (double)f[(size_t)i * k + c] / D[i];
+    };
+    int done = x0 ? 0 : 1;
+    double xr = x0 ? (on && act ? (double)x0[(size_t)r * k + c] : 0.0) : fr / Dr;
+    bool given_up = false;  // uniform over the workgroup
+    for (int s = done; s < sweeps; s++) {
+        double t = 0;
+        if (s == done) {
+            if (listed) {
+                for (int u = tid / CC; u < U; u += CO_ROWS) xs[u * CC + cl] = first(list[u]);
+            } else {
+                for (int j = rs; j < re; j++) t += val[j] * first(col[j]);
+            }
+        } else {  // the elements that sweep s - 1 published
+            const u64* p = mine + (size_t)(s - 1) * n * CC * 2;
+            unsigned tag = base + (unsigned)s;
+            auto fetch = [&](unsigned o, double& v) {  // o: bytes, below 2^32 (one register an address)
+                const u64* e = (const u64*)((const char*)p + o);
+                u64 lo = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                u64 hi = __hip_atomic_load(e + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                v = __hiloint2double((int)(unsigned)hi, (int)(unsigned)lo);
+                return (unsigned)(lo >> 32) == tag && (unsigned)(hi >> 32) == tag;
+            };
+            long long t0 = 0;
+            bool late = patience < 0;  // negative: no waiting at all
+            int j = rs;                // without a list: the entry waited for
+            int u0 = tid / CC;         // with one: the first place of the NU waited for
+            for (int poll = 0; !late; poll++) {
+                if (listed) {
+                    while (u0 < U) {
+                        double v[NU];
+                        unsigned o[NU];
+                        bool ok = true;
+#pragma unroll
+                        for (int w = 0; w < NU; w++) o[w] = ((unsigned)list[min(u0 + w * CO_ROWS, U - 1)] * CC + cl) * 16u;
+#pragma unroll
+                        for (int w = 0; w < NU; w++) ok = fetch(o[w], v[w]) & ok;
+                        if (!ok) break;
+#pragma unroll
+                        for (int w = 0; w < NU; w++) xs[min(u0 + w * CO_ROWS, U - 1) * CC + cl] = v[w];
+                        u0 += NU * CO_ROWS;
+                    }
+                    if (u0 >= U) break;
+                } else {
+                    double v;
+                    while (j < re && fetch(((unsigned)col[j] * CC + cl) * 16u, v)) t += val[j++] * v;
+                    if (j >= re) break;
+                }
+                if ((poll & 15) == 15) {
+                    if (poll == 15) t0 = wall_clock64();
+                    else if (wall_clock64() - t0 > patience) late = true;
+                    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) late = true;
+                }
+            }
+            if (late) {
+                s_late = s + 1;
+                __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+        __syncthreads();
+        if (s_late == s + 1) {
+            given_up = true;
+            break;
+        }
+        if (listed) {
+#pragma unroll
+            for (int q = 0; q < E; q += 4) {
+                if (!__any(rs + q < re)) break;
+                unsigned p01 = at[q / 2], p23 = at[q / 2 + 1];
+                asm("" : "+v"(p01), "+v"(p23));  // unpacked here: E addresses kept over the sweeps would spill
+                double v0 = xs[(p01 & 0xffffu) * CC + cl], v1 = xs[(p01 >> 16) * CC + cl];
+                double v2 = xs[(p23 & 0xffffu) * CC + cl], v3 = xs[(p23 >> 16) * CC + cl];
+                t += a[q] * v0;
+                t += a[q + 1] * v1;
+                t += a[q + 2] * v2;
+                t += a[q + 3] * v3;
+            }
+        }
+        xr = ((-t + fr) / Dr) + xr;
+        if (s + 1 < sweeps && on) {
+            u64* p = mine + (((size_t)s * n + r) * CC + cl) * 2;
+            u64 tag = (u64)(base + (unsigned)s + 1u) << 32;
+            __hip_atomic_store(p, tag | (unsigned)__double2loint(xr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(p + 1, tag | (unsigned)__double2hiint(xr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();  // xs is read: the next elements take its place
+    }
+    if (!given_up && on && act) out[(size_t)r * k + c] = (V)xr;
+    __syncthreads();
+    if (tid == 0) {
+        __threadfence();
+        s_last = atomicAdd(ctl + 1, 1u) == gridDim.x * gridDim.y - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the last workgroup: every other one has passed its waits for good
+    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        for (int q = 0; q < k; q++) {
+            double* cur = scratch;
+            double* nxt = scratch + n;
+            for (int i = tid; i < n; i += T) cur[i] = x0 ? (double)x0[(size_t)i * k + q] : (double)f[(size_t)i * k + q] / D[i];
+            __threadfence();
+            __syncthreads();
+            for (int s = done; s < sweeps; s++) {
+                for (int i = tid; i < n; i += T) {
+                    double t = 0;
+                    for (int j = row[i]; j < row[i + 1]; j++) t += val[j] * cur[col[j]];
+                    nxt[i] = ((-t + (double)f[(size_t)i * k + q]) / D[i]) + cur[i];
+                }
+                __threadfence();
+                __syncthreads();
+                double* w = cur;
+                cur = nxt;
+                nxt = w;
+            }
+            for (int i = tid; i < n; i += T) out[(size_t)i * k + q] = (V)cur[i];
+            __syncthreads();
+        }
+    }
+    if (tid == 0) {
+        ctl[0] = base + (unsigned)sweeps + 1u;
+        ctl[1] = 0;
+        ctl[2] = 0;
+    }
+}
+
+template <typename V, int E>
+static bool launch_columns(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int k, int sweeps,
+                           const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+    auto kern = k_coarse_columns<V, E>;
+    static int resident = 0;  // workgroups the device holds, per instantiation; identical devices assumed within a process
+    if (!resident) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, CO_ROWS * CO_COLS, 0) != hipSuccess) per_cu = 0;
+        resident = c->num_cus * per_cu + 1;
+    }
+    int tiles = (int)grid_for(A.n, CO_ROWS), groups = (k + CO_COLS - 1) / CO_COLS;
+    // to one workgroup a CU: beyond, the fetches of 128 bytes an element and row of columns bound a sweep (32
+    // columns of 4096 rows, 512 workgroups: 114 us, and the same as 20 launches)
+    if (tiles * groups > c->num_cus || tiles * groups * 2 > resident ||
+        (size_t)A.n * sweeps * groups * CO_COLS * 2 > cs.slots.size())
+        return false;
+    kern<<<dim3(tiles, groups), CO_ROWS * CO_COLS, 0, c->stream>>>(
+        A.n, k, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, sweeps, ix.ucnt.get(), ix.ucol.get(), ix.upos.get(),
+        cs.slots.get(), cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience);
+    BCMGX_LAUNCHED();
+    return true;
+}
+
+template <typename V>
+bool coarse_sweeps_columns(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int k, int sweeps,
+                           const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
+    if (k < 2 || !coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || !ix.ucnt || (const void*)out == (const void*)x0 ||
+        (const void*)out == (const void*)f || cs.scratch.size() < (size_t)A.n * 2)
+        return false;
+    if (A.maxrow <= 16) return launch_columns<V, 16>(c, A, D, f, x0, out, k, sweeps, ix, cs, stop);
+    if (A.maxrow <= 32) return launch_columns<V, 32>(c, A, D, f, x0, out, k, sweeps, ix, cs, stop);
+    if (A.maxrow <= 64) return launch_columns<V, 64>(c, A, D, f, x0, out, k, sweeps, ix, cs, stop);
+    return false;
+}
+template bool coarse_sweeps_columns<double>(Context*, const DCsr&, const double*, const double*, const double*, double*, int, int,
+                                            const CoarseIndex&, CoarseSync&, const int*);
+template bool coarse_sweeps_columns<float>(Context*, const DCsr&, const double*, const float*, const float*, float*, int, int,
+                                           const CoarseIndex&, CoarseSync&, const int*);
 
 }  // namespace bcmgx

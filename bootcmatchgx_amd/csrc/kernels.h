@@ -344,10 +344,10 @@ bool coarse_sweeps_fit(int n, int sweeps);
 // What the one-launch sweeps exchange through, kept with a preconditioner (one stream):
 // ctl = {tag base, finished workgroups, a wait gave up}, zero between launches but the base
 struct CoarseSync {
-    DBuf<unsigned long long> slots;  // [sweep][row][2]
+    DBuf<unsigned long long> slots;  // [sweep][row][2], or [columns][sweep][row][column][2]
     DBuf<double> scratch;            // 2 n, for the workgroup that finishes after waits gave up
     DBuf<unsigned> ctl;
-    void reserve(Context* c, int n, int sweeps);
+    void reserve(Context* c, int n, int sweeps, int k);
 };
 // the distinct columns of each 32-row tile of a coarsest operator, listed at setup (setup.hip's
 // tile columns at a fixed stride)
@@ -363,6 +363,12 @@ struct CoarseIndex {
 template <typename V>
 bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const V* f, const V* x0, V* out, int sweeps,
                    const CoarseIndex& ix, CoarseSync& cs, const int* stop, const RowProlong<V>& up = RowProlong<V>());
+
+// the same on k > 1 interleaved columns, each column's rows summed in order (the k-column kernels' bits);
+// out is neither x0 nor f
+template <typename V>
+bool coarse_sweeps_columns(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int k, int sweeps,
+                           const CoarseIndex& ix, CoarseSync& cs, const int* stop);
 
 // ---- AFSAI (afsai.hip) ------------------------------------------------------------
 void afsai_build(Context* c, const DCsr& A, DCsr& G, DCsr& GT);
