@@ -417,6 +417,7 @@ struct SolveWork {
     DBuf<FcgState> st;
     DBuf<int> flags;  // [0] all_done, [1] columns done
     FcgBufs fb;
+    DBuf<unsigned> tickets;
     FcgEntry entry;     // level-0 entry of the FP32 cycle filled by the updates
     bool fused = false;
     // FP32 z: the cycle's result kept in FP32 and widened inside the fused product and the update
@@ -844,7 +845,10 @@ void Prec::apply(const double* r, double* u, int k, bool x_zero, const int* stop
         copy_d2d(c, u, r, sizeof(double) * nk);
         break;
     case BCMGX_PREC_L1_JACOBI: {  // l1jacobi_apply (l1jacobi.cu:513-523)
-        double* res = jacobi_sweeps<double>(c, *A, H.L.empty() ? 0 : 0, pl1j.get(), r, u, tmp.get(), p.l1jacsweeps, x_zero, k, stop);
+        // from zero the sweeps can start in either buffer: so that the last one ends in u
+        double* cur = x_zero && p.l1jacsweeps > 0 && p.l1jacsweeps % 2 == 0 ? tmp.get() : u;
+        double* res = jacobi_sweeps<double>(c, *A, H.L.empty() ? 0 : 0, pl1j.get(), r, cur, cur == u ? tmp.get() : u, p.l1jacsweeps,
+                                            x_zero, k, stop);
         if (res != u) copy_d2d(c, u, res, sizeof(double) * nk);
         break;
     }
@@ -1093,7 +1097,6 @@ static void fcg_iteration_z32(Context* c, const DCsr& A, Prec* prec, SolveWork& 
     int nblk = fused_z32(c, A, s, s.q.get(), stop, s.fb.all_done);
     fcg_scalars3(c, s.fb, nblk, idx);
     fcg_update_z32(c, s.fb, s.zf.get(), s.d.get(), s.w.get(), s.q.get(), s.X.get(), s.r.get(), idx, s.entry);
-    fcg_finish_iteration(c, s.fb, idx);
 }
 
 static void fcg_iteration(Context* c, const DCsr& A, Prec* prec, SolveWork& s, int idx) {
@@ -1118,7 +1121,6 @@ static void fcg_iteration(Context* c, const DCsr& A, Prec* prec, SolveWork& s, i
         fcg_dots3(c, s.fb, s.r.get(), P0, W0, W1, idx);
     }
     fcg_update(c, s.fb, P0, P1, W0, W1, s.X.get(), s.r.get(), idx, s.entry);
-    fcg_finish_iteration(c, s.fb, idx);
 }
 
 // the Krylov workspace for k columns of A (kept per k: graphs are bound to it)
@@ -1145,6 +1147,9 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
         s.partials.reset(c, (size_t)std::max({s.fb.nblk, s.mv_blocks, s.z32_blocks, s.z32_blk_grid}) * k * 3);
         s.st.reset(c, k);
         s.flags.reset(c, 3);
+        s.tickets.reset(c, FCG_TICKETS);
+        fill<int>(c, (int*)s.tickets.get(), FCG_TICKETS, 0);
+        s.fb.tickets = s.tickets.get();
         s.fb.partials = s.partials.get();
         s.fb.st = s.st.get();
         s.fb.all_done = s.flags.get();

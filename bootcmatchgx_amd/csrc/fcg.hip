@@ -60,38 +60,6 @@ struct RowSplit {
     }
 };
 
-// NV dot products per column over a row range; partials[(blk*k + c)*3 + m]
-template <int NV>
-__global__ __launch_bounds__(WG) void k_dots(int n, int k, const double* __restrict__ a0, const double* __restrict__ b0,
-                                             const double* __restrict__ a1, const double* __restrict__ b1,
-                                             const double* __restrict__ a2, const double* __restrict__ b2,
-                                             double* __restrict__ partials, const int* __restrict__ all_done) {
-    if (all_done && *all_done) return;
-    __shared__ double s[NV][WG];
-    int tid = threadIdx.x;
-    const RowSplit sp(k);
-    int c = sp.c;
-    double acc[NV];
-#pragma unroll
-    for (int m = 0; m < NV; m++) acc[m] = 0.0;
-    if (sp.active()) {
-        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
-            long long o = i * k + c;
-            acc[0] += a0[o] * b0[o];
-            if (NV > 1) acc[1] += a1[o] * b1[o];
-            if (NV > 2) acc[2] += a2[o] * b2[o];
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < NV; m++) s[m][tid] = acc[m];
-    __syncthreads();
-    sp.sum<NV>(s, k);
-    if (tid < k) {
-#pragma unroll
-        for (int m = 0; m < NV; m++) partials[((long long)blockIdx.x * k + tid) * 3 + m] = s[m][tid];
-    }
-}
-
 // sum partials of column blockIdx.x in a fixed tree; thread 0 gets the totals
 template <int NV>
 __device__ void sum_partials(const double* __restrict__ partials, int nblk, int k, int c, double* out, double (*s)[WG]) {
@@ -114,6 +82,206 @@ __device__ void sum_partials(const double* __restrict__ partials, int nblk, int 
     if (tid == 0)
 #pragma unroll
         for (int m = 0; m < NV; m++) out[m] = s[m][0];
+}
+
+// What follows a reduction, per column from its totals.  FIN_SCALARS: FCG's theta, delta,
+// theta2; FIN_STEP: FCG's ||r||, iteration count and convergence; FIN_BETA, FIN_ALPHA,
+// FIN_ALPHA0 (first iteration) and FIN_CG: the same of CG.
+enum { FIN_NONE, FIN_SCALARS, FIN_STEP, FIN_BETA, FIN_ALPHA, FIN_ALPHA0, FIN_CG };
+constexpr int fin_values(int fin) { return fin == FIN_SCALARS ? 3 : fin == FIN_ALPHA0 ? 2 : 1; }
+struct FinArgs {
+    FcgState* st;
+    int* all_done;
+    int* ndone;
+    unsigned* tickets;  // null: a kernel of its own sums the partials
+    double rtol;
+    int itnlim, phase;
+};
+
+template <int FIN>
+__device__ void fin_column(FcgState& S, const double* tot, const FinArgs& a, int k) {
+    bool stop = false;
+    if constexpr (FIN == FIN_SCALARS) {
+        if (S.done) return;
+        S.alpha = tot[0];
+        S.beta = tot[1];
+        S.gamma = tot[2];
+        S.theta = S.gamma / S.delta;                        // FCG.cu:132
+        S.delta = S.beta - ((S.gamma * S.gamma) / S.delta);  // FCG.cu:135
+        S.theta2 = S.alpha / S.delta;                       // FCG.cu:136
+        if (a.phase == 0) {  // the x step of this iteration waits for the pair's second update
+            S.pend = S.theta2;
+            S.pad1 = 1;
+        }
+    } else if constexpr (FIN == FIN_STEP) {
+        // l2 = ||r||; iter++; stop when !(l2 > rtol*delta0 && iter < itnlim)  (FCG.cu:146-156)
+        if (a.phase == 1) S.pad1 = 0;  // this pair's update added the waiting step
+        if (S.done) return;
+        S.l2 = sqrt(tot[0]);
+        S.iter += 1;
+        stop = !(S.l2 > a.rtol * S.delta0 && S.iter < a.itnlim);
+    } else if constexpr (FIN == FIN_BETA) {
+        // rho = r.u, beta = rho / rho_prev  (CG_HS.cu:89-101)
+        if (S.done) return;
+        S.alpha = tot[0];
+        S.theta = S.alpha / S.delta;
+    } else if constexpr (FIN == FIN_ALPHA || FIN == FIN_ALPHA0) {
+        // (first iteration: rho = u.r) gamma = p.s, alpha = rho / gamma; rho_prev = rho  (CG_HS.cu:112-129)
+        if (S.done) return;
+        if constexpr (FIN == FIN_ALPHA0) S.alpha = tot[1];
+        S.gamma = tot[0];
+        S.theta2 = S.alpha / S.gamma;
+        S.delta = S.alpha;
+    } else if constexpr (FIN == FIN_CG) {
+        // l2 = ||r||; converged when l2 < rtol delta0, else the iteration count
+        // advances and itnlim stops the column (CG_HS.cu:134-163)
+        if (S.done) return;
+        S.l2 = sqrt(tot[0]);
+        if (S.l2 < a.rtol * S.delta0) {
+            S.pad0 = 1;
+            stop = true;
+        } else if (++S.iter >= a.itnlim) {
+            stop = true;
+        }
+    }
+    if (stop) {
+        S.done = 1;
+        if (atomicAdd(a.ndone, 1) + 1 == k) *a.all_done = 1;
+    }
+}
+
+// The partials of a kernel of their own, one workgroup per column
+template <int FIN>
+__global__ __launch_bounds__(WG) void k_final(const double* __restrict__ partials, int nblk, int k, FinArgs a) {
+    constexpr int NV = fin_values(FIN);
+    if (*a.all_done) return;
+    __shared__ double s[NV][WG];
+    double tot[NV];
+    int c = blockIdx.x;
+    sum_partials<NV>(partials, nblk, k, c, tot, s);
+    if (threadIdx.x == 0) fin_column<FIN>(a.st[c], tot, a, k);
+}
+
+// The end of a reducing kernel whose block's sums are in s[m][c] (m < NV, c < k): its partials
+// are left for k_final, or (tickets given) the workgroup that finishes last sums everyone's,
+// one wave a column, and does k_final's work: a launch of its own costs 4-5 us in a replayed
+// graph for less than one of work.  A partial is exchanged into its place at device scope and
+// the old value waited for, so it is visible across the XCDs before the workgroup takes its
+// ticket; no L2 is written back for it.  Tickets are taken 32 workgroups to a counter and then
+// 32 counters to one (1024 on one word queue up for microseconds), 64 bytes apart; the last
+// taker clears each for the next kernel.
+template <int FIN>
+__device__ __forceinline__ void block_end(double (*s)[WG], double* partials, int k, const FinArgs& a) {
+    constexpr int NV = fin_values(FIN);
+    int tid = threadIdx.x, nblk = gridDim.x;
+    if (!a.tickets) {
+        if (tid < k) {
+#pragma unroll
+            for (int m = 0; m < NV; m++) partials[((long long)blockIdx.x * k + tid) * 3 + m] = s[m][tid];
+        }
+        return;
+    }
+    if (tid < k) {
+        unsigned long long old[NV];
+#pragma unroll
+        for (int m = 0; m < NV; m++)
+            old[m] = __hip_atomic_exchange((unsigned long long*)partials + ((long long)blockIdx.x * k + tid) * 3 + m,
+                                           (unsigned long long)__double_as_longlong(s[m][tid]), __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int m = 0; m < NV; m++) asm volatile("" ::"v"(old[m]));  // back, so at the device's point of coherence
+    }
+    __shared__ int last;
+    __syncthreads();
+    if (tid == 0) {
+        unsigned group = blockIdx.x / 32, groups = (nblk + 31) / 32;
+        unsigned size = group + 1 < groups ? 32 : nblk - group * 32;
+        unsigned* mine = a.tickets + 16 * (1 + group);
+        last = 0;
+        if (__hip_atomic_fetch_add(mine, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == size - 1) {
+            __hip_atomic_store(mine, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (__hip_atomic_fetch_add(a.tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1) {
+                __hip_atomic_store(a.tickets, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                last = 1;
+            }
+        }
+    }
+    __syncthreads();
+    if (!last) return;
+    for (int c = tid / 64; c < k; c += WG / 64) {
+        double acc[NV];
+#pragma unroll
+        for (int m = 0; m < NV; m++) acc[m] = 0.0;
+        for (int b0 = tid & 63; b0 < nblk; b0 += 4 * 64) {  // four blocks' partials in flight
+            double v[4][NV];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                int b = b0 + u * 64 < nblk ? b0 + u * 64 : b0;
+#pragma unroll
+                for (int m = 0; m < NV; m++)
+                    v[u][m] = __longlong_as_double((long long)__hip_atomic_load(
+                        (const unsigned long long*)partials + ((long long)b * k + c) * 3 + m, __ATOMIC_RELAXED,
+                        __HIP_MEMORY_SCOPE_AGENT));
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int m = 0; m < NV; m++) acc[m] += b0 + u * 64 < nblk ? v[u][m] : 0.0;
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int m = 0; m < NV; m++) acc[m] += __shfl_xor(acc[m], o, 64);
+        if ((tid & 63) == 0) fin_column<FIN>(a.st[c], acc, a, k);
+    }
+}
+
+// The finishing step in the kernel to 1024 totals (workgroups by columns), else k_final: the
+// one workgroup that sums them is then slower than the launch it saves.  One column, 7-point
+// 10^3 1390 -> 1340 us a solve with its setup, 50^3 5.06 -> 4.83 ms, 160^3 (FP32 cycle) 67.2 -> 66.7
+// ms; 5 columns in 1024 workgroups (CG, 131150 rows) 9.5 -> 9.9 ms, so they keep k_final.
+constexpr int FIN_MAX_TOTALS = 1024;
+static FinArgs fin_args(const FcgBufs& f, int phase = 0) {
+    return FinArgs{f.st, f.all_done, f.all_done + 1, f.nblk * f.k <= FIN_MAX_TOTALS ? f.tickets : nullptr, f.rtol, f.itnlim, phase};
+}
+template <int FIN>
+static void fin_launch(Context* c, const FcgBufs& f, int nblk, const FinArgs& a) {
+    k_final<FIN><<<f.k, WG, 0, c->stream>>>(f.partials, nblk, f.k, a);
+    BCMGX_LAUNCHED();
+}
+
+// NV dot products per column over a row range; partials[(blk*k + c)*3 + m]
+template <int NV, int FIN = FIN_NONE>
+__global__ __launch_bounds__(WG) void k_dots(int n, int k, const double* __restrict__ a0, const double* __restrict__ b0,
+                                             const double* __restrict__ a1, const double* __restrict__ b1,
+                                             const double* __restrict__ a2, const double* __restrict__ b2,
+                                             double* __restrict__ partials, const int* all_done, FinArgs fa) {
+    if (all_done && *all_done) return;
+    __shared__ double s[NV][WG];
+    int tid = threadIdx.x;
+    const RowSplit sp(k);
+    int c = sp.c;
+    double acc[NV];
+#pragma unroll
+    for (int m = 0; m < NV; m++) acc[m] = 0.0;
+    if (sp.active()) {
+        for (long long i = (long long)blockIdx.x * sp.R + sp.rl; i < n; i += (long long)gridDim.x * sp.R) {
+            long long o = i * k + c;
+            acc[0] += a0[o] * b0[o];
+            if (NV > 1) acc[1] += a1[o] * b1[o];
+            if (NV > 2) acc[2] += a2[o] * b2[o];
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < NV; m++) s[m][tid] = acc[m];
+    __syncthreads();
+    sp.sum<NV>(s, k);
+    if constexpr (FIN != FIN_NONE) {
+        block_end<FIN>(s, partials, k, fa);
+    } else if (tid < k) {
+#pragma unroll
+        for (int m = 0; m < NV; m++) partials[((long long)blockIdx.x * k + tid) * 3 + m] = s[m][tid];
+    }
 }
 
 // mode 0: initial residual norm (delta0); mode 1: post-initial-step norm
@@ -171,7 +339,7 @@ void fcg_norm_entry(Context* c, const FcgBufs& f, const double* r, int mode, con
 }
 
 void fcg_norm(Context* c, const FcgBufs& f, const double* v, int mode) {
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, v, v, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
+    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, v, v, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr, FinArgs());
     BCMGX_LAUNCHED();
     k_norm_final<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, mode, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();
@@ -193,7 +361,7 @@ __global__ __launch_bounds__(WG) void k_init_scalars(const double* __restrict__ 
 }
 
 void fcg_init_dots(Context* c, const FcgBufs& f, const double* r, const double* v, const double* w) {
-    k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, v, w, v, nullptr, nullptr, f.partials, nullptr);
+    k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, v, w, v, nullptr, nullptr, f.partials, nullptr, FinArgs());
     BCMGX_LAUNCHED();
     fcg_init_scalars(c, f, f.nblk);
 }
@@ -242,39 +410,13 @@ void fcg_init_update_z32(Context* c, const FcgBufs& f, double* x, double* r, con
     BCMGX_LAUNCHED();
 }
 
-__global__ __launch_bounds__(WG) void k_scalars3(const double* __restrict__ partials, int nblk, int k, FcgState* st,
-                                                 const int* __restrict__ all_done, int phase) {
-    if (*all_done) return;
-    __shared__ double s[3][WG];
-    double tot[3];
-    int c = blockIdx.x;
-    sum_partials<3>(partials, nblk, k, c, tot, s);
-    if (threadIdx.x == 0) {
-        FcgState& S = st[c];
-        if (S.done) return;
-        S.alpha = tot[0];
-        S.beta = tot[1];
-        S.gamma = tot[2];
-        S.theta = S.gamma / S.delta;                        // FCG.cu:132
-        S.delta = S.beta - ((S.gamma * S.gamma) / S.delta);  // FCG.cu:135
-        S.theta2 = S.alpha / S.delta;                       // FCG.cu:136
-        if (phase == 0) {  // the x step of this iteration waits for the pair's second update
-            S.pend = S.theta2;
-            S.pad1 = 1;
-        }
-    }
-}
-
-void fcg_scalars3(Context* c, const FcgBufs& f, int nblk, int phase) {
-    k_scalars3<<<f.k, WG, 0, c->stream>>>(f.partials, nblk, f.k, f.st, f.all_done, phase);
-    BCMGX_LAUNCHED();
-}
+void fcg_scalars3(Context* c, const FcgBufs& f, int nblk, int phase) { fin_launch<FIN_SCALARS>(c, f, nblk, fin_args(f, phase)); }
 
 void fcg_dots3(Context* c, const FcgBufs& f, const double* r, const double* p0, const double* w0, const double* w1, int phase) {
-    k_dots<3><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, p0, w0, p0, w1, p0, f.partials, f.all_done);
+    FinArgs a = fin_args(f, phase);
+    k_dots<3, FIN_SCALARS><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, p0, w0, p0, w1, p0, f.partials, f.all_done, a);
     BCMGX_LAUNCHED();
-    k_scalars3<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done, phase);
-    BCMGX_LAUNCHED();
+    if (!a.tickets) fin_launch<FIN_SCALARS>(c, f, f.nblk, a);
 }
 
 // double_merged_axpy(P1, P0, x, -theta, theta2); double_merged_axpy(W1, W0, r, -theta, -theta2)
@@ -284,12 +426,12 @@ void fcg_dots3(Context* c, const FcgBufs& f, const double* r, const double* p0, 
 // phase 1 forms x = theta2' t' + (pend p1 + x) -- the two steps in the
 // reference's order, so x has the same bits -- and saves one x read and write.
 template <int PHASE>
-__global__ __launch_bounds__(WG) void k_update(int n, int k, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_update(int n, int k, const FcgState* st,
                                                double* __restrict__ p0, const double* __restrict__ p1,
                                                double* __restrict__ w0, const double* __restrict__ w1,
                                                double* __restrict__ x, double* __restrict__ r,
-                                               double* __restrict__ partials, const int* __restrict__ all_done,
-                                               FcgEntry e) {
+                                               double* __restrict__ partials, const int* all_done,
+                                               FcgEntry e, FinArgs fa) {
     if (*all_done) return;
     __shared__ double s[1][WG];
     int tid = threadIdx.x;
@@ -328,24 +470,26 @@ __global__ __launch_bounds__(WG) void k_update(int n, int k, const FcgState* __r
     s[0][tid] = acc;
     __syncthreads();
     sp.sum<1>(s, k);
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
+    block_end<FIN_STEP>(s, partials, k, fa);
 }
 
 void fcg_update(Context* c, const FcgBufs& f, double* p0, const double* p1, double* w0, const double* w1, double* x, double* r,
                 int phase, const FcgEntry& e) {
-    if (phase == 0) k_update<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
-    else k_update<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e);
+    FinArgs a = fin_args(f, phase);
+    if (phase == 0) k_update<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e, a);
+    else k_update<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p0, p1, w0, w1, x, r, f.partials, f.all_done, e, a);
     BCMGX_LAUNCHED();
+    if (!a.tickets) fin_launch<FIN_STEP>(c, f, f.nblk, a);
 }
 
 // k_update with z in FP32 (widened exactly) and p, w updated in place
 template <int PHASE>
-__global__ __launch_bounds__(WG) void k_update_z32(int n, int k, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_update_z32(int n, int k, const FcgState* st,
                                                    const float* __restrict__ z, double* __restrict__ p,
                                                    const double* __restrict__ w0, double* __restrict__ w,
                                                    double* __restrict__ x, double* __restrict__ r,
-                                                   double* __restrict__ partials, const int* __restrict__ all_done,
-                                                   FcgEntry e) {
+                                                   double* __restrict__ partials, const int* all_done,
+                                                   FcgEntry e, FinArgs fa) {
     if (*all_done) return;
     __shared__ double s[1][WG];
     int tid = threadIdx.x;
@@ -384,40 +528,16 @@ __global__ __launch_bounds__(WG) void k_update_z32(int n, int k, const FcgState*
     s[0][tid] = acc;
     __syncthreads();
     sp.sum<1>(s, k);
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
+    block_end<FIN_STEP>(s, partials, k, fa);
 }
 
 void fcg_update_z32(Context* c, const FcgBufs& f, const float* z, double* p, const double* w0, double* w, double* x, double* r,
                     int phase, const FcgEntry& e) {
-    if (phase == 0) k_update_z32<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
-    else k_update_z32<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e);
+    FinArgs a = fin_args(f, phase);
+    if (phase == 0) k_update_z32<0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e, a);
+    else k_update_z32<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, z, p, w0, w, x, r, f.partials, f.all_done, e, a);
     BCMGX_LAUNCHED();
-}
-
-// l2 = ||r||; iter++; stop when !(l2 > rtol*delta0 && iter < itnlim)  (FCG.cu:146-156)
-__global__ __launch_bounds__(WG) void k_finish(const double* __restrict__ partials, int nblk, int k, FcgState* st,
-                                               double rtol, int itnlim, int* all_done, int* ndone, int phase) {
-    if (*all_done) return;
-    __shared__ double s[1][WG];
-    double tot[1];
-    int c = blockIdx.x;
-    sum_partials<1>(partials, nblk, k, c, tot, s);
-    if (threadIdx.x == 0) {
-        FcgState& S = st[c];
-        if (phase == 1) S.pad1 = 0;  // this pair's update added the waiting step
-        if (S.done) return;
-        S.l2 = sqrt(tot[0]);
-        S.iter += 1;
-        if (!(S.l2 > rtol * S.delta0 && S.iter < itnlim)) {
-            S.done = 1;
-            if (atomicAdd(ndone, 1) + 1 == k) *all_done = 1;
-        }
-    }
-}
-
-void fcg_finish_iteration(Context* c, const FcgBufs& f, int phase) {
-    k_finish<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.rtol, f.itnlim, f.all_done, f.all_done + 1, phase);
-    BCMGX_LAUNCHED();
+    if (!a.tickets) fin_launch<FIN_STEP>(c, f, f.nblk, a);
 }
 
 __global__ __launch_bounds__(WG) void k_flush_pending(int n, int k, FcgState* st, const double* __restrict__ t,
@@ -480,26 +600,10 @@ __global__ __launch_bounds__(WG) void k_cg_init(const double* __restrict__ parti
 }
 
 void cg_init(Context* c, const FcgBufs& f, const double* r, int stopcrit) {
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, r, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr);
+    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, r, nullptr, nullptr, nullptr, nullptr, f.partials, nullptr, FinArgs());
     BCMGX_LAUNCHED();
     k_cg_init<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, stopcrit, f.all_done, f.all_done + 1);
     BCMGX_LAUNCHED();
-}
-
-// rho = r.u, beta = rho / rho_prev  (CG_HS.cu:89-101)
-__global__ __launch_bounds__(WG) void k_cg_beta(const double* __restrict__ partials, int nblk, int k, FcgState* st,
-                                                const int* __restrict__ all_done) {
-    if (*all_done) return;
-    __shared__ double s[1][WG];
-    double tot[1];
-    int c = blockIdx.x;
-    sum_partials<1>(partials, nblk, k, c, tot, s);
-    if (threadIdx.x == 0) {
-        FcgState& S = st[c];
-        if (S.done) return;
-        S.alpha = tot[0];
-        S.theta = S.alpha / S.delta;
-    }
 }
 
 // p = 1 u + beta p  (my_axpby, basic.cu:114-130; CG_HS.cu:103-107)
@@ -518,51 +622,32 @@ __global__ __launch_bounds__(WG) void k_cg_direction(int n, int k, const FcgStat
 }
 
 void cg_beta_direction(Context* c, const FcgBufs& f, const double* r, const double* u, double* p) {
-    k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, u, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
+    FinArgs a = fin_args(f);
+    k_dots<1, FIN_BETA><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, r, u, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done, a);
     BCMGX_LAUNCHED();
-    k_cg_beta<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
-    BCMGX_LAUNCHED();
+    if (!a.tickets) fin_launch<FIN_BETA>(c, f, f.nblk, a);
     k_cg_direction<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, u, p, f.all_done);
     BCMGX_LAUNCHED();
 }
 
-// (first iteration: rho = u.r) gamma = p.s, alpha = rho / gamma; rho_prev = rho  (CG_HS.cu:112-129)
-template <int NV>
-__global__ __launch_bounds__(WG) void k_cg_alpha(const double* __restrict__ partials, int nblk, int k, FcgState* st,
-                                                 const int* __restrict__ all_done) {
-    if (*all_done) return;
-    __shared__ double s[NV][WG];
-    double tot[NV];
-    int c = blockIdx.x;
-    sum_partials<NV>(partials, nblk, k, c, tot, s);
-    if (threadIdx.x == 0) {
-        FcgState& S = st[c];
-        if (S.done) return;
-        if (NV == 2) S.alpha = tot[1];
-        S.gamma = tot[0];
-        S.theta2 = S.alpha / S.gamma;
-        S.delta = S.alpha;
-    }
-}
-
 void cg_alpha(Context* c, const FcgBufs& f, const double* p, const double* s, const double* u, const double* r, bool first) {
+    FinArgs a = fin_args(f);
     if (first) {
-        k_dots<2><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, u, r, nullptr, nullptr, f.partials, f.all_done);
+        k_dots<2, FIN_ALPHA0><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, u, r, nullptr, nullptr, f.partials, f.all_done, a);
         BCMGX_LAUNCHED();
-        k_cg_alpha<2><<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
+        if (!a.tickets) fin_launch<FIN_ALPHA0>(c, f, f.nblk, a);
     } else {
-        k_dots<1><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done);
+        k_dots<1, FIN_ALPHA><<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, p, s, nullptr, nullptr, nullptr, nullptr, f.partials, f.all_done, a);
         BCMGX_LAUNCHED();
-        k_cg_alpha<1><<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.all_done);
+        if (!a.tickets) fin_launch<FIN_ALPHA>(c, f, f.nblk, a);
     }
-    BCMGX_LAUNCHED();
 }
 
 // x = alpha p + 1 x; r = -alpha s + 1 r (CG_HS.cu:131-132), with the ||r||^2 partials
-__global__ __launch_bounds__(WG) void k_cg_update(int n, int k, const FcgState* __restrict__ st,
+__global__ __launch_bounds__(WG) void k_cg_update(int n, int k, const FcgState* st,
                                                   const double* __restrict__ p, const double* __restrict__ sv,
                                                   double* __restrict__ x, double* __restrict__ r,
-                                                  double* __restrict__ partials, const int* __restrict__ all_done) {
+                                                  double* __restrict__ partials, const int* all_done, FinArgs fa) {
     if (*all_done) return;
     __shared__ double s[1][WG];
     int tid = threadIdx.x;
@@ -588,41 +673,14 @@ __global__ __launch_bounds__(WG) void k_cg_update(int n, int k, const FcgState* 
     s[0][tid] = acc;
     __syncthreads();
     sp.sum<1>(s, k);
-    if (tid < k) partials[((long long)blockIdx.x * k + tid) * 3] = s[0][tid];
-}
-
-// l2 = ||r||; converged when l2 < rtol delta0, else the iteration count
-// advances and itnlim stops the column (CG_HS.cu:134-163)
-__global__ __launch_bounds__(WG) void k_cg_finish(const double* __restrict__ partials, int nblk, int k, FcgState* st,
-                                                  double rtol, int itnlim, int* all_done, int* ndone) {
-    if (*all_done) return;
-    __shared__ double s[1][WG];
-    double tot[1];
-    int c = blockIdx.x;
-    sum_partials<1>(partials, nblk, k, c, tot, s);
-    if (threadIdx.x == 0) {
-        FcgState& S = st[c];
-        if (S.done) return;
-        S.l2 = sqrt(tot[0]);
-        bool stop = false;
-        if (S.l2 < rtol * S.delta0) {
-            S.pad0 = 1;
-            stop = true;
-        } else if (++S.iter >= itnlim) {
-            stop = true;
-        }
-        if (stop) {
-            S.done = 1;
-            if (atomicAdd(ndone, 1) + 1 == k) *all_done = 1;
-        }
-    }
+    block_end<FIN_CG>(s, partials, k, fa);
 }
 
 void cg_update_finish(Context* c, const FcgBufs& f, const double* p, const double* s, double* x, double* r) {
-    k_cg_update<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p, s, x, r, f.partials, f.all_done);
+    FinArgs a = fin_args(f);
+    k_cg_update<<<f.nblk, WG, 0, c->stream>>>(f.n, f.k, f.st, p, s, x, r, f.partials, f.all_done, a);
     BCMGX_LAUNCHED();
-    k_cg_finish<<<f.k, WG, 0, c->stream>>>(f.partials, f.nblk, f.k, f.st, f.rtol, f.itnlim, f.all_done, f.all_done + 1);
-    BCMGX_LAUNCHED();
+    if (!a.tickets) fin_launch<FIN_CG>(c, f, f.nblk, a);
 }
 
 }  // namespace bcmgx

@@ -170,12 +170,14 @@ void colmajor_to_interleaved(Context* c, const double* s, int ld, double* d, int
                              const int* alt_if = nullptr, double* alt = nullptr);
 void interleaved_to_colmajor(Context* c, const double* s, double* d, int ld, int n, int k, const FcgState* st = nullptr,
                              const double* p = nullptr);
+constexpr int FCG_TICKETS = 16 * 33;
 struct FcgBufs {
     int n = 0, k = 1;
     int nblk = 0;              // partial-sum blocks (fixed for a given n and k)
     double* partials = nullptr;  // nblk * k * 3
     FcgState* st = nullptr;      // k states
     int* all_done = nullptr;     // 1 when every column stopped
+    unsigned* tickets = nullptr;  // FCG_TICKETS words, zero between kernels (null: reductions finish in a kernel of their own)
     double rtol = 1e-6;
     int itnlim = 2000;
 };
@@ -223,11 +225,10 @@ void fcg_dots3(Context* c, const FcgBufs& f, const double* r, const double* p0, 
 // phase: 0 for the first iteration of a pair (its x step waits), 1 for the second
 void fcg_scalars3(Context* c, const FcgBufs& f, int nblk, int phase);
 // double_merged_axpy x2 (FCG.cu:138-144) fused with the ||r||^2 partials.  Phase 0
-// leaves x alone (its step waits in pend); phase 1 adds both steps to x in order.
+// leaves x alone (its step waits in pend); phase 1 adds both steps to x in order.  Then
+// ||r|| -> convergence test and iteration count (FCG.cu:146-156)
 void fcg_update(Context* c, const FcgBufs& f, double* p0, const double* p1, double* w0, const double* w1, double* x, double* r,
                 int phase, const FcgEntry& e = FcgEntry());
-// ||r|| -> convergence test and iteration count (FCG.cu:146-156)
-void fcg_finish_iteration(Context* c, const FcgBufs& f, int phase);
 // the update with the preconditioned residual z in FP32 and the direction p and
 // its image w updated in place: t = z - theta p, u = w0 - theta w; p = t, w = u
 // (the same operations, in the same order, as fcg_update)
