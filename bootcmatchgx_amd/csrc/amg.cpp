@@ -1239,7 +1239,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
         BCMGX_HIP(hipGraphInstantiate(&s.exec, s.graph, nullptr, nullptr, 0));
     }
     int launched = 0;
-    int* hflag = (int*)c->host_scratch(sizeof(int) * 2);
+    int hflag[2];
     while (true) {
         for (int j = 0; j < check; j += 2) {
             if (use_graph) BCMGX_HIP(hipGraphLaunch(s.exec, c->stream));
@@ -1249,8 +1249,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
             }
             launched += 2;
         }
-        BCMGX_HIP(hipMemcpyAsync(hflag, s.flags.get(), sizeof(int) * 2, hipMemcpyDeviceToHost, c->stream));
-        c->sync();
+        c->d2h(hflag, s.flags.get(), 2);
         if (hflag[0]) break;
         if (launched > p.itnlim + 2) break;  // the device stops every column at itnlim
     }
@@ -1348,14 +1347,13 @@ SolveResult cghs_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params
         }
         int check = std::max(1, p.check_every);
         int launched = 1;
-        int* hflag = (int*)c->host_scratch(sizeof(int) * 2);
+        int hflag[2];
         while (launched < p.itnlim) {
             for (int j = 0; j < check && launched < p.itnlim; j++, launched++) {
                 if (use_graph) BCMGX_HIP(hipGraphLaunch(s.cg_exec, c->stream));
                 else iteration();
             }
-            BCMGX_HIP(hipMemcpyAsync(hflag, s.flags.get(), sizeof(int) * 2, hipMemcpyDeviceToHost, c->stream));
-            c->sync();
+            c->d2h(hflag, s.flags.get(), 2);
             if (hflag[0]) break;
         }
     }

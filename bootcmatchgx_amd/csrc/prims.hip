@@ -4,6 +4,8 @@
 // written for wave64 directly.
 #include "kernels.h"
 
+#include <chrono>
+
 #include <algorithm>
 #include <cstdio>
 
@@ -91,6 +93,7 @@ Context::~Context() {
     if (stream) (void)hipStreamSynchronize(stream);
     pool.reset();
     if (pinned) (void)hipHostFree(pinned);
+    if (mail) (void)hipHostFree(mail);
     if (side) (void)hipStreamDestroy(side);
     if (stream) (void)hipStreamDestroy(stream);
 }
@@ -111,12 +114,44 @@ void* Context::host_scratch(size_t bytes) {
     return pinned;
 }
 
+// -------------------------------------------------------------- small reads ---
+// na words from a and nb from b into pinned memory, then the number of this read
+__global__ __launch_bounds__(WG) void k_mail(const unsigned* __restrict__ a, int na, const unsigned* __restrict__ b, int nb,
+                                             unsigned* box, unsigned seq) {
+    for (int w = threadIdx.x; w < na + nb; w += WG)
+        __hip_atomic_store(box + MAIL_HEAD + w, w < na ? a[w] : b[w - na], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(box, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+const unsigned* Context::mail_read(const void* a, size_t na, const void* b, size_t nb) {
+    if (!mail) {
+        BCMGX_HIP(hipHostMalloc(reinterpret_cast<void**>(&mail), (MAIL_HEAD + MAIL_WORDS) * sizeof(unsigned), hipHostMallocDefault));
+        mail[0] = 0;
+    }
+    unsigned seq = ++mail_seq ? mail_seq : ++mail_seq;
+    k_mail<<<1, WG, 0, stream>>>((const unsigned*)a, (int)na, (const unsigned*)b, (int)nb, mail, seq);
+    BCMGX_LAUNCHED();
+    auto t0 = std::chrono::steady_clock::now();
+    for (int poll = 0; __atomic_load_n(mail, __ATOMIC_ACQUIRE) != seq; poll++) {
+        if ((poll & 1023) != 1023 || std::chrono::steady_clock::now() - t0 < std::chrono::microseconds(500)) continue;
+        sync();  // long work ahead of it, or an error: waits, or throws
+        BCMGX_CHECK(__atomic_load_n(mail, __ATOMIC_ACQUIRE) == seq, BCMGX_ERR_HIP, "device read did not arrive");
+    }
+    return mail + MAIL_HEAD;
+}
+
 // ------------------------------------------------------------------ scan ---
-// Three-phase exclusive scan: per-block totals, scan of the totals in one
-// workgroup, then per-block rescan with the block offset.  1024 items per
-// block (256 threads x 4).
+// Exclusive scan: per-block totals, scan of the totals in one workgroup, then
+// per-block rescan with the block offset.  1024 items per block (256 threads x 4).
+// A launch costs 2.4 us of a setup whose levels are small, so to SCAN_FOLD blocks
+// each rescanning block sums the totals before its own itself, and to SCAN_ONE
+// items one workgroup does it all.
 constexpr int SCAN_ITEMS = 4;
 constexpr int SCAN_BLOCK = WG * SCAN_ITEMS;
+constexpr int SCAN_ONE = 4 * SCAN_BLOCK;
+constexpr int SCAN_FOLD = 4 * WG;
 
 template <typename T>
 __device__ T block_exclusive_scan(T v, T* lds_wave, T& total) {
@@ -177,8 +212,42 @@ __global__ __launch_bounds__(WG) void k_scan_single(T* __restrict__ data, long l
 }
 
 template <typename TI, typename T>
+__global__ __launch_bounds__(WG) void k_scan_one(const TI* in, int n, T* out) {
+    __shared__ T lw[4];
+    T carry = 0;
+    for (int base = 0; base < n; base += SCAN_BLOCK) {
+        int b = base + threadIdx.x * SCAN_ITEMS;
+        T v[SCAN_ITEMS];
+        T s = 0;
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) {
+            v[k] = (b + k < n) ? (T)in[b + k] : (T)0;
+            s += v[k];
+        }
+        T tot;
+        T run = carry + block_exclusive_scan<T>(s, lw, tot);
+#pragma unroll
+        for (int k = 0; k < SCAN_ITEMS; k++) {
+            if (b + k < n) out[b + k] = run;
+            run += v[k];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) out[n] = carry;
+}
+
+// FOLD: offs holds the blocks' totals, not their offsets, and out[n] is written here
+template <typename TI, typename T, bool FOLD>
 __global__ __launch_bounds__(WG) void k_scan_final(const TI* __restrict__ in, long long n, const T* __restrict__ offs, T* __restrict__ out) {
     __shared__ T lw[4];
+    T before = 0;
+    if constexpr (FOLD) {
+        T p = 0;
+        for (unsigned b = threadIdx.x; b < blockIdx.x; b += WG) p += offs[b];
+        block_exclusive_scan<T>(p, lw, before);
+    } else {
+        before = offs[blockIdx.x];
+    }
     long long base = (long long)blockIdx.x * SCAN_BLOCK + threadIdx.x * SCAN_ITEMS;
     T v[SCAN_ITEMS];
     T s = 0;
@@ -188,7 +257,8 @@ __global__ __launch_bounds__(WG) void k_scan_final(const TI* __restrict__ in, lo
         s += v[k];
     }
     T tot;
-    T run = offs[blockIdx.x] + block_exclusive_scan<T>(s, lw, tot);
+    T run = before + block_exclusive_scan<T>(s, lw, tot);
+    if (FOLD && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) out[n] = before + tot;
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; k++) {
         if (base + k < n) out[base + k] = run;
@@ -204,13 +274,22 @@ static T scan_impl(Context* c, const TI* in, T* out, long long n, bool read_tota
         fill<T>(c, out, 1, (T)0);
         return 0;
     }
+    if (n <= SCAN_ONE) {
+        k_scan_one<TI, T><<<1, WG, 0, c->stream>>>(in, (int)n, out);
+        BCMGX_LAUNCHED();
+        return read_total ? c->read1(out + n) : (T)0;
+    }
     long long nb = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
     DBuf<T> part(c, nb + 1);
     k_scan_partials<TI, T><<<(unsigned)nb, WG, 0, c->stream>>>(in, n, part.get());
     BCMGX_LAUNCHED();
-    k_scan_single<T><<<1, WG, 0, c->stream>>>(part.get(), nb, out + n);
-    BCMGX_LAUNCHED();
-    k_scan_final<TI, T><<<(unsigned)nb, WG, 0, c->stream>>>(in, n, part.get(), out);
+    if (nb <= SCAN_FOLD) {
+        k_scan_final<TI, T, true><<<(unsigned)nb, WG, 0, c->stream>>>(in, n, part.get(), out);
+    } else {
+        k_scan_single<T><<<1, WG, 0, c->stream>>>(part.get(), nb, out + n);
+        BCMGX_LAUNCHED();
+        k_scan_final<TI, T, false><<<(unsigned)nb, WG, 0, c->stream>>>(in, n, part.get(), out);
+    }
     BCMGX_LAUNCHED();
     return read_total ? c->read1(out + n) : (T)0;
 }
