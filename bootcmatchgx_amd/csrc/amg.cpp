@@ -428,8 +428,10 @@ struct SolveWork {
     int z32_blk_grid = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    hipGraph_t cg_graph = nullptr;  // one CG iteration
+    hipGraph_t cg_graph = nullptr;  // a few CG iterations
     hipGraphExec_t cg_exec = nullptr;
+    int cg_count = 0;   // iterations in it
+    bool used = false;  // solved with before
     int lanesA = 0;
     int chunkA = 0;
     int mv_blocks = 0;  // grid of the fused SpMM + dots kernel (0: not used)
@@ -1159,6 +1161,15 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
     return *sp;
 }
 
+// The iterations are captured and replayed from a workspace's second solve on: its first one, which may be the
+// only one, launches them (capture and instantiation take 0.1 ms, as much as they save a solve; launches
+// queue at 2.4 us each, no slower than a replay goes through them).
+static bool replayed(const bcmgx_params& p, SolveWork& s) {
+    bool again = s.used;
+    s.used = true;
+    return p.use_graph != 0 && again;
+}
+
 SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params& p, const double* b, double* x, int k,
                       const SolveIo* io) {
     BCMGX_CHECK(k >= 1 && k <= 64, BCMGX_ERR_ARG, "nrhs must be in [1, 64]");
@@ -1223,7 +1234,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     }
     // ---- iterations, two at a time (the buffer roles alternate)
     int check = std::max(2, p.check_every + (p.check_every & 1));
-    bool use_graph = p.use_graph != 0;
+    bool use_graph = replayed(p, s);
     if (use_graph && !s.exec) {
         BCMGX_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
         try {
@@ -1331,11 +1342,15 @@ SolveResult cghs_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params
             cg_alpha(c, s.fb, P, S, U, R, false);
             cg_update_finish(c, s.fb, P, S, s.X.get(), R);
         };
-        bool use_graph = p.use_graph != 0;
+        // to 8 of those between two polls in one graph (one a graph: 4 us more each); the device stops every
+        // column at itnlim, and what is queued past it does nothing
+        int check = std::max(1, p.check_every), per = std::min(check, 8);
+        bool use_graph = replayed(p, s);
+        if (use_graph && s.cg_exec && s.cg_count != per) s.drop_graph();
         if (use_graph && !s.cg_exec) {
             BCMGX_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             try {
-                iteration();
+                for (int j = 0; j < per; j++) iteration();
             } catch (...) {
                 hipGraph_t g;
                 (void)hipStreamEndCapture(c->stream, &g);
@@ -1344,12 +1359,12 @@ SolveResult cghs_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params
             }
             BCMGX_HIP(hipStreamEndCapture(c->stream, &s.cg_graph));
             BCMGX_HIP(hipGraphInstantiate(&s.cg_exec, s.cg_graph, nullptr, nullptr, 0));
+            s.cg_count = per;
         }
-        int check = std::max(1, p.check_every);
         int launched = 1;
         int hflag[2];
         while (launched < p.itnlim) {
-            for (int j = 0; j < check && launched < p.itnlim; j++, launched++) {
+            for (int j = 0; j < check && launched < p.itnlim; j += use_graph ? per : 1, launched += use_graph ? per : 1) {
                 if (use_graph) BCMGX_HIP(hipGraphLaunch(s.cg_exec, c->stream));
                 else iteration();
             }
