@@ -280,7 +280,8 @@ __global__ __launch_bounds__(WG) void k_weights(int n, const int* __restrict__ r
 // higher id), with key = 1 + the rank of u among y's neighbours.  key = 0 marks
 // a neighbour u never proposes to: non-positive weight (find_Candidate,
 // suitor.cu:91-94) or no mirrored entry (u is unknown to y); mir holds only
-// the pairs of positive weight.
+// the pairs of positive weight.  y's top bit marks the list's last entry.
+// Entries of one column and weight share a rank and take the places from it on.
 template <int G>
 __global__ __launch_bounds__(WG) void k_pref(int n, const int* __restrict__ Wrow, const int* __restrict__ Wcol,
                                              const int* __restrict__ rank, const int* __restrict__ mir,
@@ -293,15 +294,18 @@ __global__ __launch_bounds__(WG) void k_pref(int n, const int* __restrict__ Wrow
         int y = Wcol[a];
         int q = mir[a];  // u's entry in y's row, -1 when absent or not positive
         int key = (y >= 0 && y < n && q >= 0) ? rank[q] + 1 : 0;
-        pref[e - 1 - rank[a]] = make_int2(y, key);
+        int r = rank[a];
+        for (int b = a; b > s && Wcol[b - 1] == y && rank[b - 1] == rank[a]; b--) r++;
+        pref[e - 1 - r] = make_int2(r == 0 ? y | INT_MIN : y, key);
     }
 }
 
 // lanes per proposing vertex (the candidates one ballot looks at)
 constexpr int SUITOR_LANES = 4;
 
-// Lock-free Suitor.  S[y] = (1 + rank of y's current suitor) << 32 | suitor
-// (0: none).  A vertex proposes to its best neighbour -- positive weight,
+// Lock-free Suitor.  S[y] = (1 + rank of y's current suitor) << 32 | place
+// (0: none), the place being that of the suitor's entry in pref, its top bit set
+// when it is the suitor's last.  A vertex proposes to its best neighbour -- positive weight,
 // heaviest, ties to the higher id (find_Candidate, suitor.cu:80-147) -- that
 // would prefer it to its current suitor; atomicMax installs the offer and
 // returns the displaced suitor, which this thread then re-proposes
@@ -313,100 +317,103 @@ constexpr int SUITOR_LANES = 4;
 // One launch is one round.  Each G-lane group takes a vertex from the round's
 // work list (all vertices in round 0) and follows its proposal chain for at
 // most `maxsteps` proposals; a vertex still unsettled then goes to the next
-// round's list.  Bounding the steps keeps one long displacement chain from
-// serialising a whole launch: every round works on all pending vertices in
-// parallel with fresh offers.
+// round's list, so that one long displacement chain does not serialise a launch
+// whose other vertices wait for a place on the device.  A round of at most
+// `together` vertices, all of them on the device at once, has none waiting and
+// follows every chain to its end.
 //
-// The rounds are bound by the throughput of the device-scope suitor-word
-// reads, so each vertex keeps a cursor into its preference list: pos[v] is the
-// list position of v's last offer.  A neighbour that would not accept v (its
-// suitor word beats v's key there) never will, since suitor words only rise;
-// so v resumes after its cursor and reads only the suitor words of neighbours
-// it has not yet been refused by.  The group reads G list entries and G suitor
-// words at a time and takes the first that would accept (one ballot).  A stale
-// read of a cursor (another XCD's write not yet visible) only lowers it, which
-// costs reads, never a candidate.
+// A neighbour that would not accept v (its suitor word beats v's key there)
+// never will, since suitor words only rise; so v goes on after the place of its
+// last offer and reads only the suitor words of neighbours it has not yet been
+// refused by.  The group reads G list entries and G suitor words at a time and
+// takes the first that would accept (one ballot).
+//
+// Bound by the chains of displacements: on the constant 27-point Laplacian 128^3
+// some 800 proposals one after another, each the list entries, the suitor words
+// and the atomic.  The suitor word read says who will be displaced and where its list
+// goes on, so its next entries are on their way during the atomic and are used
+// when its result agrees: two trips to memory a proposal, where a cursor and a list
+// end kept per vertex made four.  Matchings of that setup 5.43 -> 5.19 ms, and 4.20
+// with the chains followed to their ends: of 33 rounds for the finest one 31 had
+// 46000 pending vertices or fewer, and each spent 40 us on its list's counter.
 template <int G>
-__global__ __launch_bounds__(WG) void k_suitor(int n, const int* __restrict__ Wrow, const int2* __restrict__ pref,
-                                               int* pos, unsigned long long* S, const int* __restrict__ in_list,
+__global__ __launch_bounds__(WG) void k_suitor(int n, int m, const int* __restrict__ Wrow, const int2* __restrict__ pref,
+                                               unsigned long long* S, const int* __restrict__ in_list,
                                                const int* __restrict__ in_count, int* __restrict__ out_list,
-                                               int* __restrict__ out_count, int maxsteps) {
+                                               int* __restrict__ out_count, int maxsteps, int together) {
     static_assert(G <= 32, "group mask");
     int lane = (int)threadIdx.x % G;
     int gbase = ((int)threadIdx.x & 63) - lane;  // the group's first lane in its wave
     int ngroups = gridDim.x * (WG / G);
     int total = in_list ? *in_count : n;
+    if (total <= together) maxsteps = INT_MAX;
+    auto bits = [&](bool v) { return (__ballot(v) >> gbase) & ((1ull << G) - 1); };
+    auto entries = [&](int p) { return p >= 0 && p + lane < m ? pref[p + lane] : make_int2(INT_MIN, 0); };
     for (int it = (blockIdx.x * WG + (int)threadIdx.x) / G; it < total; it += ngroups) {
         // round 0 visits the vertices from the highest id down: a suitee prefers
         // the higher suitor, so offers made in this order are rarely displaced
-        int cur = in_list ? in_list[it] : n - 1 - it;
-        int p = in_list ? pos[cur] + 1 : Wrow[cur];  // next list position to try
-        int e = Wrow[cur + 1];
-        int steps = 0;
-        while (cur >= 0) {  // uniform inside the group
+        int p;  // the next list place to try (-1: none is left)
+        if (in_list) {
+            p = in_list[it];
+        } else {
+            int v = n - 1 - it;
+            p = Wrow[v];
+            if (p == Wrow[v + 1]) p = -1;
+        }
+        int ahead = -1;  // the place whose entries were read ahead
+        int2 read = make_int2(INT_MIN, 0);
+        for (int steps = 0; p >= 0; steps++) {  // uniform inside the group
             if (steps == maxsteps) {
-                if (lane == 0) {
-                    pos[cur] = p - 1;
-                    out_list[atomicAdd(out_count, 1)] = cur;
-                }
+                if (lane == 0) out_list[atomicAdd(out_count, 1)] = p;
                 break;
             }
-            steps++;
-            int best = -1, bkey = 0, bidx = -1;
-            for (; p < e; p += G) {  // G candidates at a time, best first
-                int2 pk = make_int2(-1, 0);
-                if (p + lane < e) pk = pref[p + lane];
+            int best = -1, bkey = 0;
+            unsigned place = 0;
+            unsigned long long cur = 0;
+            int2 pk = p == ahead ? read : entries(p);
+            while (true) {  // G candidates at a time, best first
+                unsigned long long ends = bits(pk.x < 0);
+                int y = pk.x & INT_MAX;
                 bool ok = false;
-                // (the range test only matters for rows with repeated columns,
-                // which leave slots of the list unwritten)
-                if (pk.y > 0 && (unsigned)pk.x < (unsigned)n) {
-                    unsigned long long sy = __hip_atomic_load(&S[pk.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                unsigned long long sy = 0;
+                // entries past the list's last are another vertex's
+                if ((ends & ((1ull << lane) - 1)) == 0 && pk.y > 0 && y < n) {
+                    sy = __hip_atomic_load(&S[y], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     ok = (int)(sy >> 32) < pk.y;
                 }
-                unsigned long long m = (__ballot(ok) >> gbase) & ((1ull << G) - 1);
-                if (m) {
-                    int f = __ffsll(m) - 1;
-                    best = __shfl(pk.x, f, G);
+                unsigned long long accept = bits(ok);
+                if (accept) {
+                    int f = __ffsll(accept) - 1;
+                    int x = __shfl(pk.x, f, G);
+                    best = x & INT_MAX;
                     bkey = __shfl(pk.y, f, G);
-                    bidx = p + f;
+                    place = (unsigned)(p + f) | (x < 0 ? 0x80000000u : 0u);
+                    cur = __shfl(sy, f, G);
                     break;
                 }
+                if (ends) break;
+                p += G;
+                pk = entries(p);
             }
-            if (best < 0) break;  // no neighbour left that would accept cur
-            unsigned olo = 0, ohi = 0;
-            if (lane == 0) {
-                pos[cur] = bidx;
-                unsigned long long offer = ((unsigned long long)(unsigned)bkey << 32) | (unsigned)cur;
-                unsigned long long old = atomicMax(&S[best], offer);
-                olo = (unsigned)old;
-                ohi = (unsigned)(old >> 32);
-            }
-            olo = __shfl(olo, 0, G);
-            ohi = __shfl(ohi, 0, G);
-            if ((int)ohi < bkey) {  // installed; the displaced suitor (if any) resumes after its cursor
-                cur = ohi > 0 ? (int)olo : -1;
-                if (cur >= 0) {
-                    p = pos[cur] + 1;
-                    e = Wrow[cur + 1];
-                }
-            } else {
-                p = bidx + 1;  // refused: a better offer holds that neighbour
-            }
+            if (best < 0) break;  // no neighbour left that would accept the vertex
+            auto after = [](unsigned place) { return (int)place < 0 ? -1 : (int)place + 1; };
+            ahead = cur ? after((unsigned)cur) : -1;
+            read = entries(ahead);
+            unsigned long long old = 0;
+            if (lane == 0) old = atomicMax(&S[best], (unsigned long long)(unsigned)bkey << 32 | place);
+            old = __shfl(old, 0, G);
+            if ((int)(old >> 32) < bkey) p = old ? after((unsigned)old) : -1;  // installed; the displaced suitor (if any) goes on
+            else p = after(place);  // refused: a better offer holds that neighbour
         }
     }
 }
-
-// cursors before round 0: every list is untried
-__global__ void k_pos_init(int n, const int* __restrict__ Wrow, int* __restrict__ pos) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < n) pos[v] = Wrow[v] - 1;
-}
-
-__global__ void k_suitor_decode(int n, const unsigned long long* __restrict__ S, int* __restrict__ M) {
+// a suitor's rank in y's row is also its place in y's list, from the end
+__global__ void k_suitor_decode(int n, const unsigned long long* __restrict__ S, const int* __restrict__ Wrow,
+                                const int2* __restrict__ pref, int* __restrict__ M) {
     int y = blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= n) return;
-    unsigned long long s = S[y];
-    M[y] = (s >> 32) ? (int)(unsigned)s : -1;
+    int key = (int)(S[y] >> 32);
+    M[y] = key ? pref[Wrow[y + 1] - key].x & INT_MAX : -1;
 }
 
 
@@ -420,35 +427,31 @@ __global__ void k_make_wrow(int n, const int* __restrict__ row, int* __restrict_
     if (i <= n) Wrow[i] = row[i] - i;
 }
 
-// Rounds of k_suitor until no vertex is pending.  The list length is read
-// back every few rounds (an empty round costs one tiny launch).
+// Rounds of k_suitor until no vertex is pending: one while all n vertices fit the device
+// together, mostly two otherwise (2097152 vertices of the 27-point 128^3: 46000 pending after the first).
 template <int G>
-static void suitor_rounds(Context* c, int n, const int* Wrow, const int2* pref, int* pos, unsigned long long* S) {
-    // proposals per vertex per launch: short while most vertices are pending
-    // (the launch is throughput-bound), longer once only chains remain (each
-    // launch is then latency-bound and fewer launches finish them sooner)
+static void suitor_rounds(Context* c, int n, int m, const int* Wrow, const int2* pref, unsigned long long* S) {
+    // proposals per vertex of a round that does not fit: short while most vertices are pending
     auto maxsteps_of = [](int round) { return round < 8 ? 8 : round < 16 ? 16 : round < 24 ? 32 : 64; };
-    // round r counts its pending vertices in cnt[r % RING]: a ring of counters
-    // cleared together every RING rounds, not one clear per round
-    constexpr int RING = 64;
-    DBuf<int> la(c, n), lb(c, n), cnt(c, RING);
-    fill<int>(c, cnt.get(), RING, 0);
     unsigned grid = (unsigned)std::min<long long>(grid_for(n, WG / G), (long long)c->num_cus * 16);
-    k_suitor<G><<<grid, WG, 0, c->stream>>>(n, Wrow, pref, pos, S, nullptr, nullptr, la.get(), cnt.get(),
-                                             maxsteps_of(0));
-    BCMGX_LAUNCHED();
-    int* lists[2] = {la.get(), lb.get()};
-    int cur = 0;
-    for (int round = 1;; round++) {
-        // lists[cur] holds the pending vertices, counted in cnt[(round - 1) % RING]
-        if (round % RING == 0) fill<int>(c, cnt.get(), RING - 1, 0);  // every counter but this round's input
-        const int* in_cnt = cnt.get() + (round - 1) % RING;
-        int* out_cnt = cnt.get() + round % RING;
-        k_suitor<G><<<grid, WG, 0, c->stream>>>(n, Wrow, pref, pos, S, lists[cur], in_cnt, lists[cur ^ 1],
-                                                 out_cnt, maxsteps_of(round));
+    int together = c->num_cus * (2048 / G);  // 2048 threads a CU
+    if (n <= together) {
+        k_suitor<G><<<grid, WG, 0, c->stream>>>(n, m, Wrow, pref, S, nullptr, nullptr, nullptr, nullptr, 0, together);
         BCMGX_LAUNCHED();
-        cur ^= 1;
-        if (round % 8 == 0 && c->read1(out_cnt) == 0) break;
+        return;
+    }
+    DBuf<int> la(c, n), lb(c, n), cnt(c, 2);
+    int* lists[2] = {la.get(), lb.get()};
+    fill<int>(c, cnt.get(), 2, 0);
+    k_suitor<G><<<grid, WG, 0, c->stream>>>(n, m, Wrow, pref, S, nullptr, nullptr, lists[0], cnt.get(), maxsteps_of(0), together);
+    BCMGX_LAUNCHED();
+    for (int round = 1, cur = 0;; round++, cur ^= 1) {
+        // lists[cur] holds the pending vertices' next places, counted in cnt[cur]
+        if (round > 1) fill<int>(c, cnt.get() + (cur ^ 1), 1, 0);
+        k_suitor<G><<<grid, WG, 0, c->stream>>>(n, m, Wrow, pref, S, lists[cur], cnt.get() + cur, lists[cur ^ 1],
+                                                 cnt.get() + (cur ^ 1), maxsteps_of(round), together);
+        BCMGX_LAUNCHED();
+        if (c->read1(cnt.get() + (cur ^ 1)) == 0) break;
         // every round settles at least one proposal; offers are bounded by the edge count
         BCMGX_CHECK(round < 4 * n + 1024, BCMGX_ERR_NUMERIC, "matching did not settle");
     }
@@ -506,13 +509,8 @@ void suitor_match(Context* c, const DCsr& A, const double* w, int* M, const int*
 #undef BCMGX_W
     BCMGX_LAUNCHED();
     DBuf<int2> pref(c, mm);
-    DBuf<int> pos(c, n);
     DBuf<long long> S(c, n);
     fill<long long>(c, S.get(), n, 0);
-    // the cursors start below every list: a read that misses a later write
-    // (not yet visible across XCDs) still sees a valid lower bound
-    k_pos_init<<<grid_for(n, WG), WG, 0, c->stream>>>(n, Wrow.get(), pos.get());
-    BCMGX_LAUNCHED();
 #define BCMGX_MT(LL)                                                                                                   \
     case LL:                                                                                                           \
         k_pref<LL><<<grid_for(n, WG / LL), WG, 0, c->stream>>>(n, Wrow.get(), Wcol.get(), rank.get(), mir.get(),       \
@@ -527,12 +525,12 @@ void suitor_match(Context* c, const DCsr& A, const double* w, int* M, const int*
     // keep more proposal chains in flight per wave
     int LS = std::min(L, SUITOR_LANES);
     switch (LS) {
-    case 2: suitor_rounds<2>(c, n, Wrow.get(), pref.get(), pos.get(), Su); break;
-    case 4: suitor_rounds<4>(c, n, Wrow.get(), pref.get(), pos.get(), Su); break;
-    case 8: suitor_rounds<8>(c, n, Wrow.get(), pref.get(), pos.get(), Su); break;
-    default: suitor_rounds<16>(c, n, Wrow.get(), pref.get(), pos.get(), Su); break;
+    case 2: suitor_rounds<2>(c, n, (int)m, Wrow.get(), pref.get(), Su); break;
+    case 4: suitor_rounds<4>(c, n, (int)m, Wrow.get(), pref.get(), Su); break;
+    case 8: suitor_rounds<8>(c, n, (int)m, Wrow.get(), pref.get(), Su); break;
+    default: suitor_rounds<16>(c, n, (int)m, Wrow.get(), pref.get(), Su); break;
     }
-    k_suitor_decode<<<grid_for(n, WG), WG, 0, c->stream>>>(n, Su, M);
+    k_suitor_decode<<<grid_for(n, WG), WG, 0, c->stream>>>(n, Su, Wrow.get(), pref.get(), M);
     BCMGX_LAUNCHED();
 }
 
