@@ -359,24 +359,44 @@ static void build_hierarchy(Context* c, const DCsr& A0, const bcmgx_params& p, H
     H.avg_cratio = nlv > 1 ? avc / (nlv - 1) : 1;
 }
 
-// A_l P_l of every level above the coarsest, values in FP32 only: with them the
-// first post-smoothing sweep forms f - A (x + P e) as r_pre - (A P) e
-static void make_level_product(Context* c, Hierarchy& H, int l) {
+// A_l P_l of every level above the coarsest, values in the cycle's precision only:
+// with them the first post-smoothing sweep forms f - A (x + P e) as r_pre - (A P) e
+static void make_level_product(Context* c, Hierarchy& H, int l, bool f32) {
     Level& lv = *H.L[l];
     const DCsr& A = lv.mat();
     DCsr P;
     prolongator_csr(c, A.n, H.L[l + 1]->mat().n, lv.agg.get(), lv.pval.get(), P);
     spgemm(c, A, P, lv.AP);
-    lv.AP.valf.reset(c, std::max(lv.AP.nnz, 1));
-    convert<double, float>(c, lv.AP.val.get(), lv.AP.valf.get(), lv.AP.nnz);
-    lv.AP.val.release();
+    if (f32) {
+        lv.AP.valf.reset(c, std::max(lv.AP.nnz, 1));
+        convert<double, float>(c, lv.AP.val.get(), lv.AP.valf.get(), lv.AP.nnz);
+        lv.AP.val.release();
+    }
     lv.lanesAP = transfer_lanes(lv.AP);
 }
 // The same product queued with no host synchronisation (false when A_l's rows
 // are too long for it); level_product_lengths reads the lengths afterwards
-static bool level_product_async(Context* c, Hierarchy& H, int l) {
+static bool level_product_async(Context* c, Hierarchy& H, int l, bool f32) {
     Level& lv = *H.L[l];
-    return unit_product_f32_async(c, lv.mat(), H.L[l + 1]->mat().n, lv.agg.get(), lv.pval.get(), lv.AP);
+    return unit_product_async(c, lv.mat(), H.L[l + 1]->mat().n, lv.agg.get(), lv.pval.get(), lv.AP, f32);
+}
+// Whether a level keeps A P.  FP64 cycles do on large levels, where the post sweep is bound by memory and
+// reads 12 bytes an entry of A: 27-point 128^3 133 us from A, 64 from A P, and level 1's last
+// sweep no longer prolongs (30 -> 10 us); below some 4 M entries (20 us) the product costs the setup more than a solve gets back.
+static bool keeps_product(const bcmgx_params& p, const DCsr& A, bool f32) {
+    return p.post_galerkin && (f32 || A.nnz >= 4000000);
+}
+// f(), which forms a level's product; an FP64 cycle does without it where there is no memory for it (false)
+template <typename F>
+static bool product_or_none(Level& lv, bool f32, F&& f) {
+    try {
+        f();
+        return true;
+    } catch (const Error& e) {
+        if (f32 || e.code != BCMGX_ERR_ALLOC) throw;
+        lv.AP = DCsr();
+        return false;
+    }
 }
 static void level_product_lengths(Context* c, const std::vector<Level*>& lvs) {
     if (lvs.empty()) return;
@@ -487,7 +507,15 @@ void Prec::ensure_work(int k) {
             nl = std::max(nl, hrc(h).levels());
             ncoarse = std::max(ncoarse, hrc(h).L.back()->mat().n);
         }
-        if (coarse_sweeps_fit(ncoarse, p.relaxnumber_coarse)) coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse, k);
+        if (coarse_sweeps_fit(ncoarse, p.relaxnumber_coarse)) {
+            try {
+                coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse, k);
+            } catch (const Error& e) {  // no memory for k columns' slots: their sweeps are launched one by one
+                if (k == 1 || e.code != BCMGX_ERR_ALLOC) throw;
+                coarse = CoarseSync();
+                coarse.reserve(ctx, ncoarse, p.relaxnumber_coarse, 1);
+            }
+        }
         std::vector<size_t> lsz(nl, 1);
         for (int h = 0; h < n_hrc(); h++)
             for (int l = 0; l < hrc(h).levels(); l++) lsz[l] = std::max(lsz[l], (size_t)hrc(h).L[l]->mat().n);
@@ -704,9 +732,9 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
     }
     V* xc = nullptr;
     int post = p.postrelax_sweeps * coeff;
-    // from A P in FP32: the prolongation and the first post-smoothing sweep in one pass,
+    // from A P: the prolongation and the first post-smoothing sweep in one pass,
     // f - A (x + P e) = (f - A x) - (A P) e, the first term still in w.Res
-    bool from_ap = std::is_same<V, float>::value && post >= 1 && lv.AP.valf;
+    bool from_ap = post >= 1 && mat_val<V>(lv.AP);
     // else, for one column, the coarser level's last sweep prolongs its result by the
     // rows of R (every fine row is in one of them) and x is corrected without a pass of
     // its own; into the other buffer, since the coarsest level's kernel may do it twice
@@ -724,27 +752,25 @@ static V* gamg_cycle(CycleRun<V>& R, int l, const V* F, V* Xin, bool first_sweep
             if (last) break;
         }
     }
-    if constexpr (std::is_same<V, float>::value) {
-        if (xc && from_ap) {
-            V* y = post == 1 && outv ? outv : oth;
-            SpmvArgs a;
-            a.n = lv.AP.n; a.row = lv.AP.row.get(); a.col = lv.AP.col.get(); a.val = lv.AP.valf.get();
-            a.nnz = lv.AP.nnz; a.x = xc; a.y = y; a.b = w.Res.get(); a.D = lvl_M<V>(lv); a.k = k;
-            a.lanes = lv.lanesAP; a.stop = R.stop;
-            bool wide = k == 1 && post == 1 && out64;  // one column: widened in the same pass
-            if (wide) a.y64 = out64;
-            galerkin_post_sweep<V>(c, a, lv.agg.get(), lvl_pval<V>(lv), cur);
-            if (wide) return nullptr;
-            if (post == 1) {
-                if (!out64) return y;
-                convert_stop<V, double>(c, y, out64, (long long)A.n * k, R.stop);  // the result widened
-                return nullptr;
-            }
-            cur = y;
-            oth = (cur == w.X.get()) ? w.X2.get() : w.X.get();
-            return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, post - 1, false, k, R.stop, lv.chunkA,
-                                    out64, outv, up);
+    if (xc && from_ap) {
+        V* y = post == 1 && outv ? outv : oth;
+        SpmvArgs a;
+        a.n = lv.AP.n; a.row = lv.AP.row.get(); a.col = lv.AP.col.get(); a.val = mat_val<V>(lv.AP);
+        a.nnz = lv.AP.nnz; a.x = xc; a.y = y; a.b = w.Res.get(); a.D = lvl_M<V>(lv); a.k = k;
+        a.lanes = lv.lanesAP; a.stop = R.stop;
+        bool wide = k == 1 && post == 1 && out64;  // one column: widened in the same pass
+        if (wide) a.y64 = out64;
+        galerkin_post_sweep<V>(c, a, lv.agg.get(), lvl_pval<V>(lv), cur);
+        if (wide) return nullptr;
+        if (post == 1) {
+            if (!out64) return y;
+            convert_stop<V, double>(c, y, out64, (long long)A.n * k, R.stop);  // the result widened
+            return nullptr;
         }
+        cur = y;
+        oth = (cur == w.X.get()) ? w.X2.get() : w.X.get();
+        return jacobi_sweeps<V>(c, A, lv.lanesA, lvl_M<V>(lv), F, cur, oth, post - 1, false, k, R.stop, lv.chunkA, out64, outv,
+                                up);
     }
     if (corr.done) std::swap(cur, oth);
     else if (xc) prolong_add<V>(c, A.n, k, lv.agg.get(), lvl_pval<V>(lv), xc, cur, R.stop);
@@ -760,7 +786,19 @@ void Prec::refresh_level0() {
             Level& l0 = *hrc(h).L[0];
             abs_row_sum(ctx, A->n, A->row.get(), A->val.get(), l0.M.get());
             if (l0.Mf) convert<double, float>(ctx, l0.M.get(), l0.Mf.get(), A->n);
-            if (l0.AP.valf) make_level_product(ctx, hrc(h), 0);  // A P with the new values of A
+            // A P with the new values of A (its pattern, so its length and lanes, stays)
+            bool f32 = (bool)l0.AP.valf;
+            int nnz = l0.AP.nnz;
+            if (!l0.AP.row) continue;
+            bool kept = product_or_none(l0, f32, [&] {
+                if (level_product_async(ctx, hrc(h), 0, f32)) {
+                    l0.AP.nnz = nnz;
+                } else {
+                    make_level_product(ctx, hrc(h), 0, f32);
+                    drop_graphs();  // they hold the old product's addresses
+                }
+            });
+            if (!kept) drop_graphs();
         }
     }
 }
@@ -988,22 +1026,20 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
             async_product.assign(64, 0);
             Hierarchy* hp = &H;
             return [&, hp](int l) {  // runs on the side queue
-                if (!f32) return;
-                level_fp32_copy(c, *hp->L[l]);
-                if (p.post_galerkin && l + 1 < hp->levels() && l < (int)async_product.size())
-                    async_product[l] = level_product_async(c, *hp, l) ? 1 : 0;
+                if (f32) level_fp32_copy(c, *hp->L[l]);
+                if (l + 1 < hp->levels() && l < (int)async_product.size() && keeps_product(p, hp->L[l]->mat(), f32))
+                    product_or_none(*hp->L[l], f32, [&] { async_product[l] = level_product_async(c, *hp, l, f32) ? 1 : 0; });
             };
         };
         auto finish = [&](Hierarchy& H) {
             side.join();
-            if (f32 && p.post_galerkin) {
-                std::vector<Level*> queued;
-                for (int l = 0; l + 1 < H.levels(); l++) {
-                    if (l < (int)async_product.size() && async_product[l]) queued.push_back(H.L[l].get());
-                    else make_level_product(c, H, l);
-                }
-                level_product_lengths(c, queued);
+            std::vector<Level*> queued;
+            for (int l = 0; l + 1 < H.levels(); l++) {
+                if (!keeps_product(p, H.L[l]->mat(), f32)) continue;
+                if (l < (int)async_product.size() && async_product[l]) queued.push_back(H.L[l].get());
+                else product_or_none(*H.L[l], f32, [&] { make_level_product(c, H, l, f32); });
             }
+            level_product_lengths(c, queued);
             for (auto& lp : H.L) {
                 Level& l = *lp;
                 const DCsr& M = l.mat();

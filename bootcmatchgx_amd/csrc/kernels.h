@@ -299,9 +299,9 @@ void csr_shape(Context* c, DCsr& A);
 // dind (nc ints, when given)
 bool galerkin(Context* c, const DCsr& A, int nc, const int* agg, const double* pval, const DCsr& R, DCsr& C, int rmax = -1,
               int* dind = nullptr);
-// A P with FP32 values for the prolongator (agg, pval) onto nc columns, queued with no host
-// synchronisation (C.nnz = -1: the length is at C.row[n]); false when A's rows are too long
-bool unit_product_f32_async(Context* c, const DCsr& A, int nc, const int* agg, const double* pval, DCsr& C);
+// A P, its values FP32 (valf) or FP64 (val), for the prolongator (agg, pval) onto nc columns, queued with no
+// host synchronisation (C.nnz = -1: the length is at C.row[n]); false when A's rows are too long
+bool unit_product_async(Context* c, const DCsr& A, int nc, const int* agg, const double* pval, DCsr& C, bool f32);
 // P <- P P_i for one-entry-per-row operators: agg[k] = agg_i[agg[k]], pval[k] *= pval_i[agg[k]]
 void compose_prolongators(Context* c, int n, int* agg, double* pval, const int* agg_i, const double* pval_i);
 // csr of a one-entry-per-row prolongator (row = identity)

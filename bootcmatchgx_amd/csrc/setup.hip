@@ -1422,12 +1422,13 @@ void spgemm(Context* c, const DCsr& A, const DCsr& B, DCsr& C) {
 }
 
 // A P for the prolongator (agg, pval) of A's n rows onto nc, when every row of A
-// fits the one-launch product: row pointers, columns and values rounded to FP32
-// (C.valf; no FP64 values) queued on c's stream with no host synchronisation.
+// fits the one-launch product: row pointers, columns and values (rounded to
+// FP32 in C.valf alone with f32, else C.val) queued on c's stream with no host
+// synchronisation.
 // The result's length stays on the device at C.row[n] (C.nnz = -1 until read);
 // the columns and values are sized for A's entries.  False (nothing queued)
 // when A does not fit.
-bool unit_product_f32_async(Context* c, const DCsr& A, int nc, const int* agg, const double* pval, DCsr& C) {
+bool unit_product_async(Context* c, const DCsr& A, int nc, const int* agg, const double* pval, DCsr& C, bool f32) {
     int n = A.n;
     if (n <= 0 || !unit_product_fits(A, nc)) return false;
     size_t tsz = (size_t)std::max(A.nnz, 1);
@@ -1439,13 +1440,23 @@ bool unit_product_f32_async(Context* c, const DCsr& A, int nc, const int* agg, c
     C.nnz = -1;
     C.unit_rows = false;
     C.maxrow = -1;
-    C.row.reset(c, (size_t)n + 1);
+    // buffers of the right size (a product formed again) stay: captured iterations hold their addresses
+    auto room = [&](auto& b, size_t len) {
+        if (b.size() != len) b.reset(c, len);
+    };
+    room(C.row, (size_t)n + 1);
     scan_exclusive_async(c, uniq.get(), C.row.get(), n);
-    C.col.reset(c, tsz);
-    C.val.release();
-    C.valf.reset(c, tsz);
-    k_spgemm_compact<int, float><<<grid_for(n, WG / 16), WG, 0, c->stream>>>(n, A.row.get(), C.row.get(), tcol.get(),
-                                                                           tval.get(), C.col.get(), C.valf.get(), nullptr);
+    room(C.col, tsz);
+    if (f32) {
+        C.val.release();
+        room(C.valf, tsz);
+        k_spgemm_compact<int, float><<<grid_for(n, WG / 16), WG, 0, c->stream>>>(n, A.row.get(), C.row.get(), tcol.get(), tval.get(),
+                                                                               C.col.get(), C.valf.get(), nullptr);
+    } else {
+        room(C.val, tsz);
+        k_spgemm_compact<int, double><<<grid_for(n, WG / 16), WG, 0, c->stream>>>(n, A.row.get(), C.row.get(), tcol.get(), tval.get(),
+                                                                                C.col.get(), C.val.get(), nullptr);
+    }
     BCMGX_LAUNCHED();
     return true;
 }
