@@ -11,10 +11,11 @@
 // through the L1 once per tile and distinct column (9.3 per row on the 27-point
 // grid, not 27), and nothing is transposed.
 //
-// Whole calls, transposed columns and this: 27-point 128^3, k = 32: 1210 and 727 us
-// (memory 374 us), k = 8: 527 and 281, k = 2: 963 and 182; 7-point 128^3, k = 32: 838
-// and 565; 27-point 10^3, any k: 27 and 16.  Bound by the latency of a step (load,
-// barrier, 27 dependent sums): 8 columns a step, with 3 waves a SIMD where 4 columns
+// Whole calls, transposed columns and this: 27-point 128^3, k = 32: 1210 and 695 us
+// (memory 374 us), k = 8: 527 and 270, k = 2: 963 and 177; 7-point 128^3, k = 32: 838
+// and 563; 27-point 10^3, any k: 27 and 16.  Bound by the latency of a step (load,
+// barrier, 27 dependent sums; a test of the row length per 4 entries, not 8, 727): 8 columns
+// a step, with 3 waves a SIMD where 4 columns
 // have 4, gave 912 us; loads under branches, waited for one by one, 1547.
 //
 // Each column's sum runs over the row in order, product and sum rounded apart, as in
@@ -119,7 +120,7 @@ __global__ __launch_bounds__(WG, cm_waves_simd(E)) void k_spmm_cm(int n, int k, 
         for (int q = 0; q < CW; q++) t[q] = 0.0;
 #pragma unroll
         for (int j = 0; j < E; j += 4) {
-            if (!__any(j < len)) break;
+            if (j % 8 == 0 && !__any(j < len)) break;
             unsigned p01 = l2[j / 2], p23 = l2[j / 2 + 1];
             asm("" : "+v"(p01), "+v"(p23));  // unpacked here: E addresses kept over the columns would spill
             const double* x0 = xs + (p01 & 0xffffu);
