@@ -478,7 +478,17 @@ void Prec::drop_graphs() {
     for (auto& s : solves) s->drop_graph();
 }
 
+// work whose allocation fails is not there: nothing of it is taken for complete by the next call
 void Prec::ensure_work(int k) {
+    try {
+        allocate_work(k);
+    } catch (...) {
+        kcap = 0;
+        throw;
+    }
+}
+
+void Prec::allocate_work(int k) {
     if (ptype == BCMGX_PREC_BCMG && k > 1 && k != tuned_k) {
         // SpMM column chunk for this batch width (tuned outside any graph capture)
         bool f32 = p.precision == BCMGX_PRECISION_FP32;
@@ -1168,8 +1178,8 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
     for (auto& w : prec->solves)
         if (w->k == k && w->n == n) sp = w.get();
     if (!sp) {
-        prec->solves.emplace_back(new SolveWork());
-        sp = prec->solves.back().get();
+        std::unique_ptr<SolveWork> made(new SolveWork());  // kept once it is whole
+        sp = made.get();
         SolveWork& s = *sp;
         s.k = k;
         s.n = n;
@@ -1193,6 +1203,7 @@ static SolveWork& solve_work(Context* c, const DCsr& A, Prec* prec, const bcmgx_
         s.fb.all_done = s.flags.get();
         s.lanesA = p.autotune ? tune_lanes(c, A, false) : default_lanes(A.nnz, A.n);
         s.chunkA = p.autotune ? tune_chunk(c, A, false, k) : k;
+        prec->solves.push_back(std::move(made));
     }
     return *sp;
 }
@@ -1232,10 +1243,10 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     int* xzero = s.flags.get() + 2;  // the initial guess holds only zeros (set while staging it)
     if (io) {
         fill<int>(c, xzero, 1, 1);
-        colmajor_to_interleaved(c, io->x, io->ld, s.X.get(), n, k, xzero);
+        colmajor_to_interleaved(c, io->x, io->ld, s.X.get(), n, k, xzero, nullptr, nullptr, io->have);
         // a zero guess: every row sum of A x is +0, so r = b - A x is b itself
         // and b goes straight to r
-        colmajor_to_interleaved(c, io->b, io->ld, s.B.get(), n, k, nullptr, xzero, s.r.get());
+        colmajor_to_interleaved(c, io->b, io->ld, s.B.get(), n, k, nullptr, xzero, s.r.get(), io->have);
     } else {
         copy_d2d(c, s.B.get(), b, sizeof(double) * nk);
         copy_d2d(c, s.X.get(), x, sizeof(double) * nk);
@@ -1304,7 +1315,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
     // and its direction is still in v (the first iteration's p0), or in d with z in FP32
     const double* pw = s.z32 ? s.d.get() : s.v.get();
     if (io) {  // the flush rides on the way out
-        interleaved_to_colmajor(c, s.X.get(), io->x, io->ld, n, k, s.fb.st, pw);
+        interleaved_to_colmajor(c, s.X.get(), io->x, io->ld, n, k, s.fb.st, pw, io->have);
         fcg_clear_pending(c, s.fb);
     } else {
         fcg_flush_pending(c, s.fb, pw, s.X.get());

@@ -73,6 +73,7 @@ struct Prec {
 
     ~Prec();
     void ensure_work(int k);
+    void allocate_work(int k);
     void drop_graphs();
     // u <- B r for k interleaved columns; `x_zero`: u holds zeros on entry (the FCG case).
     // `entry_ready`: the level-0 entry of the cycle (see fused_entry) already holds the
@@ -112,6 +113,7 @@ struct SolveIo {
     const double* b = nullptr;
     double* x = nullptr;
     int ld = 0;
+    int have = -1;  // their columns (-1: all of the solve's); the solve's others are zero
 };
 // with io, b and x are ignored and the blocks come from io
 SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params& p, const double* b, double* x, int k,

@@ -55,7 +55,31 @@ static int record(bcmgx_context_s* ctx, int code, const char* msg) {
 
 // copy an n x k block (column-major, leading dimension ld; host or device)
 // into a device buffer with k interleaved columns
-static void stage_in(Context* c, const double* src, int ld, int mem, int n, int k, double* dst_interleaved, DBuf<double>& tmp) {
+// The columns a k-column solve or application runs with: past k zero ones, up to a width that the
+// k-column kernels take as 16-byte vectors (multiples of 4 in FP32, of 2 in FP64); a column of zeros is done
+// at once.  FP32 cycle, 27-point 64^3: 31 columns 19.7 ms alone and 11.4 as 32, 13 as 16 10.9 and 8.2, 9 as 12
+// 9.7 and 8.2, 5 as 8 6.7 and 6.4; 7-point 90^3, 31: 56.8 and 32.7.  FP64, 7-point 90^3, 31: 59.4 and 42.6, 9 as 10
+// 23.3 and 19.9; CG with l1-Jacobi, 9: 75.6 and 69.1, but 7 as 8 47.1 and 54.3, so from 9 columns on.
+static int run_columns(const Prec& P, int k) {
+    bool f32 = P.ptype == BCMGX_PREC_BCMG && P.p.precision == BCMGX_PRECISION_FP32;
+    if (f32) return k >= 5 ? (k + 3) / 4 * 4 : k;
+    return k >= 9 ? (k + 1) / 2 * 2 : k;
+}
+// run(w), with w = k where there is no memory for the wider block
+template <typename F>
+static void run_padded(const Prec& P, int k, F&& run) {
+    int w = run_columns(P, k);
+    try {
+        run(w);
+    } catch (const Error& e) {
+        if (w == k || e.code != BCMGX_ERR_ALLOC) throw;
+        run(k);
+    }
+}
+
+// w: the interleaved block's columns (0: k; more: the others are zero)
+static void stage_in(Context* c, const double* src, int ld, int mem, int n, int k, double* dst_interleaved, DBuf<double>& tmp,
+                     int w = 0) {
     size_t nk = (size_t)n * k;
     if (k == 1) {
         if (mem == BCMGX_MEM_HOST) BCMGX_HIP(hipMemcpyAsync(dst_interleaved, src, nk * 8, hipMemcpyHostToDevice, c->stream));
@@ -68,9 +92,10 @@ static void stage_in(Context* c, const double* src, int ld, int mem, int n, int 
         BCMGX_HIP(hipMemcpyAsync(tmp.get(), src, (size_t)ld * k * 8, hipMemcpyHostToDevice, c->stream));
         dsrc = tmp.get();
     }
-    colmajor_to_interleaved(c, dsrc, ld, dst_interleaved, n, k);
+    colmajor_to_interleaved(c, dsrc, ld, dst_interleaved, n, w ? w : k, nullptr, nullptr, nullptr, k);
 }
-static void stage_out(Context* c, const double* src_interleaved, double* dst, int ld, int mem, int n, int k, DBuf<double>& tmp) {
+static void stage_out(Context* c, const double* src_interleaved, double* dst, int ld, int mem, int n, int k, DBuf<double>& tmp,
+                      int w = 0) {
     size_t nk = (size_t)n * k;
     if (k == 1) {
         if (mem == BCMGX_MEM_HOST) {
@@ -84,11 +109,11 @@ static void stage_out(Context* c, const double* src_interleaved, double* dst, in
         if (ld > n) {  // keep the caller's padding rows: fetch them first
             BCMGX_HIP(hipMemcpyAsync(tmp.get(), dst, (size_t)ld * k * 8, hipMemcpyHostToDevice, c->stream));
         }
-        interleaved_to_colmajor(c, src_interleaved, tmp.get(), ld, n, k);
+        interleaved_to_colmajor(c, src_interleaved, tmp.get(), ld, n, w ? w : k, nullptr, nullptr, k);
         BCMGX_HIP(hipMemcpyAsync(dst, tmp.get(), (size_t)ld * k * 8, hipMemcpyDeviceToHost, c->stream));
         c->sync();
     } else {
-        interleaved_to_colmajor(c, src_interleaved, dst, ld, n, k);
+        interleaved_to_colmajor(c, src_interleaved, dst, ld, n, w ? w : k, nullptr, nullptr, k);
     }
 }
 
@@ -357,12 +382,14 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
     BCMGX_HIP(hipSetDevice(c->device));
     int n = prec->A->A.n;
     if (ld < n) ld = n;
-    size_t nk = (size_t)n * nrhs;
-    DBuf<double> R(c, std::max<size_t>(nk, 1)), U(c, std::max<size_t>(nk, 1)), tmp;
-    stage_in(c, r, ld, mem, n, nrhs, R.get(), tmp);
-    stage_in(c, u, ld, mem, n, nrhs, U.get(), tmp);
-    prec->P->apply(R.get(), U.get(), nrhs, false, nullptr);
-    stage_out(c, U.get(), u, ld, mem, n, nrhs, tmp);
+    run_padded(*prec->P, nrhs, [&](int w) {
+        size_t nk = std::max<size_t>((size_t)n * w, 1);
+        DBuf<double> R(c, nk), U(c, nk), tmp;
+        stage_in(c, r, ld, mem, n, nrhs, R.get(), tmp, w);
+        stage_in(c, u, ld, mem, n, nrhs, U.get(), tmp, w);
+        prec->P->apply(R.get(), U.get(), w, false, nullptr);
+        stage_out(c, U.get(), u, ld, mem, n, nrhs, tmp, w);
+    });
     c->sync();
     return BCMGX_OK;
     API_END(prec->ctx)
@@ -511,17 +538,29 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
         io.b = b;
         io.x = x;
         io.ld = ld;
-        r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, nrhs, &io);
+        io.have = nrhs;
+        run_padded(*P, nrhs, [&](int w) { r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, w, &io); });
+    } else if (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS) {
+        run_padded(*P, nrhs, [&](int w) {
+            size_t nk = (size_t)std::max(n, 1) * w;
+            DBuf<double> B(c, nk), X(c, nk), tmp;
+            stage_in(c, b, ld, mem, n, nrhs, B.get(), tmp, w);
+            stage_in(c, x, ld, mem, n, nrhs, X.get(), tmp, w);
+            r = p->solver == BCMGX_SOLVER_CGHS ? cghs_solve(c, A->A, P, *p, B.get(), X.get(), w)
+                                               : fcg_solve(c, A->A, P, *p, B.get(), X.get(), w);
+            stage_out(c, X.get(), x, ld, mem, n, nrhs, tmp, w);
+        });
     } else {
         size_t nk = (size_t)std::max(n, 1) * nrhs;
         DBuf<double> B(c, nk), X(c, nk), tmp;
         stage_in(c, b, ld, mem, n, nrhs, B.get(), tmp);
         stage_in(c, x, ld, mem, n, nrhs, X.get(), tmp);
-        r = p->solver == BCMGX_SOLVER_CGHS  ? cghs_solve(c, A->A, P, *p, B.get(), X.get(), nrhs)
-            : p->solver != BCMGX_SOLVER_FCG ? cgs_solve(c, A->A, P, *p, B.get(), X.get(), nrhs)
-                                            : fcg_solve(c, A->A, P, *p, B.get(), X.get(), nrhs);
+        r = cgs_solve(c, A->A, P, *p, B.get(), X.get(), nrhs);
         stage_out(c, X.get(), x, ld, mem, n, nrhs, tmp);
     }
+    for (auto* v : {&P->last_exit, &P->last_rel})  // the caller's columns
+        if ((int)v->size() > nrhs) v->resize(nrhs);
+    if ((int)P->last_niter.size() > nrhs) P->last_niter.resize(nrhs);
     c->sync();
     if (out) {
         out->retv = r.retv;

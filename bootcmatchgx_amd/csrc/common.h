@@ -181,8 +181,8 @@ template <typename T>
 void DBuf<T>::reset(Context* c, size_t n) {
     release();
     ctx_ = c;
-    n_ = n;
     p_ = n ? c->dalloc<T>(n) : nullptr;
+    n_ = n;  // (0 when the allocation throws)
 }
 template <typename T>
 void DBuf<T>::release() {

@@ -166,10 +166,11 @@ struct FcgState {
 // zero_flag (may be null) is cleared when the block holds a nonzero; the block
 // goes to alt instead of d when alt_if (may be null) is set and nonzero; st/p
 // (may be null) add the waiting FCG x step (pad1, pend) of each column on the way out.
+// The column-major side has the first `have` columns (-1: all k); the others come in as zeros.
 void colmajor_to_interleaved(Context* c, const double* s, int ld, double* d, int n, int k, int* zero_flag = nullptr,
-                             const int* alt_if = nullptr, double* alt = nullptr);
+                             const int* alt_if = nullptr, double* alt = nullptr, int have = -1);
 void interleaved_to_colmajor(Context* c, const double* s, double* d, int ld, int n, int k, const FcgState* st = nullptr,
-                             const double* p = nullptr);
+                             const double* p = nullptr, int have = -1);
 constexpr int FCG_TICKETS = 16 * 33;
 struct FcgBufs {
     int n = 0, k = 1;

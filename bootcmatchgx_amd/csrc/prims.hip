@@ -417,10 +417,11 @@ static int tile_rows(int k) { return std::max(1, TILE_ELEMS / k); }
 static size_t tile_bytes(int k) { return (size_t)tile_rows(k) * (k + 1) * sizeof(double); }
 
 // zero_flag (may be null) is cleared when any element read is nonzero; the
-// block goes to alt instead of d when alt_if is set and nonzero
+// block goes to alt instead of d when alt_if is set and nonzero; s has the first
+// `have` columns, the others are zeros
 __global__ __launch_bounds__(WG) void k_cm_to_rm(const double* __restrict__ s, int ld, double* __restrict__ d, int n,
-                                                 int k, int TR, int* __restrict__ zero_flag, const int* __restrict__ alt_if,
-                                                 double* __restrict__ alt) {
+                                                 int k, int have, int TR, int* __restrict__ zero_flag,
+                                                 const int* __restrict__ alt_if, double* __restrict__ alt) {
     extern __shared__ double tile[];
     if (alt_if && *alt_if) d = alt;
     long long i0 = (long long)blockIdx.x * TR;
@@ -429,7 +430,7 @@ __global__ __launch_bounds__(WG) void k_cm_to_rm(const double* __restrict__ s, i
     for (int idx = threadIdx.x; idx < TR * k; idx += WG) {
         int r = idx % TR, c = idx / TR;
         if (r < rows) {
-            double v = s[(long long)c * ld + i0 + r];
+            double v = c < have ? s[(long long)c * ld + i0 + r] : 0.0;
             nz |= v != 0.0;
             tile[r * (k + 1) + c] = v;
         }
@@ -442,9 +443,10 @@ __global__ __launch_bounds__(WG) void k_cm_to_rm(const double* __restrict__ s, i
     }
 }
 
-// st/p (may be null): columns whose FCG step waits (pad1) get x + pend * p on the way out
+// st/p (may be null): columns whose FCG step waits (pad1) get x + pend * p on the way out; d
+// takes the first `have` columns
 __global__ __launch_bounds__(WG) void k_rm_to_cm(const double* __restrict__ s, double* __restrict__ d, int ld, int n,
-                                                 int k, int TR, const FcgState* __restrict__ st,
+                                                 int k, int have, int TR, const FcgState* __restrict__ st,
                                                  const double* __restrict__ p) {
     extern __shared__ double tile[];
     __shared__ double pend[64];
@@ -466,24 +468,24 @@ __global__ __launch_bounds__(WG) void k_rm_to_cm(const double* __restrict__ s, d
     __syncthreads();
     for (int idx = threadIdx.x; idx < TR * k; idx += WG) {
         int r = idx % TR, c = idx / TR;
-        if (r < rows) d[(long long)c * ld + i0 + r] = tile[r * (k + 1) + c];
+        if (r < rows && c < have) d[(long long)c * ld + i0 + r] = tile[r * (k + 1) + c];
     }
 }
 
 void colmajor_to_interleaved(Context* c, const double* s, int ld, double* d, int n, int k, int* zero_flag,
-                             const int* alt_if, double* alt) {
+                             const int* alt_if, double* alt, int have) {
     if ((long long)n * k == 0) return;
     int TR = tile_rows(k);
-    k_cm_to_rm<<<(unsigned)((n + TR - 1) / TR), WG, tile_bytes(k), c->stream>>>(s, ld, d, n, k, TR, zero_flag, alt_if,
-                                                                                  alt);
+    k_cm_to_rm<<<(unsigned)((n + TR - 1) / TR), WG, tile_bytes(k), c->stream>>>(s, ld, d, n, k, have < 0 ? k : have, TR,
+                                                                                zero_flag, alt_if, alt);
     BCMGX_LAUNCHED();
 }
 void interleaved_to_colmajor(Context* c, const double* s, double* d, int ld, int n, int k, const FcgState* st,
-                             const double* p) {
+                             const double* p, int have) {
     if ((long long)n * k == 0) return;
     BCMGX_CHECK(k <= 64, BCMGX_ERR_ARG, "at most 64 columns");
     int TR = tile_rows(k);
-    k_rm_to_cm<<<(unsigned)((n + TR - 1) / TR), WG, tile_bytes(k), c->stream>>>(s, d, ld, n, k, TR, st, p);
+    k_rm_to_cm<<<(unsigned)((n + TR - 1) / TR), WG, tile_bytes(k), c->stream>>>(s, d, ld, n, k, have < 0 ? k : have, TR, st, p);
     BCMGX_LAUNCHED();
 }
 

@@ -986,7 +986,10 @@ static void launchk(Context* c, const SpmvArgs& a) {
     }
     for (int c0 = 0; c0 < a.k; c0 += kc) {
         int w = a.k - c0 < kc ? a.k - c0 : kc;
-        int KP = 2;
+        // lanes a row, and as many gathers in flight for each: at least 4 on rows of over 12 entries (two
+        // columns of 27-point 64^3: CG with l1-Jacobi 34.7 ms with 2, 14.0 with 4, 14.9 with 8; 7-point 90^3 23.1,
+        // 24.0 and 31.4)
+        int KP = a.nnz > 12ll * a.n ? 4 : 2;
         while (KP < w) KP <<= 1;
 #define BCMGX_K(KK)                                                                                              \
     case KK:                                                                                                     \
