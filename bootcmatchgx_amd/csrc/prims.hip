@@ -127,7 +127,7 @@ __global__ __launch_bounds__(WG) void k_mail(const unsigned* __restrict__ a, int
 
 const unsigned* Context::mail_read(const void* a, size_t na, const void* b, size_t nb) {
     if (!mail) {
-        BCMGX_HIP(hipHostMalloc(reinterpret_cast<void**>(&mail), (MAIL_HEAD + MAIL_WORDS) * sizeof(unsigned), hipHostMallocDefault));
+        BCMGX_HIP(hipHostMalloc(reinterpret_cast<void**>(&mail), (MAIL_HEAD + MAIL_WORDS) * sizeof(unsigned), hipHostMallocCoherent));
         mail[0] = 0;
     }
     unsigned seq = ++mail_seq ? mail_seq : ++mail_seq;

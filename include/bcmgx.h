@@ -85,7 +85,8 @@ typedef struct bcmgx_params {
     /* ---- extension keys (no counterpart in the reference) ---- */
     int max_coarse_size;    /* "max_coarse_size": 0 = reference formula (int)(40*cbrt(N)) */
     int precision;          /* "precision": FP64 (default) or FP32 hierarchy + V-cycle */
-    int use_graph;          /* "use_graph": capture the FCG iteration in a hipGraph (default 1) */
+    int use_graph;          /* "use_graph": from the second solve of a preconditioner and column count on, replay
+                               the FCG or CG iterations from a hipGraph (default 1) */
     int autotune;           /* "autotune": pick SpMV/SpMM lanes-per-row by timing (default 1) */
     int check_every;        /* "check_every": FCG iterations between host convergence polls (default 8) */
     int fcg_z32;            /* "fcg_z32": with an FP32 hierarchy, FCG keeps the cycle's result z in FP32 and
