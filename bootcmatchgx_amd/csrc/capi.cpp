@@ -382,6 +382,12 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
     BCMGX_HIP(hipSetDevice(c->device));
     int n = prec->A->A.n;
     if (ld < n) ld = n;
+    // one device column is applied where it is: three copies less, 4-5 us each in a call of some 100 us
+    if (nrhs == 1 && mem != BCMGX_MEM_HOST && on_device(c, r) && on_device(c, u) && apart(r, n, u, n)) {
+        prec->P->apply(r, u, 1, false, nullptr);
+        c->sync();
+        return BCMGX_OK;
+    }
     run_padded(*prec->P, nrhs, [&](int w) {
         size_t nk = std::max<size_t>((size_t)n * w, 1);
         DBuf<double> R(c, nk), U(c, nk), tmp;
@@ -540,6 +546,9 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
         io.ld = ld;
         io.have = nrhs;
         run_padded(*P, nrhs, [&](int w) { r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, w, &io); });
+    } else if (nrhs == 1 && mem != BCMGX_MEM_HOST && (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS)) {
+        // one device column: copied into the solver's own buffers and back by the solver
+        r = p->solver == BCMGX_SOLVER_CGHS ? cghs_solve(c, A->A, P, *p, b, x, 1) : fcg_solve(c, A->A, P, *p, b, x, 1);
     } else if (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS) {
         run_padded(*P, nrhs, [&](int w) {
             size_t nk = (size_t)std::max(n, 1) * w;
