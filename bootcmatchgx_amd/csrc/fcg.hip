@@ -7,8 +7,8 @@
 // replayed from a hipGraph and the host only polls a flag.
 //
 // Reductions are deterministic: a fixed number of partial blocks (a function
-// of n and k only), a fixed in-block tree, then one block per column summing the
-// partials in a fixed tree.  k vectors are interleaved (x[i*k + c]); every
+// of n and k only), a fixed in-block tree, then one block per column (or the
+// workgroup that finishes last, few partials) summing them in a fixed tree.  k vectors are interleaved (x[i*k + c]); every
 // column has its own scalars and stop flag.
 #include "kernels.h"
 
