@@ -145,11 +145,12 @@ __global__ void k_blk_counts(int nt, const int* __restrict__ ucnt, int* __restri
     blocks[t] = (g + 15) / 16;
 }
 
-// per tile: its columns 16 groups at a time (the tail repeats the last column) and its masks
+// per tile: its columns 16 groups at a time (the tail repeats the last column) and its masks; twice
+// counts the entries whose column the row has already listed
 __global__ __launch_bounds__(64) void k_blk_masks(int n, const int* __restrict__ rows, const int* __restrict__ row, int stride, const int* __restrict__ ucnt,
                                                   const int* __restrict__ list, const unsigned short* __restrict__ upos,
                                                   const int* __restrict__ gptr, const int* __restrict__ bptr,
-                                                  int* __restrict__ bcol, u64* __restrict__ bmask) {
+                                                  int* __restrict__ bcol, u64* __restrict__ bmask, int* __restrict__ twice) {
     __shared__ u64 mask[BLK_MAX_ENTRIES / 4];
     int t = blockIdx.x, lane = threadIdx.x;
     int U = ucnt[t], G = (U + 3) / 4, NB = (G + 15) / 16;
@@ -164,7 +165,8 @@ __global__ __launch_bounds__(64) void k_blk_masks(int n, const int* __restrict__
         int r = rows[t * BT + q];
         for (int j = row[r] + lane % 16; j < row[r + 1]; j += 16) {
             int u = upos[j];
-            atomicOr(&mask[u >> 2], 1ull << ((u & 3) * 16 + q));
+            u64 bit = 1ull << ((u & 3) * 16 + q);
+            if (atomicOr(&mask[u >> 2], bit) & bit) atomicAdd(twice, 1);
         }
     }
     blk_sync();
@@ -238,9 +240,17 @@ static bool form_blocks(Context* c, DCsr& A, const int* order, double min_reuse)
     }
     DBuf<int> bcol(c, (size_t)(nb + 1) * 64);
     DBuf<u64> mask(c, (size_t)ng + 16);
+    DBuf<int> twice(c, 1);
+    fill<int>(c, twice.get(), 1, 0);
     k_blk_masks<<<nt, 64, 0, c->stream>>>(A.n, rows.get(), A.row.get(), stride, ucnt.get(), list.get(), upos.get(), gptr.get(), bptr.get(),
-                                          bcol.get(), mask.get());
+                                          bcol.get(), mask.get(), twice.get());
     BCMGX_LAUNCHED();
+    // a block has one place per row and column: a matrix that lists a column twice in a row, which
+    // the CSR products add up, stays with them
+    if (c->read1(twice.get()) != 0) {
+        A.blk.refused = true;
+        return false;
+    }
     A.blk.rows = std::move(rows);
     A.blk.vptr = std::move(vptr);
     A.blk.gptr = std::move(gptr);

@@ -231,7 +231,7 @@ struct BlockForm {
     DBuf<double> val64;
     int m = 0;                      // columns of the matrix
     long long groups = 0;
-    bool refused = false;           // the pattern shares too few columns
+    bool refused = false;           // the pattern shares too few columns, or repeats some in a row
     bool built() const { return (bool)mask; }
 };
 

@@ -320,7 +320,7 @@ constexpr int BLK_CODE = -64;
 inline bool blk_width(int k) { return k == 8 || k == 16 || k == 32 || k == 64; }
 constexpr double BLK_MIN_REUSE = 1.5;  // entries per x row loaded below which the form is not used
 // A's block form over tiles of 16 rows taken from order (a permutation of the rows, on the device);
-// false (nothing kept) where rows are too long or share too few columns
+// false (nothing kept) where rows are too long, share too few columns or list a column twice
 bool build_blocks(Context* c, DCsr& A, const int* order, double min_reuse = BLK_MIN_REUSE);
 // the values in block order, on first need; false: no memory for them
 bool block_values32(Context* c, DCsr& A);
