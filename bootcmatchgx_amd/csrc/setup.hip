@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <climits>
+#include <cmath>
 
 namespace bcmgx {
 
@@ -158,7 +159,11 @@ __global__ void k_make_C(int n, const double* __restrict__ val, const int* __res
 // with -1 beforehand: other entries keep it).
 //
 // Preference ranks.  Vertex i orders its neighbours c by (W(i,c), c) -- the
-// Suitor tie rule "heavier, then higher id" (suitor.cu:108,115,136-140).
+// Suitor tie rule "heavier, then higher id" (suitor.cu:108,115,136-140) -- and
+// the entries of one column and weight by their place.  A NaN weight is -inf,
+// below every other (log of a positive number is never -inf).  The order is
+// total whatever the values, so a row's ranks are a permutation and its list
+// has no slot unwritten.
 // rank[e] = position of entry e of row i in that order (0: the least liked).
 // A row of at most L off-diagonal entries keeps one entry per lane, staged in
 // LDS, where the group reads every entry of the row by broadcast; a longer row
@@ -171,7 +176,8 @@ __device__ __forceinline__ double ah_of(double a, double wt, double norm) {
 
 __device__ __forceinline__ double weight_of(double v) {
     double s = fabs(v);
-    return log(s != 0.0 ? s : SUITOR_EPS / (0.999 * DBL_EPSILON));
+    double l = log(s != 0.0 ? s : SUITOR_EPS / (0.999 * DBL_EPSILON));
+    return l == l ? l : -HUGE_VAL;
 }
 
 __device__ __forceinline__ int lower_bound_dev(const int* a, int len, int key) {
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(WG) void k_weights(int n, const int* __restrict__ r
             for (int b = 0; b < len; b++) {
                 double wb = sw[gb + b];
                 int cb = sc[gb + b];
-                r += (wb < wa || (wb == wa && cb < ca)) ? 1 : 0;
+                r += (wb < wa || (wb == wa && (cb < ca || (cb == ca && b < lane)))) ? 1 : 0;
             }
             rank[si + lane] = r;
         }
@@ -269,7 +275,8 @@ __global__ __launch_bounds__(WG) void k_weights(int n, const int* __restrict__ r
         int r = 0;
         for (int b = si; b < si + len; b++) {
             double wb = W[b];
-            r += (wb < wv || (wb == wv && Wcol[b] < cw)) ? 1 : 0;
+            int cb = Wcol[b];
+            r += (wb < wv || (wb == wv && (cb < cw || (cb == cw && b < a)))) ? 1 : 0;
         }
         rank[a] = r;
     }
@@ -281,7 +288,6 @@ __global__ __launch_bounds__(WG) void k_weights(int n, const int* __restrict__ r
 // a neighbour u never proposes to: non-positive weight (find_Candidate,
 // suitor.cu:91-94) or no mirrored entry (u is unknown to y); mir holds only
 // the pairs of positive weight.  y's top bit marks the list's last entry.
-// Entries of one column and weight share a rank and take the places from it on.
 template <int G>
 __global__ __launch_bounds__(WG) void k_pref(int n, const int* __restrict__ Wrow, const int* __restrict__ Wcol,
                                              const int* __restrict__ rank, const int* __restrict__ mir,
@@ -295,7 +301,6 @@ __global__ __launch_bounds__(WG) void k_pref(int n, const int* __restrict__ Wrow
         int q = mir[a];  // u's entry in y's row, -1 when absent or not positive
         int key = (y >= 0 && y < n && q >= 0) ? rank[q] + 1 : 0;
         int r = rank[a];
-        for (int b = a; b > s && Wcol[b - 1] == y && rank[b - 1] == rank[a]; b--) r++;
         pref[e - 1 - r] = make_int2(r == 0 ? y | INT_MIN : y, key);
     }
 }
@@ -413,7 +418,7 @@ __global__ void k_suitor_decode(int n, const unsigned long long* __restrict__ S,
     int y = blockIdx.x * blockDim.x + threadIdx.x;
     if (y >= n) return;
     int key = (int)(S[y] >> 32);
-    M[y] = key ? pref[Wrow[y + 1] - key].x & INT_MAX : -1;
+    M[y] = key > 0 && key <= Wrow[y + 1] - Wrow[y] ? pref[Wrow[y + 1] - key].x & INT_MAX : -1;
 }
 
 
