@@ -69,6 +69,17 @@ struct RowPart {
     }
 };
 
+// Thread 0 of a workgroup that has passed its waits: 0, or for the last of them 1, or 2 when
+// one gave up.  A workgroup's word of that (ctl[2]) is stored by its own thread 0, so the fence
+// here has it visible before the ticket is counted, and no such store is left to land
+// after the last workgroup has cleared the word.
+__device__ __forceinline__ int coarse_ticket(unsigned* ctl, unsigned workgroups) {
+    __threadfence();
+    if (atomicAdd(ctl + 1, 1u) != workgroups - 1) return 0;
+    __threadfence();
+    return __hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 2 : 1;
+}
+
 // The exchanging kernel: a workgroup owns CO_ROWS rows, L lanes each.  An
 // iterate's element travels as two 64-bit words, each half of the double with a
 // 32-bit tag beside it, written and read with device scope: a reader that finds
@@ -173,17 +184,17 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
                 if ((poll & 15) == 15) {
                     if (poll == 15) t0 = wall_clock64();
                     else if (wall_clock64() - t0 > patience) late = true;
-                    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) late = true;
+                    if (__hip_atomic_load(&s_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == s + 1 ||
+                        __hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                        late = true;
                 }
             }
-            if (late) {
-                s_late = s + 1;
-                __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            if (late) __hip_atomic_store(&s_late, s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         __syncthreads();  // the other half of xs is written before the next one
         if (s_late == s + 1) {  // not a faster wave's of the next sweep
             given_up = true;
+            if (tid == 0) __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
         }
         if (listed) {
@@ -205,14 +216,11 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
         else if (lane == 0) out[r] = (V)xr;
     }
     __syncthreads();
-    if (tid == 0) {
-        __threadfence();
-        s_last = atomicAdd(ctl + 1, 1u) == gridDim.x - 1;
-    }
+    if (tid == 0) s_last = coarse_ticket(ctl, gridDim.x);
     __syncthreads();
     if (!s_last) return;
     // the last workgroup: every other one has passed its waits for good
-    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+    if (s_last == 2) {
         double* cur = scratch;
         double* nxt = scratch + n;
         for (int i = tid; i < n; i += T) cur[i] = first(i);
@@ -467,17 +475,17 @@ __global__ __launch_bounds__(CO_ROWS * CO_COLS, E > 32 ? 2 : E > 16 ? 3 : 4) voi
                 if ((poll & 15) == 15) {
                     if (poll == 15) t0 = wall_clock64();
                     else if (wall_clock64() - t0 > patience) late = true;
-                    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) late = true;
+                    if (__hip_atomic_load(&s_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == s + 1 ||
+                        __hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                        late = true;
                 }
             }
-            if (late) {
-                s_late = s + 1;
-                __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            if (late) __hip_atomic_store(&s_late, s + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
         __syncthreads();
         if (s_late == s + 1) {
             given_up = true;
+            if (tid == 0) __hip_atomic_store(ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             break;
         }
         if (listed) {
@@ -505,14 +513,11 @@ __global__ __launch_bounds__(CO_ROWS * CO_COLS, E > 32 ? 2 : E > 16 ? 3 : 4) voi
     }
     if (!given_up && on && act) out[(size_t)r * k + c] = (V)xr;
     __syncthreads();
-    if (tid == 0) {
-        __threadfence();
-        s_last = atomicAdd(ctl + 1, 1u) == gridDim.x * gridDim.y - 1;
-    }
+    if (tid == 0) s_last = coarse_ticket(ctl, gridDim.x * gridDim.y);
     __syncthreads();
     if (!s_last) return;
     // the last workgroup: every other one has passed its waits for good
-    if (__hip_atomic_load(ctl + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+    if (s_last == 2) {
         for (int q = 0; q < k; q++) {
             double* cur = scratch;
             double* nxt = scratch + n;
