@@ -15,6 +15,7 @@
 #include "amg.h"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <functional>
@@ -800,15 +801,23 @@ void Prec::refresh_level0() {
             bool f32 = (bool)l0.AP.valf;
             int nnz = l0.AP.nnz;
             if (!l0.AP.row) continue;
-            bool kept = product_or_none(l0, f32, [&] {
-                if (level_product_async(ctx, hrc(h), 0, f32)) {
-                    l0.AP.nnz = nnz;
-                } else {
-                    make_level_product(ctx, hrc(h), 0, f32);
-                    drop_graphs();  // they hold the old product's addresses
-                }
-            });
-            if (!kept) drop_graphs();
+            auto buffers = [&] {
+                return std::array<const void*, 4>{l0.AP.row.get(), l0.AP.col.get(), l0.AP.val.get(), l0.AP.valf.get()};
+            };
+            auto before = buffers();
+            try {
+                product_or_none(l0, f32, [&] {
+                    if (level_product_async(ctx, hrc(h), 0, f32)) l0.AP.nnz = nnz;
+                    else make_level_product(ctx, hrc(h), 0, f32);
+                });
+            } catch (...) {  // not the old values' product with the new matrix
+                l0.AP = DCsr();
+                drop_graphs();
+                throw;
+            }
+            // captured iterations hold the old product's addresses: it may be gone, or (formed with the other
+            // product's buffers at setup, where there was no memory for this one's) in buffers of another size
+            if (buffers() != before) drop_graphs();
         }
     }
 }

@@ -656,6 +656,15 @@ int bcmgx_internal_coarse_patience(bcmgx_context ctx, long long ticks) {
     return BCMGX_OK;
 }
 
+// Not part of the public interface: the device allocation after the next `after` on this context
+// fails (negative: none); *count, when given, is the number of them so far.
+int bcmgx_internal_fail_allocation(bcmgx_context ctx, long long after, long long* count) {
+    if (!ctx) return BCMGX_ERR_ARG;
+    ctx->c->pool->fail_after(after);
+    if (count) *count = ctx->c->pool->allocations();
+    return BCMGX_OK;
+}
+
 // Not part of the public interface: one product of the block form (blocked.hip) over tiles of
 // 16 rows in `order`, on host arrays of k interleaved columns.  op 1: y = A x, 2: y = b - A x (b
 // FP32), 3: the Jacobi sweep with D, 4: b in FP64 and y = b - A x, all FP32; 5: y = A x in FP64 with

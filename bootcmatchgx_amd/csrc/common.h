@@ -63,6 +63,9 @@ public:
     // until the first stream has been made to wait for it (release_deferred()).
     void set_defer(bool d) { defer_ = d; }
     void release_deferred();
+    // the allocation after the next n fails, as one that finds no memory does (negative: none)
+    void fail_after(long long n) { fail_after_ = n; }
+    long long allocations() const { return count_; }
 
 private:
     static size_t size_class(size_t b);
@@ -72,6 +75,7 @@ private:
     std::multimap<size_t, void*> free_;
     std::map<void*, size_t> live_;
     size_t in_use_ = 0;
+    long long count_ = 0, fail_after_ = -1;
 };
 
 struct Context;

@@ -27,6 +27,8 @@ size_t DevicePool::size_class(size_t b) {
 
 void* DevicePool::alloc(size_t bytes) {
     size_t c = size_class(bytes);
+    count_++;
+    if (fail_after_ >= 0 && fail_after_-- == 0) throw Error(BCMGX_ERR_ALLOC, "allocation failed as asked for");
     auto it = free_.find(c);
     void* p = nullptr;
     if (it != free_.end()) {
