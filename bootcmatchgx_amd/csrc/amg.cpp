@@ -489,13 +489,23 @@ void Prec::ensure_work(int k) {
     }
 }
 
+void Prec::go_lean() {
+    lean = true;
+    solves.clear();
+    wd.clear();
+    wf.clear();
+    for (auto* b : {&cd_F, &cd_X, &cd_X2, &tmp, &tmp2, &tmp3}) b->release();
+    coarse = CoarseSync();
+    kcap = tuned_k = 0;
+}
+
 void Prec::allocate_work(int k) {
     if (ptype == BCMGX_PREC_BCMG && k > 1 && k != tuned_k) {
         // SpMM column chunk for this batch width (tuned outside any graph capture)
         bool f32 = p.precision == BCMGX_PRECISION_FP32;
         // the caller's matrix in block form (its pattern once, kept with the matrix) for the FP32
         // cycle's products with it: rows of 6 entries and more, which can share columns
-        if (f32 && p.autotune && blk_width(k) && A->n >= 65536 && (long long)A->nnz >= 6ll * A->n) {
+        if (f32 && p.autotune && !lean && blk_width(k) && A->n >= 65536 && (long long)A->nnz >= 6ll * A->n) {
             DCsr& M = const_cast<DCsr&>(*A);
             const Level& l0 = *H.L[0];
             // tiles of rows that aggregate together share the most columns

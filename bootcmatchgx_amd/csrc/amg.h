@@ -74,6 +74,11 @@ struct Prec {
     ~Prec();
     void ensure_work(int k);
     void allocate_work(int k);
+    // set where a call found no memory for what it can do without: columns beside the caller's, the
+    // matrix's block form
+    bool lean = false;
+    // gives the first up, with every buffer that the next call allocates again (nothing is queued any more)
+    void go_lean();
     void drop_graphs();
     // u <- B r for k interleaved columns; `x_zero`: u holds zeros on entry (the FCG case).
     // `entry_ready`: the level-0 entry of the cycle (see fused_entry) already holds the

@@ -275,6 +275,7 @@ bool build_blocks(Context* c, DCsr& A, const int* order, double min_reuse) {
 
 template <typename T>
 static bool have_values(Context* c, DCsr& A, DBuf<T>& out) {
+    if (!A.blk.built()) return false;
     try {
         if (!out) block_values<T>(c, A, out);
         return true;

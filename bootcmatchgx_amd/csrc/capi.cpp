@@ -61,19 +61,25 @@ static int record(bcmgx_context_s* ctx, int code, const char* msg) {
 // 9.7 and 8.2, 5 as 8 6.7 and 6.4; 7-point 90^3, 31: 56.8 and 32.7.  FP64, 7-point 90^3, 31: 59.4 and 42.6, 9 as 10
 // 23.3 and 19.9; CG with l1-Jacobi, 9: 75.6 and 69.1, but 7 as 8 47.1 and 54.3, so from 9 columns on.
 static int run_columns(const Prec& P, int k) {
+    if (P.lean) return k;
     bool f32 = P.ptype == BCMGX_PREC_BCMG && P.p.precision == BCMGX_PRECISION_FP32;
     if (f32) return k >= 5 ? (k + 3) / 4 * 4 : k;
     return k >= 9 ? (k + 1) / 2 * 2 : k;
 }
-// run(w), with w = k where there is no memory for the wider block
+// run(), which reads its arguments before it writes any; where it finds no memory, again without what it can
+// do without.  What the first attempt allocated goes back before: kept beside the second's it would
+// refuse columns that fit, and the preconditioner does not try again what did not fit.
 template <typename F>
-static void run_padded(const Prec& P, int k, F&& run) {
-    int w = run_columns(P, k);
+static void run_or_lean(Prec& P, F&& run) {
+    bool blocks = P.A->blk.built();
     try {
-        run(w);
+        run();
     } catch (const Error& e) {
-        if (w == k || e.code != BCMGX_ERR_ALLOC) throw;
-        run(k);
+        if (P.lean || e.code != BCMGX_ERR_ALLOC) throw;
+        P.ctx->sync();
+        P.go_lean();
+        if (!blocks && P.A->blk.built()) const_cast<DCsr*>(P.A)->blk = BlockForm();  // made by the attempt
+        run();
     }
 }
 
@@ -388,7 +394,8 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
         c->sync();
         return BCMGX_OK;
     }
-    run_padded(*prec->P, nrhs, [&](int w) {
+    run_or_lean(*prec->P, [&] {
+        int w = run_columns(*prec->P, nrhs);
         size_t nk = std::max<size_t>((size_t)n * w, 1);
         DBuf<double> R(c, nk), U(c, nk), tmp;
         stage_in(c, r, ld, mem, n, nrhs, R.get(), tmp, w);
@@ -545,12 +552,13 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
         io.x = x;
         io.ld = ld;
         io.have = nrhs;
-        run_padded(*P, nrhs, [&](int w) { r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, w, &io); });
+        run_or_lean(*P, [&] { r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, run_columns(*P, nrhs), &io); });
     } else if (nrhs == 1 && mem != BCMGX_MEM_HOST && (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS)) {
         // one device column: copied into the solver's own buffers and back by the solver
         r = p->solver == BCMGX_SOLVER_CGHS ? cghs_solve(c, A->A, P, *p, b, x, 1) : fcg_solve(c, A->A, P, *p, b, x, 1);
     } else if (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS) {
-        run_padded(*P, nrhs, [&](int w) {
+        run_or_lean(*P, [&] {
+            int w = run_columns(*P, nrhs);
             size_t nk = (size_t)std::max(n, 1) * w;
             DBuf<double> B(c, nk), X(c, nk), tmp;
             stage_in(c, b, ld, mem, n, nrhs, B.get(), tmp, w);
@@ -662,6 +670,15 @@ int bcmgx_internal_fail_allocation(bcmgx_context ctx, long long after, long long
     if (!ctx) return BCMGX_ERR_ARG;
     ctx->c->pool->fail_after(after);
     if (count) *count = ctx->c->pool->allocations();
+    return BCMGX_OK;
+}
+
+// Not part of the public interface: device allocations that would bring this context's bytes in use
+// over `limit` fail (0: none); *peak, when given, is the most in use since the last call.
+int bcmgx_internal_memory_limit(bcmgx_context ctx, long long limit, long long* peak) {
+    if (!ctx || limit < 0) return BCMGX_ERR_ARG;
+    if (peak) *peak = (long long)ctx->c->pool->peak();
+    ctx->c->pool->limit((size_t)limit);
     return BCMGX_OK;
 }
 

@@ -66,6 +66,12 @@ public:
     // the allocation after the next n fails, as one that finds no memory does (negative: none)
     void fail_after(long long n) { fail_after_ = n; }
     long long allocations() const { return count_; }
+    // allocations that would bring the bytes in use over this fail too (0: any may); the most in use since then
+    void limit(size_t bytes) {
+        limit_ = bytes;
+        peak_ = in_use_;
+    }
+    size_t peak() const { return peak_; }
 
 private:
     static size_t size_class(size_t b);
@@ -74,7 +80,7 @@ private:
     std::vector<std::pair<size_t, void*>> deferred_;
     std::multimap<size_t, void*> free_;
     std::map<void*, size_t> live_;
-    size_t in_use_ = 0;
+    size_t in_use_ = 0, limit_ = 0, peak_ = 0;
     long long count_ = 0, fail_after_ = -1;
 };
 

@@ -322,7 +322,7 @@ constexpr double BLK_MIN_REUSE = 1.5;  // entries per x row loaded below which t
 // A's block form over tiles of 16 rows taken from order (a permutation of the rows, on the device);
 // false (nothing kept) where rows are too long, share too few columns or list a column twice
 bool build_blocks(Context* c, DCsr& A, const int* order, double min_reuse = BLK_MIN_REUSE);
-// the values in block order, on first need; false: no memory for them
+// the values in block order, on first need; false: no memory for them, or no form
 bool block_values32(Context* c, DCsr& A);
 bool block_values64(Context* c, DCsr& A);
 void refresh_blocks(Context* c, DCsr& A);  // after A's values changed

@@ -28,7 +28,7 @@ size_t DevicePool::size_class(size_t b) {
 void* DevicePool::alloc(size_t bytes) {
     size_t c = size_class(bytes);
     count_++;
-    if (fail_after_ >= 0 && fail_after_-- == 0) throw Error(BCMGX_ERR_ALLOC, "allocation failed as asked for");
+    if ((fail_after_ >= 0 && fail_after_-- == 0) || (limit_ && in_use_ + c > limit_)) throw Error(BCMGX_ERR_ALLOC, "allocation failed as asked for");
     auto it = free_.find(c);
     void* p = nullptr;
     if (it != free_.end()) {
@@ -51,6 +51,7 @@ void* DevicePool::alloc(size_t bytes) {
     }
     live_[p] = c;
     in_use_ += c;
+    peak_ = std::max(peak_, in_use_);
     return p;
 }
 
