@@ -384,8 +384,9 @@ static bool level_product_async(Context* c, Hierarchy& H, int l, bool f32) {
 // Whether a level keeps A P.  FP64 cycles do on large levels, where the post sweep is bound by memory and
 // reads 12 bytes an entry of A: 27-point 128^3 133 us from A, 64 from A P, and level 1's last
 // sweep no longer prolongs (30 -> 10 us); below some 4 M entries (20 us) the product costs the setup more than a solve gets back.
-static bool keeps_product(const bcmgx_params& p, const DCsr& A, bool f32) {
-    return p.post_galerkin && (f32 || A.nnz >= 4000000);
+static bool keeps_product(const Prec& pr, const DCsr& A) {
+    bool f32 = pr.p.precision == BCMGX_PRECISION_FP32;
+    return pr.p.post_galerkin && (f32 || (!pr.lean && A.nnz >= 4000000));
 }
 // f(), which forms a level's product; an FP64 cycle does without it where there is no memory for it (false)
 template <typename F>
@@ -497,6 +498,9 @@ void Prec::go_lean() {
     for (auto* b : {&cd_F, &cd_X, &cd_X2, &tmp, &tmp2, &tmp3}) b->release();
     coarse = CoarseSync();
     kcap = tuned_k = 0;
+    if (p.precision != BCMGX_PRECISION_FP32)
+        for (int h = 0; ptype == BCMGX_PREC_BCMG && h < n_hrc(); h++)
+            for (auto& lp : hrc(h).L) lp->AP = DCsr();
 }
 
 void Prec::allocate_work(int k) {
@@ -1018,13 +1022,14 @@ static void bootstrap(Context* c, const DCsr& A, Prec* pr, Build build_next) {
     }
 }
 
-std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& p) {
+std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& p, bool lean) {
     double t0 = now_s();
     std::unique_ptr<Prec> pr(new Prec());
     pr->ctx = c;
     pr->A = &A;
     pr->p = p;
     pr->ptype = p.preconditioner;
+    pr->lean = lean;
     // the row-tile index of the caller's matrix (its pattern only: built once, kept
     // with the matrix) serves the one-column products with it
     if (A.n >= 65536 && p.autotune) build_tile_index(c, const_cast<DCsr&>(A));
@@ -1056,7 +1061,7 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
             Hierarchy* hp = &H;
             return [&, hp](int l) {  // runs on the side queue
                 if (f32) level_fp32_copy(c, *hp->L[l]);
-                if (l + 1 < hp->levels() && l < (int)async_product.size() && keeps_product(p, hp->L[l]->mat(), f32))
+                if (l + 1 < hp->levels() && l < (int)async_product.size() && keeps_product(*pr, hp->L[l]->mat()))
                     product_or_none(*hp->L[l], f32, [&] { async_product[l] = level_product_async(c, *hp, l, f32) ? 1 : 0; });
             };
         };
@@ -1064,7 +1069,7 @@ std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& 
             side.join();
             std::vector<Level*> queued;
             for (int l = 0; l + 1 < H.levels(); l++) {
-                if (!keeps_product(p, H.L[l]->mat(), f32)) continue;
+                if (!keeps_product(*pr, H.L[l]->mat())) continue;
                 if (l < (int)async_product.size() && async_product[l]) queued.push_back(H.L[l].get());
                 else product_or_none(*H.L[l], f32, [&] { make_level_product(c, H, l, f32); });
             }

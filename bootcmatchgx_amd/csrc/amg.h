@@ -75,9 +75,9 @@ struct Prec {
     void ensure_work(int k);
     void allocate_work(int k);
     // set where a call found no memory for what it can do without: columns beside the caller's, the
-    // matrix's block form
+    // matrix's block form, the products A P of an FP64 hierarchy
     bool lean = false;
-    // gives the first up, with every buffer that the next call allocates again (nothing is queued any more)
+    // gives all but the form up, with every buffer that the next call allocates again (nothing is queued any more)
     void go_lean();
     void drop_graphs();
     // u <- B r for k interleaved columns; `x_zero`: u holds zeros on entry (the FCG case).
@@ -101,7 +101,7 @@ struct Prec {
     void refresh_level0();
 };
 
-std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& p);
+std::unique_ptr<Prec> prec_setup(Context* c, const DCsr& A, const bcmgx_params& p, bool lean = false);
 
 inline double now_s() {
     return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();

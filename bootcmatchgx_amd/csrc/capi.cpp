@@ -369,7 +369,14 @@ int bcmgx_prec_setup(bcmgx_context ctx, bcmgx_matrix A, const bcmgx_params* p, b
     h->ctx = ctx;
     h->A = A;
     try {
-        h->P = prec_setup(ctx->c, A->A, *p);
+        try {
+            h->P = prec_setup(ctx->c, A->A, *p);
+        } catch (const Error& e) {  // without the products A P that an FP64 hierarchy can do without
+            if (e.code != BCMGX_ERR_ALLOC || p->preconditioner != BCMGX_PREC_BCMG || p->precision == BCMGX_PRECISION_FP32 ||
+                !p->post_galerkin)
+                throw;
+            h->P = prec_setup(ctx->c, A->A, *p, true);
+        }
     } catch (...) {
         delete h;
         throw;
@@ -390,7 +397,7 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
     if (ld < n) ld = n;
     // one device column is applied where it is: three copies less, 4-5 us each in a call of some 100 us
     if (nrhs == 1 && mem != BCMGX_MEM_HOST && on_device(c, r) && on_device(c, u) && apart(r, n, u, n)) {
-        prec->P->apply(r, u, 1, false, nullptr);
+        run_or_lean(*prec->P, [&] { prec->P->apply(r, u, 1, false, nullptr); });
         c->sync();
         return BCMGX_OK;
     }
@@ -555,7 +562,9 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
         run_or_lean(*P, [&] { r = fcg_solve(c, A->A, P, *p, nullptr, nullptr, run_columns(*P, nrhs), &io); });
     } else if (nrhs == 1 && mem != BCMGX_MEM_HOST && (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS)) {
         // one device column: copied into the solver's own buffers and back by the solver
-        r = p->solver == BCMGX_SOLVER_CGHS ? cghs_solve(c, A->A, P, *p, b, x, 1) : fcg_solve(c, A->A, P, *p, b, x, 1);
+        run_or_lean(*P, [&] {
+            r = p->solver == BCMGX_SOLVER_CGHS ? cghs_solve(c, A->A, P, *p, b, x, 1) : fcg_solve(c, A->A, P, *p, b, x, 1);
+        });
     } else if (p->solver == BCMGX_SOLVER_FCG || p->solver == BCMGX_SOLVER_CGHS) {
         run_or_lean(*P, [&] {
             int w = run_columns(*P, nrhs);
@@ -568,12 +577,14 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
             stage_out(c, X.get(), x, ld, mem, n, nrhs, tmp, w);
         });
     } else {
-        size_t nk = (size_t)std::max(n, 1) * nrhs;
-        DBuf<double> B(c, nk), X(c, nk), tmp;
-        stage_in(c, b, ld, mem, n, nrhs, B.get(), tmp);
-        stage_in(c, x, ld, mem, n, nrhs, X.get(), tmp);
-        r = cgs_solve(c, A->A, P, *p, B.get(), X.get(), nrhs);
-        stage_out(c, X.get(), x, ld, mem, n, nrhs, tmp);
+        run_or_lean(*P, [&] {
+            size_t nk = (size_t)std::max(n, 1) * nrhs;
+            DBuf<double> B(c, nk), X(c, nk), tmp;
+            stage_in(c, b, ld, mem, n, nrhs, B.get(), tmp);
+            stage_in(c, x, ld, mem, n, nrhs, X.get(), tmp);
+            r = cgs_solve(c, A->A, P, *p, B.get(), X.get(), nrhs);
+            stage_out(c, X.get(), x, ld, mem, n, nrhs, tmp);
+        });
     }
     for (auto* v : {&P->last_exit, &P->last_rel})  // the caller's columns
         if ((int)v->size() > nrhs) v->resize(nrhs);

@@ -93,10 +93,11 @@ typedef struct bcmgx_params {
                                widens it exactly inside its kernels (fewer bytes; the dot products are blocked
                                differently, so iterates may differ in the last bits; default 1) */
     int post_galerkin;      /* "post_galerkin": the first post-smoothing sweep of each level (with an FP64
-                               hierarchy, of those whose operator has 4 M entries or more) takes its residual
-                               as r_pre - (A P) e, from the pre-smoothing residual and the product A P kept
-                               from setup, in place of f - A (x + P e) (the same value in exact arithmetic,
-                               from the sparser A P; default 1) */
+                               hierarchy, of those whose operator has 4 M entries or more, where there is
+                               memory for the product) takes its residual as r_pre - (A P) e, from the
+                               pre-smoothing residual and the product A P kept from setup, in place of
+                               f - A (x + P e) (the same value in exact arithmetic, from the sparser A P;
+                               default 1) */
 } bcmgx_params;
 
 /* Defaults of src/config/Params.h:238-291. */

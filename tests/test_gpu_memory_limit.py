@@ -1,5 +1,6 @@
 """Solves and applications where memory is short: what a call can do without (zero columns beside its own, the
-matrix's block form) is given up before the call is refused, and not asked for again."""
+matrix's block form, the product A P of an FP64 hierarchy) is given up before the call is refused, and not asked for
+again."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -37,7 +38,7 @@ def check_solve(ctx, A, S, p, P, k, seed):
     B = np.random.default_rng(seed).normal(size=(S.shape[0], k))
     x, info = bx.solve(ctx, A, B, None, p, P)
     assert info["retv"] == 0
-    assert (np.linalg.norm(B - S @ x, axis=0) <= 1.01 * p.rtol * np.linalg.norm(B, axis=0)).all()
+    assert (np.linalg.norm(B - S @ x.reshape(B.shape), axis=0) <= 1.01 * p.rtol * np.linalg.norm(B, axis=0)).all()
 
 
 # 21060 rows: 30 and 31 FP64 columns take 5 MB, 32 take 6; 7 FP32 columns of 74088 rows 2 MB, 8 take 3
@@ -94,5 +95,83 @@ def test_block_form(k):
         check_solve(ctx, A, S, p, P, k, seed)
     memory(ctx, 0)
     P.finalize()
+    A.close()
+    ctx.close()
+
+
+def large(ctx, **more):
+    """an FP64 hierarchy that keeps A P of its finest level (from 4 M entries on), unless post_galerkin=0"""
+    return bx.Params(solver="FCG", preconditioner="BCMG", precision="FP64", rtol=1e-7, prerelax_sweeps=1, postrelax_sweeps=1,
+                     dispnorm=0, **more)
+
+
+@pytest.mark.parametrize("solver, k, device", [("FCG", 1, False), ("FCG", 1, True), ("FCG", 2, False), ("FCG", 3, True), ("CGHS", 2, False),
+                                               ("CGS", 1, False), ("apply", 1, False), ("apply", 2, False)])
+def test_product_of_the_finest_level(solver, k, device):
+    """what fits a hierarchy without the product fits one with it; the values of the matrix may change afterwards"""
+    ctx = bx.Context(0)
+    A, S = problem(ctx, 27, (56, 55, 54))
+    n = S.shape[0]
+    b = np.random.default_rng(1).normal(size=(n, k))
+    dB, dX = bx.DeviceArray(ctx, (k * n,)), bx.DeviceArray(ctx, (k * n,))
+    dB.upload(b.T.ravel())
+
+    def call(p, P):
+        if device:
+            dX.upload(np.zeros(k * n))
+        if solver == "apply":
+            if not device:
+                return P.apply(b)
+            bx._check(bx.lib().bcmgx_prec_apply(P.h, dB.ptr, dX.ptr, k, n, bx.MEM_DEVICE), ctx)
+        elif device:
+            bx.solve_device(ctx, A, dB.ptr, dX.ptr, k, p, P, n)
+        else:
+            return bx.solve(ctx, A, b, None, p, P)[0]
+        return dX.download().reshape(k, n).T
+
+    method = {} if solver == "apply" else {"solver": solver, "sstep": 2} if solver == "CGS" else {"solver": solver}
+    results, limit = [], 0
+    for post in (0, 1):
+        p = large(ctx, post_galerkin=post)
+        for key, v in method.items():
+            p.set(key, v)
+        P = bx.prec_setup(ctx, A, p)
+        memory(ctx, 0)
+        if post:
+            memory(ctx, limit + MB)
+        results.append([call(p, P) for _ in range(3)])
+        if post:
+            memory(ctx, 0)
+            A.update_values(A.to_scipy().data)
+            results.append([call(p, P)])
+        else:
+            limit = memory(ctx, 0)
+        P.finalize()
+    for x in results[1] + results[2]:  # without the product: the same operations
+        assert np.array_equal(x, results[0][0])
+    A.close()
+    ctx.close()
+
+
+def test_setup():
+    """a setup that finds no memory for the product's sake is made without"""
+    ctx = bx.Context(0)
+    A, S = problem(ctx, 27, (56, 55, 54))
+    p = large(ctx, post_galerkin=0)
+    memory(ctx, 0)
+    P = bx.prec_setup(ctx, A, p)
+    need = memory(ctx, 0)
+    P.finalize()
+    p = large(ctx)
+    for limit in (need + MB, need + 20 * MB, need + 40 * MB, need + 60 * MB, need + 80 * MB):
+        memory(ctx, limit)
+        P = bx.prec_setup(ctx, A, p)
+        memory(ctx, 0)
+        check_solve(ctx, A, S, p, P, 1, 1)
+        P.finalize()
+    memory(ctx, need // 2)
+    with pytest.raises(bx.BcmgxError):
+        bx.prec_setup(ctx, A, p)
+    memory(ctx, 0)
     A.close()
     ctx.close()
