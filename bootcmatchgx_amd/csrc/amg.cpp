@@ -480,6 +480,18 @@ void Prec::drop_graphs() {
     for (auto& s : solves) s->drop_graph();
 }
 
+bool Prec::gave_up() {
+    if (!ctx->coarse_gave_up()) return false;
+    coarse.off = true;
+    drop_graphs();
+    return true;
+}
+void Prec::wait_again() {
+    if (!coarse.off) return;
+    coarse.off = false;
+    drop_graphs();
+}
+
 // work whose allocation fails is not there: nothing of it is taken for complete by the next call
 void Prec::ensure_work(int k) {
     try {
@@ -1332,6 +1344,7 @@ SolveResult fcg_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params&
             launched += 2;
         }
         c->d2h(hflag, s.flags.get(), 2);
+        if (prec->gave_up()) use_graph = false;
         if (hflag[0]) break;
         if (launched > p.itnlim + 2) break;  // the device stops every column at itnlim
     }
@@ -1440,6 +1453,7 @@ SolveResult cghs_solve(Context* c, const DCsr& A, Prec* prec, const bcmgx_params
                 else iteration();
             }
             c->d2h(hflag, s.flags.get(), 2);
+            if (prec->gave_up()) use_graph = false;
             if (hflag[0]) break;
         }
     }

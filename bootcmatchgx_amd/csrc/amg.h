@@ -80,6 +80,10 @@ struct Prec {
     // gives all but the form up, with every buffer that the next call allocates again (nothing is queued any more)
     void go_lean();
     void drop_graphs();
+    // (with nothing queued) true when coarsest sweeps gave up waiting: they are launched one by one from now
+    // on, and the captured iterations, which hold the other launches, are dropped
+    bool gave_up();
+    void wait_again();  // undoes it
     // u <- B r for k interleaved columns; `x_zero`: u holds zeros on entry (the FCG case).
     // `entry_ready`: the level-0 entry of the cycle (see fused_entry) already holds the
     // first sweep X = F / M and, in FP32, F = (float) r (unless the cycle reads r itself).

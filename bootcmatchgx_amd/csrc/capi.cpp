@@ -399,6 +399,7 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
     if (nrhs == 1 && mem != BCMGX_MEM_HOST && on_device(c, r) && on_device(c, u) && apart(r, n, u, n)) {
         run_or_lean(*prec->P, [&] { prec->P->apply(r, u, 1, false, nullptr); });
         c->sync();
+        prec->P->gave_up();
         return BCMGX_OK;
     }
     run_or_lean(*prec->P, [&] {
@@ -411,6 +412,7 @@ int bcmgx_prec_apply(bcmgx_prec prec, const double* r, double* u, int nrhs, int 
         stage_out(c, U.get(), u, ld, mem, n, nrhs, tmp, w);
     });
     c->sync();
+    prec->P->gave_up();
     return BCMGX_OK;
     API_END(prec->ctx)
 }
@@ -590,6 +592,7 @@ int bcmgx_solve(bcmgx_context ctx, bcmgx_matrix A, bcmgx_prec prec, const bcmgx_
         if ((int)v->size() > nrhs) v->resize(nrhs);
     if ((int)P->last_niter.size() > nrhs) P->last_niter.resize(nrhs);
     c->sync();
+    P->gave_up();
     if (out) {
         out->retv = r.retv;
         out->niter = r.niter;
@@ -668,12 +671,16 @@ int bcmgx_dump_info(const char* path, const bcmgx_params* p, bcmgx_prec prec, co
 
 // Not part of the public interface (no declaration in bcmgx.h): the clock ticks a wait of the
 // one-launch coarsest sweeps may take on this context before its fallback computes them
-// (negative: no wait, always the fallback).
+// (negative: no wait, always the fallback).  Preconditioners that gave the waits up take them up again.
 int bcmgx_internal_coarse_patience(bcmgx_context ctx, long long ticks) {
     if (!ctx) return BCMGX_ERR_ARG;
     ctx->c->coarse_patience = ticks;
+    for (auto* p : ctx->precs)
+        if (p->P) p->P->wait_again();
     return BCMGX_OK;
 }
+// Not part of the public interface: how often calls on this context found that such a wait had ended in vain.
+long long bcmgx_internal_coarse_give_ups(bcmgx_context ctx) { return ctx ? ctx->c->coarse_give_ups : -1; }
 
 // Not part of the public interface: the device allocation after the next `after` on this context
 // fails (negative: none); *count, when given, is the number of them so far.

@@ -97,13 +97,15 @@ __device__ __forceinline__ int coarse_ticket(unsigned* ctl, unsigned workgroups)
 // grid to half of what the device holds; whatever else occupies it, each
 // wait is bounded: a workgroup that waits longer than `patience` clock ticks
 // raises ctl[2], all give up, and the workgroup that finishes last computes the
-// sweeps alone.  Workgroups that had their values wrote the same ones.
+// sweeps alone.  Workgroups that had their values wrote the same ones.  It says
+// so in *gave_up (the host's memory), and the host goes back to a launch a sweep:
+// whatever holds the device would have every cycle wait.
 template <typename V, int L, int E>
 __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
     int n, const int* __restrict__ row, const int* __restrict__ col, const double* __restrict__ val,
     const double* __restrict__ D, const V* __restrict__ f, const V* __restrict__ x0, V* __restrict__ out, int sweeps,
     const int* __restrict__ ucnt, const int* __restrict__ ucol, const unsigned short* __restrict__ upos, u64* slots,
-    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience, RowProlong<V> up) {
+    double* scratch, unsigned* ctl, unsigned* gave_up, const int* __restrict__ stop, long long patience, RowProlong<V> up) {
     constexpr int T = CO_ROWS * L, NU = CO_FETCH;
     if (stop && *stop) return;
     __shared__ double xs[2][TILE_MAX_COLS];
@@ -221,6 +223,7 @@ __global__ __launch_bounds__(CO_ROWS * L) void k_coarse_exchange(
     if (!s_last) return;
     // the last workgroup: every other one has passed its waits for good
     if (s_last == 2) {
+        if (tid == 0) __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         double* cur = scratch;
         double* nxt = scratch + n;
         for (int i = tid; i < n; i += T) cur[i] = first(i);
@@ -317,7 +320,7 @@ static bool launch_exchange(Context* c, const DCsr& A, const double* D, const V*
     if ((long long)grid * 2 > resident) return false;
     kern<<<grid, CO_ROWS * L, 0, c->stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, sweeps,
                                               ix.ucnt.get(), ix.ucol.get(), ix.upos.get(), cs.slots.get(),
-                                              cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience, up);
+                                              cs.scratch.get(), cs.ctl.get(), c->mailbox() + MAIL_GAVE_UP, stop, c->coarse_patience, up);
     BCMGX_LAUNCHED();
     return true;
 }
@@ -369,7 +372,7 @@ bool coarse_sweeps(Context* c, const DCsr& A, int lanes, const double* D, const 
         BCMGX_LAUNCHED();
         return true;
     }
-    if (!ix.ucnt || cs.slots.size() < (size_t)A.n * sweeps * 2 || cs.scratch.size() < (size_t)A.n * 2) return false;
+    if (cs.off || !ix.ucnt || cs.slots.size() < (size_t)A.n * sweeps * 2 || cs.scratch.size() < (size_t)A.n * 2) return false;
 #define BCMGX_CX(LL)                                                                                         \
     case LL:                                                                                                 \
         if (A.maxrow <= 2 * LL) return launch_exchange<V, LL, 2>(c, A, D, f, x0, out, sweeps, ix, cs, stop, up);     \
@@ -396,7 +399,7 @@ __global__ __launch_bounds__(CO_ROWS * CO_COLS, E > 32 ? 2 : E > 16 ? 3 : 4) voi
     int n, int k, const int* __restrict__ row, const int* __restrict__ col, const double* __restrict__ val,
     const double* __restrict__ D, const V* __restrict__ f, const V* __restrict__ x0, V* __restrict__ out, int sweeps,
     const int* __restrict__ ucnt, const int* __restrict__ ucol, const unsigned short* __restrict__ upos, u64* slots,
-    double* scratch, unsigned* ctl, const int* __restrict__ stop, long long patience) {
+    double* scratch, unsigned* ctl, unsigned* gave_up, const int* __restrict__ stop, long long patience) {
     constexpr int CC = CO_COLS, T = CO_ROWS * CC, NU = CO_COL_FETCH;
     if (stop && *stop) return;
     __shared__ double xs[CO_COL_PLACES * CC];
@@ -518,6 +521,7 @@ __global__ __launch_bounds__(CO_ROWS * CO_COLS, E > 32 ? 2 : E > 16 ? 3 : 4) voi
     if (!s_last) return;
     // the last workgroup: every other one has passed its waits for good
     if (s_last == 2) {
+        if (tid == 0) __hip_atomic_store(gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         for (int q = 0; q < k; q++) {
             double* cur = scratch;
             double* nxt = scratch + n;
@@ -565,7 +569,7 @@ static bool launch_columns(Context* c, const DCsr& A, const double* D, const V* 
         return false;
     kern<<<dim3(tiles, groups), CO_ROWS * CO_COLS, 0, c->stream>>>(
         A.n, k, A.row.get(), A.col.get(), A.val.get(), D, f, x0, out, sweeps, ix.ucnt.get(), ix.ucol.get(), ix.upos.get(),
-        cs.slots.get(), cs.scratch.get(), cs.ctl.get(), stop, c->coarse_patience);
+        cs.slots.get(), cs.scratch.get(), cs.ctl.get(), c->mailbox() + MAIL_GAVE_UP, stop, c->coarse_patience);
     BCMGX_LAUNCHED();
     return true;
 }
@@ -573,7 +577,7 @@ static bool launch_columns(Context* c, const DCsr& A, const double* D, const V* 
 template <typename V>
 bool coarse_sweeps_columns(Context* c, const DCsr& A, const double* D, const V* f, const V* x0, V* out, int k, int sweeps,
                            const CoarseIndex& ix, CoarseSync& cs, const int* stop) {
-    if (k < 2 || !coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || !ix.ucnt || (const void*)out == (const void*)x0 ||
+    if (cs.off || k < 2 || !coarse_sweeps_fit(A.n, sweeps) || A.maxrow < 0 || !ix.ucnt || (const void*)out == (const void*)x0 ||
         (const void*)out == (const void*)f || cs.scratch.size() < (size_t)A.n * 2)
         return false;
     if (A.maxrow <= 16) return launch_columns<V, 16>(c, A, D, f, x0, out, k, sweeps, ix, cs, stop);

@@ -120,7 +120,8 @@ private:
 // Small device-to-host reads (Context::d2h, d2h2): a kernel writes the words and then the read's number
 // into pinned memory, and the host polls for the number.  6 us a read, where a copy and a stream
 // synchronisation take 12; a setup makes 15 to 100 of them, each a point where the host waits.
-constexpr int MAIL_HEAD = 16;     // words: the number, on a cache line of its own
+constexpr int MAIL_HEAD = 16;     // words: the number, and MAIL_GAVE_UP, before the read's
+constexpr int MAIL_GAVE_UP = 1;   // set by a launch of coarsest sweeps whose waits ended in vain
 constexpr int MAIL_WORDS = 2048;  // the most one read takes
 
 struct Context {
@@ -136,12 +137,16 @@ struct Context {
     size_t pinned_bytes = 0;
     unsigned* mail = nullptr;
     unsigned mail_seq = 0;
+    unsigned* mailbox();  // mail, there from the first use on
     // words of a, then of b, read after everything queued on the stream; valid until the next read
     const unsigned* mail_read(const void* a, size_t words_a, const void* b, size_t words_b);
     // autotune cache: matrix signature -> lanes per row
     std::map<std::string, int> tuned_lanes;
     // clock ticks (100 MHz) a wait of the one-launch coarsest sweeps may take before its fallback
     long long coarse_patience = 500000;
+    // whether one gave up since the last call (with nothing queued); how often that was so
+    bool coarse_gave_up();
+    long long coarse_give_ups = 0;
     // this device's copy of the fixed scratch array of the allocation-free entry point
     void* scratch = nullptr;
 

@@ -349,6 +349,7 @@ struct CoarseSync {
     DBuf<unsigned long long> slots;  // [sweep][row][2], or [columns][sweep][row][column][2]
     DBuf<double> scratch;            // 2 n, for the workgroup that finishes after waits gave up
     DBuf<unsigned> ctl;
+    bool off = false;                // waits ended in vain: launch by launch from now on
     void reserve(Context* c, int n, int sweeps, int k);
 };
 // the distinct columns of each 32-row tile of a coarsest operator, listed at setup (setup.hip's

@@ -128,11 +128,23 @@ __global__ __launch_bounds__(WG) void k_mail(const unsigned* __restrict__ a, int
     if (threadIdx.x == 0) __hip_atomic_store(box, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-const unsigned* Context::mail_read(const void* a, size_t na, const void* b, size_t nb) {
+unsigned* Context::mailbox() {
     if (!mail) {
         BCMGX_HIP(hipHostMalloc(reinterpret_cast<void**>(&mail), (MAIL_HEAD + MAIL_WORDS) * sizeof(unsigned), hipHostMallocCoherent));
-        mail[0] = 0;
+        std::fill(mail, mail + MAIL_HEAD, 0u);
     }
+    return mail;
+}
+
+bool Context::coarse_gave_up() {
+    if (!mail || !__atomic_load_n(mail + MAIL_GAVE_UP, __ATOMIC_ACQUIRE)) return false;
+    __atomic_store_n(mail + MAIL_GAVE_UP, 0u, __ATOMIC_RELAXED);
+    coarse_give_ups++;
+    return true;
+}
+
+const unsigned* Context::mail_read(const void* a, size_t na, const void* b, size_t nb) {
+    mailbox();
     unsigned seq = ++mail_seq ? mail_seq : ++mail_seq;
     k_mail<<<1, WG, 0, stream>>>((const unsigned*)a, (int)na, (const unsigned*)b, (int)nb, mail, seq);
     BCMGX_LAUNCHED();

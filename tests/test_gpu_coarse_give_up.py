@@ -30,3 +30,39 @@ def test_bounded_waits(points, dims, k, precision):
     P.finalize()
     A.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("solver, use_graph", [("FCG", 1), ("FCG", 0), ("CGHS", 1), ("CGS", 1)])
+@pytest.mark.parametrize("k", [1, 3])
+def test_not_waited_for_again(solver, use_graph, k):
+    """A call whose waits ended in vain is the last that waits: the next ones, and the rest of a solve, launch the
+    sweeps one by one, with the same bits."""
+    if solver == "CGS" and k > 1:
+        pytest.skip("one column")
+    L = bx.lib()
+    patience, give_ups = L.bcmgx_internal_coarse_patience, L.bcmgx_internal_coarse_give_ups
+    patience.argtypes = [bx.C.c_void_p, bx.C.c_longlong]
+    give_ups.argtypes, give_ups.restype = [bx.C.c_void_p], bx.C.c_longlong
+    ctx = bx.Context(0)
+    n, row, col, val = bx.laplacian3d(7, 41, 40, 39)
+    A = bx.CSR(ctx, n, n, row, col, val)
+    p = bx.Params(solver=solver, preconditioner="BCMG", rtol=1e-8, check_every=2, sstep=2, use_graph=use_graph, dispnorm=0)
+    P = bx.prec_setup(ctx, A, p)
+    b = np.random.default_rng(3).normal(size=(n, k))
+    solve = lambda: bx.solve(ctx, A, b, None, p, P)[0]
+    x, u = solve(), P.apply(b)
+    assert np.array_equal(solve(), x)  # replayed, where it is
+    assert give_ups(ctx.h) == 0
+    for call, result in ((solve, x), (lambda: P.apply(b), u)):
+        before = give_ups(ctx.h)
+        assert patience(ctx.h, -1) == 0
+        for _ in range(3):
+            assert np.array_equal(call(), result)
+        assert give_ups(ctx.h) - before == 1
+        assert patience(ctx.h, 500000) == 0
+        for _ in range(2):
+            assert np.array_equal(call(), result)
+        assert give_ups(ctx.h) - before == 1
+    P.finalize()
+    A.close()
+    ctx.close()
