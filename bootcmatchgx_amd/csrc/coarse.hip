@@ -335,10 +335,13 @@ void CoarseIndex::build(Context* c, const DCsr& A) {
 }
 
 void CoarseSync::reserve(Context* c, int n, int sweeps, int k) {
-    size_t need = (size_t)n * (size_t)std::max(sweeps, 1) * 2;
-    if (k > 1) {  // whole groups of columns
-        size_t all = need * CO_COLS * ((k + CO_COLS - 1) / CO_COLS);
-        if (all <= CO_SLOT_WORDS) need = all;
+    size_t words = (size_t)std::max(sweeps, 1) * 2, need = n * words;
+    if (k > 1) {
+        // as many groups of columns as launch_columns takes, a workgroup a CU, whatever k is: a wide
+        // solve's slots serve the narrow ones after it (20 sweeps of 4096 rows: 21 MB)
+        size_t rows = (size_t)c->num_cus * CO_ROWS, groups = (k + CO_COLS - 1) / CO_COLS;
+        size_t all = std::min(n * groups, rows) * words * CO_COLS;
+        if ((size_t)n <= rows && all <= CO_SLOT_WORDS) need = std::max(need, all);
     }
     if (slots.size() >= need && scratch.size() >= (size_t)n * 2) return;
     slots.reset(c, need);

@@ -66,3 +66,26 @@ def test_not_waited_for_again(solver, use_graph, k):
     P.finalize()
     A.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("widths, n_exchanges", [((64, 8), 1), ((64, 16, 3), 2), ((32, 8), 1), ((8, 64, 8), 2)])
+def test_narrow_after_wide(widths, n_exchanges):
+    """The exchange for a few columns does not depend on the widths before: 4096 rows run it to 16 columns."""
+    L = bx.lib()
+    patience, give_ups = L.bcmgx_internal_coarse_patience, L.bcmgx_internal_coarse_give_ups
+    patience.argtypes = [bx.C.c_void_p, bx.C.c_longlong]
+    give_ups.argtypes, give_ups.restype = [bx.C.c_void_p], bx.C.c_longlong
+    ctx = bx.Context(0)
+    n, row, col, val = bx.laplacian3d(27, 16, 16, 16)
+    A = bx.CSR(ctx, n, n, row, col, val)
+    P = bx.prec_setup(ctx, A, bx.Params(preconditioner="BCMG", max_levels=1, relaxnumber_coarse=20, dispnorm=0))
+    for k in widths:
+        f = np.random.default_rng(k).normal(size=(n, k))
+        assert patience(ctx.h, 500000) == 0
+        x = P.apply(f)
+        assert patience(ctx.h, -1) == 0  # an exchange gives up at once, and says so
+        assert np.array_equal(P.apply(f), x)
+    assert give_ups(ctx.h) == n_exchanges
+    P.finalize()
+    A.close()
+    ctx.close()
