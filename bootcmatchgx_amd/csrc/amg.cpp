@@ -123,12 +123,15 @@ static float time_spmm(Context* c, const DCsr& A, const void* val, int k, int ch
     return ms;
 }
 
+// the block form's cost goes by the columns that its tiles share: matrices of one size may differ in that
+static std::string blocks_key(const DCsr& A) { return "b" + std::to_string(A.blk.groups); }
+
 int tune_chunk(Context* c, const DCsr& A, bool fp32, int k) {
     if (k <= 4 || A.n < 65536) return k;
     if (fp32 && !A.valf) throw Error(BCMGX_ERR_STATE, "tune_chunk: FP32 values not built");
     bool blocks = fp32 && A.blk.built() && A.blk.val32 && blk_width(k);
     std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + (fp32 ? "f" : "d") + ":k" + std::to_string(k) +
-                      (blocks ? "b" : "");
+                      (blocks ? blocks_key(A) : "");
     auto it = c->tuned_lanes.find(sig);
     if (it != c->tuned_lanes.end()) return it->second;
     hipEvent_t e0, e1;
@@ -1134,7 +1137,7 @@ static int fused_z32(Context* c, const DCsr& A, SolveWork& s, const double* wold
 }
 
 // The block form's code where the fused product is faster from it than from
-// k_spmmp, else 0: timed once for each (n, nnz, k) on the workspace's own
+// k_spmmp, else 0: timed once for each (n, nnz, k, groups) on the workspace's own
 // vectors.  It is asked only where the cycle's FP32 products run from the block
 // form, and is a choice of its own: the block form saves half of the reads of x,
 // but here it gathers w's and r's rows as well, in the tiles' order.  27-point
@@ -1142,7 +1145,7 @@ static int fused_z32(Context* c, const DCsr& A, SolveWork& s, const double* wold
 // against 433; 27-point 41x40x40, 64 columns: 43 against 36; 7-point 100x90x80, 16
 // columns: 110 against 84.
 static int tune_fused_z32(Context* c, DCsr& A, SolveWork& s) {
-    std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + "z:k" + std::to_string(s.k);
+    std::string sig = std::to_string(A.n) + ":" + std::to_string(A.nnz) + "z:k" + std::to_string(s.k) + blocks_key(A);
     auto it = c->tuned_lanes.find(sig);
     if (it != c->tuned_lanes.end()) return it->second == BLK_CODE && block_values64(c, A) ? BLK_CODE : 0;
     bool had = (bool)A.blk.val64;  // another width's captured iterations may hold them
