@@ -265,10 +265,9 @@ bool build_blocks(Context* c, DCsr& A, const int* order, double min_reuse) {
     if (A.blk.built()) return true;
     try {
         return form_blocks(c, A, order, min_reuse);
-    } catch (const Error& e) {  // no memory for it: the products run from CSR as before
+    } catch (const Error& e) {  // no memory for it now: the products run from CSR as before
         if (e.code != BCMGX_ERR_ALLOC) throw;
         A.blk = BlockForm();
-        A.blk.refused = true;
         return false;
     }
 }

@@ -1,5 +1,5 @@
 """When the 16-row block form (csrc/blocked.hip) is made and how its use is chosen: a choice timed on one matrix serves
-matrices of the same sharing of columns."""
+matrices of the same sharing of columns, and an allocation that fails once refuses the form once."""
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -40,3 +40,27 @@ def test_choice_goes_by_the_sharing():
         A.close()
     ctx.close()
     assert counts[1] < counts[0] and counts[3] < counts[2]
+
+
+def test_a_failed_allocation_is_not_for_good(ctx):
+    n, row, col, val = bx.laplacian3d(27, 9, 8, 7)
+    k, order = 8, np.arange(n, dtype=np.int32)
+    x, y, dots = np.ones((n, k), np.float32), np.zeros((n, k), np.float32), np.zeros((k, 3))
+    p = lambda v: v.ctypes.data_as(bx.C.c_void_p)
+    product = lambda A: bx.lib().bcmgx_internal_block_product(ctx.h, A.h, p(order), k, 1, p(x), None, None, p(y), p(dots))
+    A = bx.CSR(ctx, n, n, row, col, val)
+    before = allocations(ctx)
+    assert product(A) == 0
+    total = allocations(ctx) - before
+    ref = y.copy()
+    A.close()
+    for fail in range(total):
+        A = bx.CSR(ctx, n, n, row, col, val)
+        allocations(ctx, fail)
+        code = product(A)
+        allocations(ctx)
+        assert code != 0
+        y[:] = 0
+        assert product(A) == 0
+        assert np.array_equal(y, ref)
+        A.close()
