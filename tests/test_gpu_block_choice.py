@@ -64,3 +64,26 @@ def test_a_failed_allocation_is_not_for_good(ctx):
         assert product(A) == 0
         assert np.array_equal(y, ref)
         A.close()
+
+
+def test_products_follow_new_values(ctx):
+    """the form is kept with the matrix, its values (FP32 and FP64) change with the matrix's: twice and thrice the product, to
+    the bit for a power of two, within the sums' rounding (28 eps of sum |a||x|) else"""
+    n, row, col, val = bx.laplacian3d(27, 21, 19, 13)
+    S = sp.csr_matrix((val, col, row), shape=(n, n))
+    k, order = 16, np.arange(n, dtype=np.int32)
+    r = np.random.default_rng(4)
+    x, wr, dots = r.normal(size=(n, k)).astype(np.float32), r.normal(size=(2, n, k)), np.zeros((k, 3))
+    p = lambda v: v.ctypes.data_as(bx.C.c_void_p)
+    A = bx.CSR(ctx, n, n, row, col, val)
+    for op, dtype, eps in ((1, np.float32, 2.0 ** -24), (5, np.float64, 2.0 ** -53)):
+        first = None
+        for scale in (1.0, 2.0, 3.0):
+            A.update_values(val * scale)
+            y = np.zeros((n, k), dtype)
+            assert bx.lib().bcmgx_internal_block_product(ctx.h, A.h, p(order), k, op, p(x), p(wr), None, p(y), p(dots)) == 0
+            first = y if first is None else first
+            ref = scale * (S @ x.astype(np.float64))
+            assert (abs(y - ref) <= 28 * eps * scale * (abs(S) @ abs(x.astype(np.float64)))).all()
+            assert scale == 3.0 or np.array_equal(y, scale * first)
+    A.close()
