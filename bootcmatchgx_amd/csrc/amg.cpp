@@ -443,7 +443,7 @@ struct SolveWork {
     DBuf<int> flags;  // [0] all_done, [1] columns done
     FcgBufs fb;
     DBuf<unsigned> tickets;
-    FcgEntry entry;     // level-0 entry of the FP32 cycle filled by the updates
+    FcgEntry entry;     // level-0 entry of the cycle filled by the updates
     bool fused = false;
     // FP32 z: the cycle's result kept in FP32 and widened inside the fused product and the update
     bool z32 = false;

@@ -18,7 +18,7 @@ struct Level {
     DBuf<double> pval;
     DBuf<float> pvalf;
     DCsr R;                 // restrictor P^T (rows sorted by fine index)
-    DCsr AP;                // A P, FP32 values only (valf): the first post-smoothing sweep of an FP32 cycle
+    DCsr AP;                // A P for the first post-smoothing sweep, values in the cycle's precision only (may be empty)
     CoarseIndex cix;        // of the coarsest level
     int lanesA = 0, lanesR = 0, lanesAP = 0;
     int chunkA = 0;         // columns per SpMM launch for the current batch width

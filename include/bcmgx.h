@@ -87,7 +87,10 @@ typedef struct bcmgx_params {
     int precision;          /* "precision": FP64 (default) or FP32 hierarchy + V-cycle */
     int use_graph;          /* "use_graph": from the second solve of a preconditioner and column count on, replay
                                the FCG or CG iterations from a hipGraph (default 1) */
-    int autotune;           /* "autotune": pick SpMV/SpMM lanes-per-row by timing (default 1) */
+    int autotune;           /* "autotune": pick SpMV/SpMM kernels and lanes-per-row by timing (default 1).  Some
+                               round differently (one-column sums over more or fewer lanes; the k-column FP32
+                               products and FCG's fused product on the matrix cores), so two processes may
+                               differ in the last bits; 0 picks by sizes alone */
     int check_every;        /* "check_every": FCG iterations between host convergence polls (default 8) */
     int fcg_z32;            /* "fcg_z32": with an FP32 hierarchy, FCG keeps the cycle's result z in FP32 and
                                widens it exactly inside its kernels (fewer bytes; the dot products are blocked
@@ -156,7 +159,9 @@ int bcmgx_csr_update_values(bcmgx_matrix A, const double* val, int mem);
  * that list; one-column products with A then stage those x entries in LDS once
  * per tile.  It depends on the pattern only, so it is kept across value
  * updates and preconditioner setups on A; it costs 2 bytes per entry plus 4
- * per listed column of device memory. */
+ * per listed column of device memory.  bcmgx_spmm multiplies several device
+ * columns where they are, without transposing them, once the index is there;
+ * by itself it does not build one. */
 int bcmgx_csr_analyse(bcmgx_matrix A, double* seconds);
 
 /* Host-side problem generators: src/generator/laplacian.cu:119-334 (7-point),
